@@ -62,42 +62,47 @@ __device__ __forceinline__ float dot3(float ax, float ay, float az, float bx, fl
     return ax * bx + ay * by + az * bz;
 }
 
-// Wave-wide (64-lane) reductions.
+// Wave-wide (64-lane) reductions, every lane active; the result is uniform.
+// Row shifts within 16 lanes, then lane 15 / 31 broadcasts, in the VALU's data
+// path: 12 instructions and a readlane, where a butterfly of cross-lane reads
+// goes through the LDS unit six times, one round trip after the other.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int dpp_or(int old, int v) {   // old where the source lane does not exist
+    return __builtin_amdgcn_update_dpp(old, v, CTRL, ROWS, 0xf, false);
+}
+template <typename F>
+__device__ __forceinline__ int wave_reduce(int v, F&& f, bool sum) {
+    v = f(v, dpp_or<0x111, 0xf>(sum ? 0 : v, v));   // row_shr:1, 2, 4, 8
+    v = f(v, dpp_or<0x112, 0xf>(sum ? 0 : v, v));
+    v = f(v, dpp_or<0x114, 0xf>(sum ? 0 : v, v));
+    v = f(v, dpp_or<0x118, 0xf>(sum ? 0 : v, v));
+    v = f(v, dpp_or<0x142, 0xa>(sum ? 0 : v, v));   // row_bcast:15, 31
+    v = f(v, dpp_or<0x143, 0xc>(sum ? 0 : v, v));
+    return __builtin_amdgcn_readlane(v, 63);
+}
 __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) v = max(v, (uint32_t)__shfl_xor((int)v, o, 64));
-    return v;
+    return (uint32_t)wave_reduce((int)v, [](int a, int b) { return (int)max((uint32_t)a, (uint32_t)b); }, false);
 }
 __device__ __forceinline__ uint32_t wave_min_u32(uint32_t v) {
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) v = min(v, (uint32_t)__shfl_xor((int)v, o, 64));
-    return v;
+    return (uint32_t)wave_reduce((int)v, [](int a, int b) { return (int)min((uint32_t)a, (uint32_t)b); }, false);
 }
 __device__ __forceinline__ int wave_min_i32(int v) {
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) v = min(v, __shfl_xor(v, o, 64));
-    return v;
+    return wave_reduce(v, [](int a, int b) { return min(a, b); }, false);
 }
 __device__ __forceinline__ int wave_max_i32(int v) {
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) v = max(v, __shfl_xor(v, o, 64));
-    return v;
+    return wave_reduce(v, [](int a, int b) { return max(a, b); }, false);
 }
 __device__ __forceinline__ int wave_sum_i32(int v) {
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
+    return wave_reduce(v, [](int a, int b) { return a + b; }, true);
 }
 // NaN-ignoring float extrema over the wave (fmaxf / fminf)
 __device__ __forceinline__ float wave_max_f32(float v) {
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
-    return v;
+    return __int_as_float(wave_reduce(__float_as_int(v), [](int a, int b) {
+        return __float_as_int(fmaxf(__int_as_float(a), __int_as_float(b))); }, false));
 }
 __device__ __forceinline__ float wave_min_f32(float v) {
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) v = fminf(v, __shfl_xor(v, o, 64));
-    return v;
+    return __int_as_float(wave_reduce(__float_as_int(v), [](int a, int b) {
+        return __float_as_int(fminf(__int_as_float(a), __int_as_float(b))); }, false));
 }
 __device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
 

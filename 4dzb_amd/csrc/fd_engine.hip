@@ -77,6 +77,15 @@ void light_setup(const fd_area_light& d, FdLight& L) {
     L.res = W;
     L.resNum = W * H;
     L.wpr = (W <= 32) ? 1 : 2;
+    const double a[3] = {L.xd[0], L.xd[1], L.xd[2]}, b[3] = {L.yd[0], L.yd[1], L.yd[2]};
+    const double n[3] = {a[1] * b[2] - a[2] * b[1], a[2] * b[0] - a[0] * b[2], a[0] * b[1] - a[1] * b[0]};
+    const double nn = n[0] * n[0] + n[1] * n[1] + n[2] * n[2];
+    for (int k = 0; k < 3; ++k) {
+        const int i = (k + 1) % 3, j = (k + 2) % 3;
+        L.X[k] = (float)((b[i] * n[j] - b[j] * n[i]) / nn);
+        L.Y[k] = (float)((n[i] * a[j] - n[j] * a[i]) / nn);
+        L.N[k] = (float)(n[k] / std::sqrt(nn));
+    }
 }
 
 }  // namespace fdh
@@ -196,7 +205,13 @@ size_t layout(FdArgs& a, char* base, bool countOps) {
     a.st = (FdState*)take(sizeof(FdState));
     a.rec = (float4*)take(WH * sizeof(float4));
     a.rxKey = (uint16_t*)take(WH * sizeof(uint16_t));
-    a.histR = (uint32_t*)take(a.nR * sizeof(uint32_t));
+    // the histograms are done with once the tables exist: the work-item records
+    // take their place (and more only where both are a few KB)
+    const size_t hr = ((size_t)a.nR * sizeof(uint32_t) + 255) & ~(size_t)255;
+    char* hist = (char*)take(std::max(hr + (size_t)a.nT * sizeof(uint32_t), (size_t)a.chunkSlots * sizeof(FdChunk)));
+    a.histR = (uint32_t*)hist;
+    a.histT = hist ? (uint32_t*)(hist + hr) : nullptr;
+    a.chunks = (FdChunk*)hist;
     a.sortedId = (int*)take(WH * sizeof(int));
     a.sortedRec = (FdRxRec*)take(WH * sizeof(FdRxRec));
     a.binStat = (uint32_t*)take((size_t)nb * 5 * sizeof(uint32_t));
@@ -204,7 +219,6 @@ size_t layout(FdArgs& a, char* base, bool countOps) {
     a.tri = (FdTri*)take(T * sizeof(FdTri));
     a.triCount = (int*)take(T * sizeof(int));
     a.triRange = (uint2*)take(T * sizeof(uint2));
-    a.histT = (uint32_t*)take(a.nT * sizeof(uint32_t));
     a.triOff = (uint32_t*)take(T * sizeof(uint32_t));
     a.triClass = (uint8_t*)take(T);
     a.pairKT = (uint32_t*)take((size_t)a.pairCap * sizeof(uint32_t));
@@ -763,7 +777,7 @@ size_t build_plan(const std::vector<FdArgs>& args, bool anyTris, char* devBase, 
                 case FD_MAP_TRI: blocks = a.nblkT; break;
                 case FD_MAP_SCANT: blocks = fdk::scan_chunks(a.nT); break;
                 case FD_MAP_SCANO: blocks = fdk::scan_chunks(std::max(a.ntris, 1)); break;
-                case FD_MAP_NB: blocks = nb; break;
+                case FD_MAP_NB: blocks = nb + 1; break;
                 case FD_MAP_ZERO: blocks = a.segs > 1 ? fdk::zero_blocks(a) : 0; break;
                 case FD_MAP_FIN: blocks = a.segs > 1 ? a.chunkSlots : 0; break;
                 default: blocks = a.chunkSlots * a.segs; break;

@@ -16,6 +16,14 @@
 #define FD_ORDER_CACHE 32768   // list entries whose walk keys the area-order pass keeps in LDS
 #define FD_ORDER_THREADS 1024  // threads per bin in the area-order pass
 
+// One occlusion work item: receivers s0 .. s0 + n - 1 of the sorted order and
+// their bin's triangle list.
+struct FdChunk {
+    int s0;
+    int nbin;    // n | bin << 8
+    int ts, te;
+};
+
 // Everything one frame's kernels read, passed by value (kernarg segment).
 struct FdArgs {
     FdLight L;
@@ -64,7 +72,8 @@ struct FdArgs {
     int* rxEnd;           // nb + 1
     int* triStart;        // nb
     int* triEnd;          // nb
-    int* chunkStart;      // nb + 2: work-item prefix over the bins in occlusion order (by rank)
+    int* chunkStart;      // nb + 1: first work item of each bin (in occlusion order)
+    FdChunk* chunks;      // chunkSlots: the work items (over histR / histT, done with by then)
     int* binAtRank;       // nb + 1: occlusion order of the bins, longest triangle list first
     uint64_t* scanPart;   // scan partial sums
     uint32_t* part;       // per-block partials: 8 per k_reduce block (value-major), then 1 per pair-count block
@@ -110,6 +119,24 @@ struct FdArgs {
 #define FD_WAVES8_ITEMS 8192
 inline int fd_default_waves(int wpr, long items) { return (wpr == 2 || items <= FD_WAVES8_ITEMS) ? 8 : 4; }
 inline bool fd_valid_waves(int w) { return w == 2 || w == 4 || w == 8; }
+
+// LDS of an occlusion work item: its light rows ([row][receiver], a stride of
+// 65 words, so that lanes that walk one receiver's rows, or one lane per row,
+// use different banks: the write-out and the prefilter's occupancy pass), the
+// full-row masks (one row word per receiver) and the receivers' rectangles and
+// depths (5 floats).
+#define FD_ROW_STRIDE 65
+inline size_t fd_occ_lds(int wpr, int res) {
+    return (size_t)wpr * res * FD_ROW_STRIDE * sizeof(uint32_t) + 64 * (wpr * sizeof(uint32_t) + 5 * sizeof(float));
+}
+// Column strips of the light grid in the occlusion prefilter
+#define FD_OCC_STRIPS 8
+// The prefilter's test against the receivers' rows: for lists of FD_PRUNE_LIST
+// entries per wave and more, on a block's remaining triangles (FD_PRUNE_LEFT or
+// more) before every FD_PRUNE_STEPS pairs.
+#define FD_PRUNE_LIST 64
+#define FD_PRUNE_LEFT 4
+#define FD_PRUNE_STEPS 24
 
 // Occlusion classes of a batched launch: 32-bit / 64-bit rows x 2 / 4 / 8
 // waves per work item (one launch each).

@@ -15,6 +15,7 @@
 // fixed launch sequence with no host round trip (graph-capturable).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <type_traits>
 #include "fd_device.h"
 #include "fd_kernels.h"
 
@@ -577,48 +578,6 @@ __device__ __forceinline__ TriClamp tri_clamp(const float4 mn, const float4 mx, 
     return c;
 }
 
-// Visits, in ascending bin order, every bin of the light-plane grid that the
-// bin rectangle [sx, ex) x [sy, ey) of at least one lane covers, calling
-// body(bp, i, j, mine) with a wave-uniform bin bp = j << log2G | i and
-// mine = the lane's rectangle holds it.  Two schedules with the same visiting
-// order (so the per-bin ballot ranking of the callers stays stable):
-//  * the union rectangle of the wave, row by row (cheap per bin; best when
-//    the lanes' rectangles overlap);
-//  * "next covered bin": every lane walks its own rectangle and the wave
-//    takes the smallest next bin of any lane (a wave minimum per bin; best
-//    when the rectangles are scattered, where the union is mostly empty).
-// The cheaper one is picked per wave from the union area and the summed
-// rectangle areas.
-template <typename F>
-__device__ __forceinline__ void for_covered_bins(bool has, int sx, int sy, int ex, int ey, int log2G, F&& body) {
-    const int ux0 = uniform(wave_min_i32(has ? sx : 1 << 20));
-    const int uy0 = uniform(wave_min_i32(has ? sy : 1 << 20));
-    const int ux1 = uniform(wave_max_i32(has ? ex : 0));
-    const int uy1 = uniform(wave_max_i32(has ? ey : 0));
-    if (ux1 <= ux0 || uy1 <= uy0) return;
-    const int unionArea = (ux1 - ux0) * (uy1 - uy0);
-    const int sumArea = uniform(wave_sum_i32(has ? (ex - sx) * (ey - sy) : 0));
-    if (unionArea <= 2 * sumArea) {
-        for (int j = uy0; j < uy1; ++j)
-            for (int i = ux0; i < ux1; ++i)
-                body(j << log2G | i, i, j, has && j >= sy && j < ey && i >= sx && i < ex);
-        return;
-    }
-    constexpr int DONE = 1 << 30;
-    int ci = sx, cj = sy;
-    int cur = has ? (cj << log2G | ci) : DONE;
-    for (;;) {
-        const int bp = uniform(wave_min_i32(cur));
-        if (bp == DONE) break;
-        const bool mine = cur == bp;
-        body(bp, bp & ((1 << log2G) - 1), bp >> log2G, mine);
-        if (mine) {
-            if (++ci == ex) { ci = sx; ++cj; }
-            cur = cj < ey ? (cj << log2G | ci) : DONE;
-        }
-    }
-}
-
 // Pair passes: a lane walks its own bin rectangle when it holds at most
 // FD_BIG_AREA bins; larger rectangles (a triangle spanning much of the light
 // plane) are walked by the whole wave, one rectangle at a time, so that one
@@ -740,7 +699,7 @@ __device__ __forceinline__ void tri_count_body(const FdArgs& a, const int blk) {
                 FdTri d;
                 for (int k = 0; k < 3; ++k) { d.v0[k] = v0[k]; d.v1[k] = v1[k]; d.v2[k] = v2[k]; }
                 d.bminx = mn.x; d.bminy = mn.y; d.bmaxx = mx.x; d.bmaxy = mx.y;
-                d.minz = mn.z; d.maxz = mx.z; d.pad0 = 0.0f;
+                d.minz = mn.z; d.maxz = mx.z;
                 // occlusion-side triangle constants, same expressions as
                 // Step5_2_shadowCalPerSample.inl:130 and :7
                 const float ax = v1[0] - v0[0], ay = v1[1] - v0[1], az = v1[2] - v0[2];
@@ -750,6 +709,15 @@ __device__ __forceinline__ void tri_count_body(const FdArgs& a, const int blk) {
                     d.e01[k] = v0[k] - v1[k];
                     d.e12[k] = v1[k] - v2[k];
                     d.e20[k] = v2[k] - v0[k];
+                }
+                {   // light_window's edge term, e the largest edge (1-norm); 2^20 at most, or infinite
+                    auto n1 = [](const float (&v)[3]) { return fabsf(v[0]) + fabsf(v[1]) + fabsf(v[2]); };
+                    auto ni = [](const float (&v)[3]) { return fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fabsf(v[2])); };
+                    const float e = fmaxf(fmaxf(n1(d.e01), n1(d.e12)), n1(d.e20));
+                    const float rl = (float)a.L.res * (ni(a.L.xd) + ni(a.L.yd));
+                    // 52u, 40u (u = 2^-24), 2^-60
+                    d.we = fmaxf(fmaxf(3.0994415e-06f * e, 2.3841858e-06f * e * (e / rl)), 8.6736174e-19f);
+                    if (!(d.we <= 1048576.0f)) d.we = INFINITY;
                 }
                 d.pad1[0] = d.pad1[1] = d.pad1[2] = d.pad1[3] = 0.0f;
                 a.tri[t] = d;
@@ -1093,14 +1061,11 @@ __device__ __forceinline__ void tables_body(const FdArgs& a, const int blk) {
             if (i < w) off += wsum[i];
             all += wsum[i];
         }
-        if (r <= nb) a.chunkStart[r] = off + x - nch;
+        if (r <= nb) a.chunkStart[a.binAtRank[r]] = off + x - nch;
         carry += all;
         __syncthreads();
     }
-    if (threadIdx.x == 0) {
-        a.chunkStart[nb + 1] = carry;
-        s->totalChunks = carry;
-    }
+    if (threadIdx.x == 0) s->totalChunks = carry;
 }
 
 // Area order of one bin's triangle list (frames whose walk order is
@@ -1118,9 +1083,14 @@ __device__ __forceinline__ void tri_order_body(const FdArgs& a, const int bin) {
     __shared__ int keyBase[K];
     __shared__ uint8_t keyCache[FD_ORDER_CACHE];
     const FdState* s = a.st;
-    if (s->status != FD_EXIT_OK || s->triOrder == FD_TRI_ORDER_LIST || bin >= s->nb) return;
-    const int ts = a.triStart[bin], te = a.triEnd[bin];
-    if (te <= ts) return;
+    if (s->status != FD_EXIT_OK || bin > s->nb) return;
+    const int ts = bin < s->nb ? a.triStart[bin] : 0, te = bin < s->nb ? a.triEnd[bin] : 0;
+    {   // the bin's work items: one record each, so that the occlusion finds its own in one load
+        const int c0 = a.chunkStart[bin], rs = a.rxStart[bin], re = a.rxEnd[bin];
+        for (int i = threadIdx.x; rs + 64 * i < re; i += FD_ORDER_THREADS)
+            a.chunks[c0 + i] = FdChunk{rs + 64 * i, min(64, re - rs - 64 * i) | bin << 8, ts, te};
+    }
+    if (s->triOrder == FD_TRI_ORDER_LIST || te <= ts) return;
     const int lane = lane_id(), w = threadIdx.x >> 6;
     int* out = (int*)a.pairKT;
     const int big = s->triOrder == FD_TRI_ORDER_MESH ? mesh_big_class(s->log2G) : -1;
@@ -1263,12 +1233,14 @@ template <>
 struct Bits<uint32_t> {
     static constexpr int width = 32;
     __device__ static int ctz(uint32_t v) { return __builtin_ctz(v); }
+    __device__ static int last(uint32_t v) { return 31 - __builtin_clz(v); }
     __device__ static int popc(uint32_t v) { return __popc(v); }
 };
 template <>
 struct Bits<uint64_t> {
     static constexpr int width = 64;
     __device__ static int ctz(uint64_t v) { return __builtin_ctzll(v); }
+    __device__ static int last(uint64_t v) { return 63 - __builtin_clzll(v); }
     __device__ static int popc(uint64_t v) { return __popcll(v); }
 };
 
@@ -1502,6 +1474,228 @@ __device__ __forceinline__ T row_window(const Edge (&e)[3], float Rf, float mAB)
     return interval_bits<T>(w, (unsigned)(-nlc));
 }
 
+// The light samples that one triangle can occlude from one receiver, bounded
+// by projecting the triangle's three vertices from the receiver Q onto the
+// light's sample grid -- before (and mostly instead of) the edge planes.
+//
+// With a_j = v_j - Q, N the light plane's normal, l = L0 - Q, h = l.N > 0 the
+// light's height over Q and X, Y dual to the sample steps (xd.X = 1,
+// yd.X = N.X = 0), vertex j projects to row r_j = (a_j.X) h / (a_j.N) - l.X
+// and column c_j likewise with Y.
+//
+// Bound.  A set bit (r, c) has every edge value >= -tau in the float
+// coefficients (tau = 4u (|A| R + |B| R + |C|), row_window above), whose own
+// rounding is at most 8u |a|_1 |e|_1 (|l|_inf + R |xd|_inf + R |yd|_inf),
+// u = 2^-24 (a, e: the largest vertex offset and triangle edge); so every
+// exact edge value is >= -T with T = 12.5u a e Ld,
+// Ld = |l|_1 + (R + 1) (|xd|_1 + |yd|_1) (2nd-order terms included).  The
+// edge values of a sample P are |V| times the coordinates alpha_j of P - Q in
+// the basis a_0, a_1, a_2 (V = det(a_0, a_1, a_2) = a_0.n), and the weights
+// w_j = alpha_j (a_j.N) / h sum to 1 with r = sum w_j r_j.  For a_j.N > 0:
+// w_j >= -eta, eta = wmax T / |V|, wmax = max a_j.N / h, so
+//   min r_j - 2 eta (max r_j - min r_j) <= r <= max r_j + 2 eta (max - min).
+// With d_j = projected vertex - Q, |a_j| = (a_j.N / h) |d_j| and |d_j|_1 <=
+// t = Ld + |r_j|max |xd|_1 + |c_j|max |yd|_1 give a <= wmax t.  The record
+// holds we >= max(52u e, 40u e^2 / (R (|xd|_inf + |yd|_inf))), so
+//   q = we Ld t max(wmax, 1) >= 4 T  and  m = wmax q / |V| >= 4 wmax T / |V|
+// (float V).
+// m < 2 keeps the float V at 20u a e^2 or more (the second term of we), its
+// rounding at 9u a e^2: the reference's sign of it is the exact one, the
+// exact |V| at least half of it, and m >= 2 eta.  The projections are off by less
+// than 64u t (1 + t / h) |X|_inf rows (axial lights: 11u (|r| + |l.X|), with
+// |l.X| <= 2^12 under 2^-8), which with a constant makes the rest of the
+// margin (vertices beyond |r| = 512 are off by a larger amount, but outside
+// the grid by far more).  Vertices at or below Q,
+// projections beyond 2^21 and NaN leave the window unknown: the caller then
+// uses the exact row range and row_window.  (we <= 2^20, or infinite, and
+// Ld t <= 2^40 keep the planes of the others finite, |A|, |B| < 2^78; q is at
+// least 2^-100, which keeps underflow out of T.)  q is also at least
+// 52u (|A| R + |B| R + |C|) of every edge.
+//
+// What bounds it: the VALU.  add, mul, fma and the bit operations on vector
+// registers or literals issue at twice the rate of everything else (compares,
+// selects, min/max, conversions, shifts, and any operation with a scalar
+// register operand: 2.4 against 4.2 cycles per wave and SIMD measured), so
+// rounding to integers goes through the addition of 1.5 * 2^23 and the tests
+// are sign bits of integer differences, combined by and / or.
+struct LightProj {   // uniform
+    float kL, kr, kc;   // Ld^2, Ld |xd|_1, Ld |yd|_1 for the work item's largest Ld; infinite: no window
+    float er, ec, iL;   // 64u |X|_inf, 64u |Y|_inf, 1 / Ld (lights that are not axial)
+};
+
+constexpr float WIN_MAGIC = 12582912.0f;       // 1.5 * 2^23: x + WIN_MAGIC holds the nearest integer of x in its low bits
+constexpr int WIN_BASE = 0x4b400000;           // its bits: the integer is bits - WIN_BASE
+constexpr float WIN_MARGIN = 0.0078125f;       // 2^-7 rows / columns
+constexpr float WIN_MAX_OFFSET = 4096.0f;      // largest |l.X|, |l.Y| of axial lights (2^12)
+
+// a: vertices in the light's frame (axial lights: the world's; else X, Y, N);
+// h: light height; hr, hc: rows / columns per unit of a.x, a.y at that height;
+// nr, nc: -l.X - 1/2, -l.Y - 1/2.  Returns whether a sample may be set: the
+// rows are lo - WIN_BASE .. hi - WIN_BASE where known < 0, else unknown.
+template <bool AXIAL>
+__device__ __forceinline__ bool light_window(const LightProj& P, const float (&a)[3][3], float h, float hr, float hc,
+                                             float nr, float nc, float V, float we, int nsubBits, int& lo, int& hi,
+                                             int& known, float& q) {
+    float r[3], c[3], ra[3];
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+        ra[j] = __builtin_amdgcn_rcpf(a[j][2]);
+        r[j] = __builtin_fmaf(a[j][0] * ra[j], hr, nr);
+        c[j] = __builtin_fmaf(a[j][1] * ra[j], hc, nc);
+    }
+    const float rwmin = fminf(fminf(ra[0], ra[1]), ra[2]) * h;   // 1 / wmax
+    const float rmin = fminf(fminf(r[0], r[1]), r[2]), rmax = fmaxf(fmaxf(r[0], r[1]), r[2]);
+    const float cmin = fminf(fminf(c[0], c[1]), c[2]), cmax = fmaxf(fmaxf(c[0], c[1]), c[2]);
+    const float rs = fabsf(rmin) + fabsf(rmax), cs = fabsf(cmin) + fabsf(cmax);
+    const float t = __builtin_fmaf(rs, P.kr, __builtin_fmaf(cs, P.kc, P.kL));   // Ld t
+    const float den = fabsf(V) * rwmin;
+    const float m = (we * t) * __builtin_amdgcn_rcpf(den * fminf(rwmin, 1.0f));
+    q = m * den;
+    float mr = WIN_MARGIN, mc = WIN_MARGIN;
+    if (!AXIAL) {
+        const float tt = t * P.iL;
+        const float e = __builtin_fmaf(tt * __builtin_amdgcn_rcpf(h), tt, tt);
+        mr = __builtin_fmaf(e, P.er, mr);
+        mc = __builtin_fmaf(e, P.ec, mc);
+    }
+    mr = __builtin_fmaf(m, rmax - rmin, mr);
+    mc = __builtin_fmaf(m, cmax - cmin, mc);
+    // nearest integers of (bound - 1/2) + 1 and (bound - 1/2): the ceiling of
+    // the lower, the floor of the upper bound
+    lo = __float_as_int((rmin - mr) + (WIN_MAGIC + 1.0f));
+    hi = __float_as_int((rmax + mr) + WIN_MAGIC);
+    const int clo = __float_as_int((cmin - mc) + (WIN_MAGIC + 1.0f));
+    const int chi = __float_as_int((cmax + mc) + WIN_MAGIC);
+    // negative: no row or no column of the grid
+    const int none = (hi - lo) | (hi - WIN_BASE) | (nsubBits - lo) | (chi - clo) | (chi - WIN_BASE) | (nsubBits - clo);
+    // negative: m < 2 (a NaN is not, of either sign), rs + cs < 2^21, rwmin > 0
+    known = ((__float_as_int(m) & 0x7fffffff) - 0x40000000) & (__float_as_int(rs + cs) - 0x4a000000) &
+            __float_as_int(0.0f - rwmin);
+    return (none & known) >= 0;
+}
+
+// The same for all receivers of a work item at once, one triangle per lane
+// (the block prefilter): bounds of the rows and columns over the receivers'
+// box.  In the light's frame relative to L0 (rows, columns, height; the
+// light plane at height 0), the line from Q through v meets the light at
+// row v.x + (v.x - Q.x) k, k = -v.z / (v.z - Q.z), so each vertex gives an
+// interval over the box, and V = det / |xd x yd|^-1 is linear in Q.  The
+// frame's coordinates, dz and k are off by at most 2^-18 S (1 + |k|)(1 + S / dz)
+// of a row (times |X|_inf), S = the largest 1-norm of a vertex or receiver
+// relative to L0.  m <= 1/8 here (the float V is off by a further 20u a e^2).
+struct TileBox {   // uniform
+    float x0, x1, y0, y1, z0, z1;   // receivers in the light's frame relative to L0
+    float Ld, tr, tc;               // the largest Ld; |xd|_1, |yd|_1
+    float sx, sy;                   // |X|_inf, |Y|_inf
+    float A;                        // |xd x yd|
+};
+
+// v: vertices in the frame relative to L0, S0: their largest 1-norm in the
+// world.  Returns whether rows lo..hi and columns clo..chi (clipped to the
+// grid; lo > hi: none) bound every sample the triangle can set.
+__device__ __forceinline__ bool tile_window(const TileBox& b, const float (&v)[3][3], float S0, float we, int n, int& lo,
+                                            int& hi, int& clo, int& chi) {
+    float rmin = 3.0e38f, rmax = -3.0e38f, cmin = 3.0e38f, cmax = -3.0e38f, kk = 0.0f, idz = 0.0f, g = 1.0f;   // g >= wmax, 1
+    bool ok = true;
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+        const float x = v[j][0], y = v[j][1], z = v[j][2];
+        const float dz1 = z - b.z1, i1 = __builtin_amdgcn_rcpf(dz1);
+        const float k0 = -z * __builtin_amdgcn_rcpf(z - b.z0), k1 = -z * i1;
+        ok = ok && dz1 > 0.0f;
+        const float dx0 = x - b.x1, dx1 = x - b.x0, dy0 = y - b.y1, dy1 = y - b.y0;
+        const float xa = dx0 * k0, xb = dx0 * k1, xc = dx1 * k0, xd = dx1 * k1;
+        const float ya = dy0 * k0, yb = dy0 * k1, yc = dy1 * k0, yd = dy1 * k1;
+        rmin = fminf(rmin, x + fminf(fminf(xa, xb), fminf(xc, xd)));
+        rmax = fmaxf(rmax, x + fmaxf(fmaxf(xa, xb), fmaxf(xc, xd)));
+        cmin = fminf(cmin, y + fminf(fminf(ya, yb), fminf(yc, yd)));
+        cmax = fmaxf(cmax, y + fmaxf(fmaxf(ya, yb), fmaxf(yc, yd)));
+        kk = fmaxf(kk, fabsf(k1));
+        g = fmaxf(g, (z - b.z0) / -b.z1);
+        idz = fmaxf(idz, i1);
+    }
+    const float e1[3] = {v[1][0] - v[0][0], v[1][1] - v[0][1], v[1][2] - v[0][2]};
+    const float e2[3] = {v[2][0] - v[1][0], v[2][1] - v[1][1], v[2][2] - v[1][2]};
+    const float n0 = e1[1] * e2[2] - e1[2] * e2[1], n1 = e1[2] * e2[0] - e1[0] * e2[2], n2 = e1[0] * e2[1] - e1[1] * e2[0];
+    const float Vc = dot3(v[0][0] - 0.5f * (b.x0 + b.x1), v[0][1] - 0.5f * (b.y0 + b.y1), v[0][2] - 0.5f * (b.z0 + b.z1),
+                          n0, n1, n2);
+    const float Vh = dot3(0.5f * (b.x1 - b.x0), 0.5f * (b.y1 - b.y0), 0.5f * (b.z1 - b.z0), fabsf(n0), fabsf(n1), fabsf(n2));
+    const float V = (fabsf(Vc) - Vh) * b.A;
+    const float S = fmaxf(S0, b.Ld);
+    const float t = b.Ld + (fabsf(rmin) + fabsf(rmax)) * b.tr + (fabsf(cmin) + fabsf(cmax)) * b.tc;
+    const float m = we * b.Ld * t * (g * g) / V;
+    const float E = 3.814697265625e-06f * S * (1.0f + kk) * (1.0f + S * idz);
+    const float mr = m * (rmax - rmin) + (E * b.sx + WIN_MARGIN), mc = m * (cmax - cmin) + (E * b.sy + WIN_MARGIN);
+    ok = ok && V > 0.0f && m <= 0.125f && mr <= 4194304.0f && mc <= 4194304.0f;
+    const float nf = (float)n;
+    lo = (int)__builtin_amdgcn_fmed3f(ceilf(rmin - mr), 0.0f, nf + 1.0f);
+    hi = (int)__builtin_amdgcn_fmed3f(floorf(rmax + mr), -1.0f, nf);
+    clo = (int)__builtin_amdgcn_fmed3f(ceilf(cmin - mc), 0.0f, nf + 1.0f);
+    chi = (int)__builtin_amdgcn_fmed3f(floorf(cmax + mc), -1.0f, nf);
+    return ok;
+}
+
+// Which rows still lack samples of some receiver, per strip of columns: U[s]
+// has bit r set when row r is not full in the columns [s << lsw, (s + 1) <<
+// lsw) of every receiver of the work item.  Lane r ands the receivers' words
+// of row r (FD_ROW_STRIDE keeps the lanes on different banks); the other waves
+// may add bits meanwhile, which only makes the answer older.
+template <typename T>
+__device__ __forceinline__ void row_occupancy(const uint32_t* lds, int R, int lsw, T FULL, uint64_t (&U)[FD_OCC_STRIPS]) {
+    const int lane = lane_id();
+    T a = ~(T)0;
+    if constexpr (Bits<T>::width == 32) {   // half the receivers per half wave
+        const int r = min(lane & 31, R - 1);
+        const uint32_t* p = lds + r * FD_ROW_STRIDE + (lane & 32);
+        uint32_t x = ~0u;
+#pragma unroll 8
+        for (int l = 0; l < 32; ++l) x &= p[l];
+        x &= (uint32_t)__shfl_xor((int)x, 32, 64);
+        a = (T)x;
+    } else {
+        const int r = min(lane, R - 1);
+        const uint32_t* p = lds + r * FD_ROW_STRIDE;
+        const uint32_t* p1 = p + R * FD_ROW_STRIDE;
+        uint32_t x = ~0u, y = ~0u;
+#pragma unroll 8
+        for (int l = 0; l < 64; ++l) {
+            x &= p[l];
+            y &= p1[l];
+        }
+        a = (T)(((uint64_t)y << 32) | x);
+    }
+    a = ~a & FULL;
+    const uint64_t rows = R >= 64 ? ~0ull : (1ull << R) - 1ull;
+    const T strip = (T)(((T)1 << (1 << lsw)) - (T)1);
+#pragma unroll
+    for (int s = 0; s < FD_OCC_STRIPS; ++s)
+        U[s] = (s << lsw) < R ? __ballot((a & (T)(strip << (s << lsw))) != (T)0) & rows : 0ull;
+}
+
+// One row of a pair with finite planes, decided with exact quotients: the AND
+// of the three edge masks, empty when the row is not in the reference's
+// row-range mask (three_edges<T, true>).  The reference only visits rows of
+// that mask.
+template <typename T>
+__device__ __forceinline__ T row_exact(const Edge (&e)[3], float fr, float nsub, int R) {
+    const int r = (int)fr;
+    T m = (R >= Bits<T>::width) ? ~(T)0 : (((T)1 << R) - (T)1);
+    bool in = true;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        float A = e[k].A, B = e[k].B;
+        asm volatile("" : "+v"(A), "+v"(B));   // rare: keep the divisions out of the caller's set-up
+        const float DN = (B > 0 ? B * nsub : 0.0f) + e[k].C;
+        const bool f1 = DN >= 0.0f, f2 = (A * nsub + DN) >= 0.0f;
+        in = in && (f1 == f2 ? f1 : f1 == (r < k_exact(DN, A, R)));
+        const float D = A * fr + e[k].C;
+        const bool g1 = D >= 0.0f, g2 = (B * nsub + D) >= 0.0f;
+        const T low = low_mask<T>(k_exact(D, B, R));
+        m &= g1 == g2 ? (g1 ? ~(T)0 : (T)0) : (g1 ? low : ~low);
+    }
+    return in ? m : (T)0;
+}
+
 // test3DPointInTriangle, Step5_2_shadowCal.inl:213-222
 __device__ __forceinline__ bool point_in_tri(const float* A, const float* B, const float* C, float px, float py, float pz) {
     auto cross = [](float ax, float ay, float az, float bx, float by, float bz, float* o) {
@@ -1516,11 +1710,17 @@ __device__ __forceinline__ bool point_in_tri(const float* A, const float* B, con
     return true;
 }
 
-// The work item's rows go out; LDS holds row r's low words at [r][lane],
-// the high words (64-bit rows) R rows further.  The waves of the work item
+// Receiver of word j of a work item's masks, iper = 1 / (words per receiver):
+// j / per, exact as j + 1/2 stays 1/2 word from a receiver's ends while the
+// float product is off by less than 2^-16 (j < 2^13).
+__device__ __forceinline__ int word_receiver(int j, float iper) { return (int)(((float)j + 0.5f) * iper); }
+
+// The work item's rows go out; LDS holds row r's low words at [r][lane]
+// (FD_ROW_STRIDE words per row), the high words (64-bit rows) R rows further.  The waves of the work item
 // share the write-out.
 __device__ __forceinline__ void store_masks(const FdArgs& a, const uint32_t* lds, int id, int n, int R, int wpr,
                                             int wave = 0, int waves = 1) {
+    const float iper = 1.0f / (float)(R * wpr);
     // coalesced write-out: consecutive lanes write consecutive words of one
     // receiver's mask (rows x wpr words); the receiver id comes from its
     // lane by a cross-lane read with every lane active
@@ -1528,28 +1728,29 @@ __device__ __forceinline__ void store_masks(const FdArgs& a, const uint32_t* lds
     const int total = n * per;
     for (int j0 = wave * 64; j0 < total; j0 += 64 * waves) {
         const int j = j0 + lane_id();
-        const int l = min(j, total - 1) / per, w = j - l * per;
+        const int l = word_receiver(min(j, total - 1), iper), w = j - l * per;
         const int idl = __shfl(id, l, 64);
         if (j < total) {
-            const int r = w / wpr, h = w - r * wpr;
-            a.masks[(size_t)idl * per + w] = lds[(h * R + r) * 64 + l];
+            const int r = w >> (wpr - 1), h = w & (wpr - 1);
+            a.masks[(size_t)idl * per + w] = lds[(h * R + r) * FD_ROW_STRIDE + l];
         }
     }
 }
 
 // Masks of n receivers (lane l holds the id of receiver l) set to all
 // occluded (back) or none, written straight to the output.
-__device__ __forceinline__ void fill_masks(const FdArgs& a, int id, bool back, int n, int R, int wpr) {
+__device__ __forceinline__ void fill_masks(const FdArgs& a, int id, bool back, int n, int R, int wpr, int wave, int waves) {
     const int per = R * wpr;
     const int total = n * per;
+    const float iper = 1.0f / (float)per;
     const uint32_t w0 = (R >= 32) ? 0xffffffffu : ((1u << R) - 1u);
     const uint32_t w1 = (R >= 64) ? 0xffffffffu : (R > 32 ? (1u << (R - 32)) - 1u : 0u);
-    for (int j0 = 0; j0 < total; j0 += 64) {
+    for (int j0 = wave * 64; j0 < total; j0 += 64 * waves) {
         const int j = j0 + lane_id();
-        const int l = min(j, total - 1) / per, w = j - l * per;
+        const int l = word_receiver(min(j, total - 1), iper), w = j - l * per;
         const int idl = __shfl(id, l, 64);
         const bool bk = __shfl((int)back, l, 64) != 0;
-        if (j < total) a.masks[(size_t)idl * per + w] = bk ? ((w % wpr) == 0 ? w0 : w1) : 0u;
+        if (j < total) a.masks[(size_t)idl * per + w] = bk ? ((w & (wpr - 1)) == 0 ? w0 : w1) : 0u;
     }
 }
 
@@ -1557,29 +1758,19 @@ __device__ __forceinline__ void fill_masks(const FdArgs& a, int id, bool back, i
 // the (zeroed) output; same word order as store_masks.
 __device__ __forceinline__ void or_masks(const FdArgs& a, const uint32_t* lds, int id, int n, int R, int wpr,
                                          int wave = 0, int waves = 1) {
+    const float iper = 1.0f / (float)(R * wpr);
     const int per = R * wpr;
     const int total = n * per;
     for (int j0 = wave * 64; j0 < total; j0 += 64 * waves) {
         const int j = j0 + lane_id();
-        const int l = min(j, total - 1) / per, w = j - l * per;
+        const int l = word_receiver(min(j, total - 1), iper), w = j - l * per;
         const int idl = __shfl(id, l, 64);
         if (j < total) {
-            const int r = w / wpr, h = w - r * wpr;
-            const uint32_t v = lds[(h * R + r) * 64 + l];
+            const int r = w >> (wpr - 1), h = w & (wpr - 1);
+            const uint32_t v = lds[(h * R + r) * FD_ROW_STRIDE + l];
             if (v) atomicOr(a.masks + (size_t)idl * per + w, v);
         }
     }
-}
-
-// Work item -> rank of its bin in the occlusion order: binary search over
-// the work-item prefix (the bin is binAtRank[rank]).
-__device__ __forceinline__ int chunk_rank(const FdArgs& a, int c, int nb) {
-    int lo = 0, hi = nb + 1;
-    while (hi - lo > 1) {
-        const int mid = (lo + hi) >> 1;
-        if (a.chunkStart[mid] <= c) lo = mid; else hi = mid;
-    }
-    return uniform(lo);
 }
 
 // --------------------------------------------------------------------------
@@ -1638,7 +1829,7 @@ __device__ __forceinline__ float bcast(float v, int l) {
 
 // The triangle loop of the variant for one work item: n receivers (lane s
 // holds receiver s in q), triangle list entries [ts, te).  Rows go to lds
-// (row r of receiver s at lds[r * 64 + s], high words R * 64 further).
+// (row r of receiver s at lds[r * FD_ROW_STRIDE + s], high words R rows further).
 template <typename T>
 __device__ __forceinline__ void cta_tris(const FdArgs& a, uint32_t* lds, T* fullRows, int ts, int te, int n,
                                          const FdRxRec& q, int R) {
@@ -1738,11 +1929,11 @@ __device__ __forceinline__ void cta_tris(const FdArgs& a, uint32_t* lds, T* full
                 if (m != (T)0) {
                     T cur;
                     if (Bits<T>::width == 32) {
-                        cur = (T)(atomicOr(lds + i * 64 + s, (uint32_t)m) | (uint32_t)m);
+                        cur = (T)(atomicOr(lds + i * FD_ROW_STRIDE + s, (uint32_t)m) | (uint32_t)m);
                     } else {
                         const uint64_t mm = (uint64_t)m;
-                        const uint32_t lo = atomicOr(lds + i * 64 + s, (uint32_t)mm) | (uint32_t)mm;
-                        const uint32_t hi = atomicOr(lds + (R + i) * 64 + s, (uint32_t)(mm >> 32)) | (uint32_t)(mm >> 32);
+                        const uint32_t lo = atomicOr(lds + i * FD_ROW_STRIDE + s, (uint32_t)mm) | (uint32_t)mm;
+                        const uint32_t hi = atomicOr(lds + (R + i) * FD_ROW_STRIDE + s, (uint32_t)(mm >> 32)) | (uint32_t)(mm >> 32);
                         cur = (T)(((uint64_t)hi << 32) | lo);
                     }
                     if (cur == FULL) atomicOr(fullRows + s, (T)1 << i);
@@ -1758,8 +1949,8 @@ __device__ __forceinline__ void cta_tris(const FdArgs& a, uint32_t* lds, T* full
 // merged with LDS atomics), so a CU holds twice the waves for the same LDS.
 template <typename T, bool COUNT, bool CTA = false, int NW = 1>
 __device__ __forceinline__ void occlude_body(const FdArgs& a, const int blkIn) {
-    // wpr * R * 64 row words, then 64 full-row masks (T, 64-bit atomics for
-    // 64-bit rows: the array is aligned for them)
+    // wpr * R rows of FD_ROW_STRIDE words, then 64 full-row masks (T, 64-bit
+    // atomics for 64-bit rows: the array is aligned for them)
     extern __shared__ __align__(16) uint32_t lds[];
     const FdState* s = a.st;
     const int status = s->status;
@@ -1775,7 +1966,7 @@ __device__ __forceinline__ void occlude_body(const FdArgs& a, const int blkIn) {
     const int c = blkIn - seg * a.chunkSlots;
 
     if (status != FD_EXIT_OK) {
-        if (seg != 0 || wv != 0) return;
+        if (seg != 0) return;
         // early exit of the frame: every receiver shadow 0, except back-facing
         // receivers once the back-face stage has run (FD/api.cpp:489,
         // Step2_1_samplerRectangleAABB.inl:97)
@@ -1786,21 +1977,21 @@ __device__ __forceinline__ void occlude_body(const FdArgs& a, const int blkIn) {
         bool back = false;
         if (lane < n) {
             back = backStage && __float_as_uint(a.rec[i0 + lane].w) == FD_TAG_BACK;
-            a.shadow[i0 + lane] = back ? 1.0f : 0.0f;
+            if (wv == 0) a.shadow[i0 + lane] = back ? 1.0f : 0.0f;
         }
-        fill_masks(a, i0 + lane, back, n, R, wpr);
+        fill_masks(a, i0 + lane, back, n, R, wpr, wv, NW);
         return;
     }
     if (c >= s->totalChunks) return;
     const int nb = s->nb;
-    const int rank = chunk_rank(a, c, nb);
-    const int bin = uniform(a.binAtRank[rank]);
+    const FdChunk ck = a.chunks[c];
+    const int bin = ck.nbin >> 8, n = ck.nbin & 255;
     if (bin == nb && seg != 0) return;
     // this work item's stretch of the bin's triangle list (bins 0..nb-1)
     int ts = 0, te = 0;
     if (bin != nb) {
-        ts = a.triStart[bin];
-        te = a.triEnd[bin];
+        ts = ck.ts;
+        te = ck.te;
         if (S > 1) {
             int per = (te - ts + S - 1) / S;
             if (CTA) per = (per + 31) & ~31;   // stretches keep the groups of 32
@@ -1809,8 +2000,7 @@ __device__ __forceinline__ void occlude_body(const FdArgs& a, const int blkIn) {
             if (ts >= te) return;   // nothing to add; the finishing pass counts the merged masks
         }
     }
-    const int s0 = a.rxStart[bin] + (c - a.chunkStart[rank]) * 64;
-    const int n = min(64, a.rxEnd[bin] - s0);
+    const int s0 = ck.s0;
     const bool act = lane < n;
     int id = 0;
     if (act) id = a.sortedId[s0 + lane];
@@ -1818,30 +2008,40 @@ __device__ __forceinline__ void occlude_body(const FdArgs& a, const int blkIn) {
 
     if (bin == nb) {
         // receivers outside the light plane, invalid or back-facing
-        if (wv != 0) return;
         bool back = false;
         if (act) {
             back = __float_as_uint(a.rec[id].w) == FD_TAG_BACK;
-            a.shadow[id] = back ? 1.0f : 0.0f;
+            if (wv == 0) a.shadow[id] = back ? 1.0f : 0.0f;
         }
-        fill_masks(a, id, back, n, R, wpr);
+        fill_masks(a, id, back, n, R, wpr, wv, NW);
         return;
     }
 
     FdRxRec q{};
     if (act) q = a.sortedRec[s0 + lane];
+    // rows of lanes without a receiver start full (row_occupancy)
     for (int r = wv; r < R; r += NW) {
-        lds[r * 64 + lane] = 0u;
-        if (wpr == 2) lds[(R + r) * 64 + lane] = 0u;
+        lds[r * FD_ROW_STRIDE + lane] = act ? 0u : (uint32_t)FULL;
+        if (wpr == 2) lds[(R + r) * FD_ROW_STRIDE + lane] = act ? 0u : (uint32_t)((uint64_t)FULL >> 32);
     }
     // rows shared by several waves: the rows each receiver has full, as any
     // wave found them (after the rows)
     constexpr bool SHARE_FULL = NW > 1 && !CTA;
-    T* const fullSh = (T*)(lds + wpr * R * 64);
-    if (SHARE_FULL && wv == 0) fullSh[lane] = (T)0;
+    T* const fullSh = (T*)(lds + wpr * R * FD_ROW_STRIDE);
+    // the receivers' rectangles and depths (after the full-row masks), for the
+    // cull of the few pairs that get there: five registers more per lane spill
+    float* const rectSh = (float*)(fullSh + 64);
+    if (!CTA && wv == 0) {
+        fullSh[lane] = (T)0;
+        rectSh[lane] = q.rminx;
+        rectSh[64 + lane] = q.rminy;
+        rectSh[128 + lane] = q.rmaxx;
+        rectSh[192 + lane] = q.rmaxy;
+        rectSh[256 + lane] = q.z;
+    }
     if (NW > 1) __syncthreads();
     if (CTA) {
-        T* fullRows = (T*)(lds + wpr * R * 64);
+        T* fullRows = (T*)(lds + wpr * R * FD_ROW_STRIDE);
         fullRows[lane] = (T)0;
         __syncthreads();
         cta_tris<T>(a, lds, fullRows, ts, te, n, q, R);
@@ -1849,8 +2049,8 @@ __device__ __forceinline__ void occlude_body(const FdArgs& a, const int blkIn) {
         if (S == 1) {
             int cnt = 0;
             for (int r = 0; r < R; ++r) {
-                cnt += __popc(lds[r * 64 + lane]);
-                if (wpr == 2) cnt += __popc(lds[(R + r) * 64 + lane]);
+                cnt += __popc(lds[r * FD_ROW_STRIDE + lane]);
+                if (wpr == 2) cnt += __popc(lds[(R + r) * FD_ROW_STRIDE + lane]);
             }
             if (act) a.shadow[id] = (float)cnt / (float)a.L.resNum;   // :1080-1088
             store_masks(a, lds, id, n, R, wpr);
@@ -1873,6 +2073,67 @@ __device__ __forceinline__ void occlude_body(const FdArgs& a, const int blkIn) {
     const float Rf = (float)R;
     const float Rs = Rf + 2.44140625e-4f;   // R + 2^-12, exact
     const float eps = a.eps;
+    auto su = [](float v) { return __int_as_float(uniform(__float_as_int(v))); };   // into a scalar register
+    // the projected sample window's constants.  Axial lights below their
+    // receivers take the general form, whose normal can point either way.
+    const bool axialW = axial && su(Lz) > 0.0f;
+    LightProj P;
+    TileBox tb{};
+    const bool longList = te - ts >= FD_PRUNE_LIST * NW;   // the prune pays
+    float hw, hr, hc, nr, nc;   // light_window's h, hr, hc, nr, nc
+    float sgN = 1.0f;           // the light-plane normal's sign towards the light
+    {
+        auto n1 = [](const float (&v)[3]) { return fabsf(v[0]) + fabsf(v[1]) + fabsf(v[2]); };
+        auto ni = [](const float (&v)[3]) { return fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fabsf(v[2])); };
+        const float x1 = n1(a.L.xd), y1 = n1(a.L.yd);
+        float off = 0.0f;   // |l.X|, |l.Y| of axial lights
+        if (axialW) {
+            hw = Lz;
+            hr = Lz * a.L.X[0];
+            hc = Lz * a.L.Y[1];
+            nr = -__builtin_fmaf(Lx, a.L.X[0], 0.5f);
+            nc = -__builtin_fmaf(Ly, a.L.Y[1], 0.5f);
+            off = fmaxf(fabsf(nr), fabsf(nc));
+        } else {
+            hw = dot3(Lx, Ly, Lz, a.L.N[0], a.L.N[1], a.L.N[2]);
+            if (su(hw) < 0.0f) sgN = -1.0f;
+            hw *= sgN;
+            hr = hc = hw;
+            nr = -(dot3(Lx, Ly, Lz, a.L.X[0], a.L.X[1], a.L.X[2]) + 0.5f);
+            nc = -(dot3(Lx, Ly, Lz, a.L.Y[0], a.L.Y[1], a.L.Y[2]) + 0.5f);
+        }
+        const float L1 = fabsf(Lx) + fabsf(Ly) + fabsf(Lz);
+        float Ld = wave_max_f32(act ? L1 : 0.0f) + (Rf + 1.0f) * (x1 + y1);
+        // Ld t is at most Ld (Ld + 2^21 (|xd|_1 + |yd|_1)); receivers at or above the light have no window
+        if (!(Ld >= 9.5367431640625e-07f && Ld * (Ld + 2097152.0f * (x1 + y1)) <= 1.09951163e+12f) ||
+            __any(act && !(L1 <= Ld && hw > 0.0f && off <= WIN_MAX_OFFSET)))
+            Ld = INFINITY;
+        P.kL = Ld * Ld;
+        P.kr = Ld * x1;
+        P.kc = Ld * y1;
+        P.iL = 1.0f / Ld;
+        P.er = 3.814697265625e-06f * ni(a.L.X);
+        P.ec = 3.814697265625e-06f * ni(a.L.Y);
+        if (longList) {
+            // receivers relative to L0: -l in the frame
+            tb.x0 = wave_min_f32(act ? nr + 0.5f : INFINITY);
+            tb.x1 = wave_max_f32(act ? nr + 0.5f : -INFINITY);
+            tb.y0 = wave_min_f32(act ? nc + 0.5f : INFINITY);
+            tb.y1 = wave_max_f32(act ? nc + 0.5f : -INFINITY);
+            tb.z0 = wave_min_f32(act ? -hw : INFINITY);
+            tb.z1 = wave_max_f32(act ? -hw : -INFINITY);
+            tb.Ld = Ld;
+            tb.tr = x1;
+            tb.tc = y1;
+            tb.sx = ni(a.L.X);
+            tb.sy = ni(a.L.Y);
+            const float cx = xd1 * yd2 - xd2 * yd1, cy = xd2 * yd0 - xd0 * yd2, cz = xd0 * yd1 - xd1 * yd0;
+            tb.A = sqrtf(cx * cx + cy * cy + cz * cz);
+        }
+    }
+    // strips of 1 << lsw columns: 8 cover the grid
+    const int lsw = R <= 8 ? 0 : R <= 16 ? 1 : R <= 32 ? 2 : 3;
+    const int nsubBits = WIN_BASE + R - 1;
     T full = 0;
     unsigned long long nCand = 0, nPass = 0, nRows = 0, nWaveIt = 0, nWaveRows = 0, nRefRows = 0, nPlanes = 0;
     // read-only for this kernel: the constant address space lets the uniform
@@ -1901,29 +2162,29 @@ __device__ __forceinline__ void occlude_body(const FdArgs& a, const int blkIn) {
     const int* listV = walkOrder != FD_TRI_ORDER_LIST ? (const int*)a.pairKT : a.sortedTri;
     float gx0 = 0.0f, gy0 = 0.0f, gx1 = 0.0f, gy1 = 0.0f, gz = 0.0f;
     if (!COUNT) {
-        auto su = [](float v) { return __int_as_float(uniform(__float_as_int(v))); };   // into a scalar register
-        gx0 = su(wave_max_f32(act ? q.rminx : -INFINITY));
-        gy0 = su(wave_max_f32(act ? q.rminy : -INFINITY));
-        gx1 = su(wave_min_f32(act ? q.rmaxx : INFINITY));
-        gy1 = su(wave_min_f32(act ? q.rmaxy : INFINITY));
-        gz = su(wave_max_f32(act ? q.z : -INFINITY));
+        gx0 = wave_max_f32(act ? q.rminx : -INFINITY);
+        gy0 = wave_max_f32(act ? q.rminy : -INFINITY);
+        gx1 = wave_min_f32(act ? q.rmaxx : INFINITY);
+        gy1 = wave_min_f32(act ? q.rmaxy : INFINITY);
+        gz = wave_max_f32(act ? q.z : -INFINITY);
     }
-    // one pair (triangle tid, this wave's receivers): cull, planes, rows
-    auto step = [&](const int tid) {
+    // one pair (triangle tid, this wave's receivers): sample window, cull,
+    // planes, rows
+    auto step = [&](const int tid, auto axialT) {
+        constexpr bool AXIAL = decltype(axialT)::value;
         if ((unsigned)tid >= (unsigned)a.ntris) return;   // defensive: pair entries are triangle ids
-        if (SHARE_FULL) {   // rows the other waves filled
-            full |= (T)fullSh[lane];
-            if (full == FULL) live = false;
-        }
         const FdTri t = tris[tid];
-        // the whole record in one round trip (the prefiltered pairs mostly
-        // pass the cull below, which needs only part of it)
+        // the whole record in one round trip
         if (!COUNT) asm volatile("" ::"s"(t.v0[0]), "s"(t.bminx), "s"(t.minz), "s"(t.n[0]), "s"(t.e20[0]));
         // containment + depth cull (:120-127)
-        const bool pass = live && t.bminx <= q.rminx && t.bminy <= q.rminy && q.rmaxx <= t.bmaxx &&
-                          q.rmaxy <= t.bmaxy && t.minz <= q.z;
-        if (!pass) return;
-        if (COUNT) ++nPass;
+        auto culled = [&]() {
+            const float* rc = rectSh + lane;   // rminx, rminy, rmaxx, rmaxy, z
+            return !(t.bminx <= rc[0] && t.bminy <= rc[64] && rc[128] <= t.bmaxx && rc[192] <= t.bmaxy && t.minz <= rc[256]);
+        };
+        if (COUNT) {
+            if (!live || culled()) return;
+            ++nPass;
+        }
         // planes (Q,v0,v1), (Q,v1,v2), (Q,v2,v0) (:150-172) start from
         // a_k = v_{k+1} - Q; a_2 = v0 - Q also gives
         // dir = dot(Q - v0, n) (:130-132) = -dot(v0 - Q, n), exactly (every
@@ -1944,11 +2205,42 @@ __device__ __forceinline__ void occlude_body(const FdArgs& a, const int blkIn) {
         // outcome is the same: a skipped pair sets nothing).
         const bool onTri = fabsf(ndir) < eps;
         if (COUNT && onTri && point_in_tri(t.v0, t.v1, t.v2, q.q[0], q.q[1], q.q[2])) return;
+        // samples that can be set, from the projected vertices; most pairs of
+        // small triangles end here
+        int lo, hi, known;
+        float tol;
+        bool may;
+        if constexpr (AXIAL) {
+            may = light_window<true>(P, av, hw, hr, hc, nr, nc, ndir, t.we, nsubBits, lo, hi, known, tol);
+        } else {
+            float af[3][3];
+#pragma unroll
+            for (int k = 0; k < 3; ++k)
+#pragma unroll
+                for (int d = 0; d < 3; ++d) {
+                    const float (&u)[3] = d == 0 ? a.L.X : d == 1 ? a.L.Y : a.L.N;
+                    af[k][d] = __builtin_fmaf(av[k][2], u[2], __builtin_fmaf(av[k][1], u[1], av[k][0] * u[0]));
+                    if (d == 2) af[k][d] *= sgN;
+                }
+            may = light_window<false>(P, af, hw, hr, hc, nr, nc, ndir, t.we, nsubBits, lo, hi, known, tol);
+        }
+        if (!COUNT && !(live && may)) return;
+        if (SHARE_FULL) {   // rows the other waves filled
+            full |= (T)fullSh[lane];
+            if (full == FULL) live = false;
+        }
+        T valid = ~(T)0;
+        if (known < 0) {
+            const int l0 = max(lo - WIN_BASE, 0), w = max(min(hi - WIN_BASE, R - 1) + 1 - l0, 0);
+            valid = may ? interval_bits<T>((unsigned)w, (unsigned)l0) : (T)0;
+        }
+        valid &= (~full) & FULL;
+        if (!COUNT && (valid == (T)0 || culled())) return;
         // The reference negates t0, t1, L0_Q when dir < 0.  The sign is put
         // into L0 - Q and the light axes before the products (a sign flip
         // commutes with every rounding): A, B, C come out negated, identical
         // up to the sign of zero results, which no later step can observe.
-        const uint32_t sg = (ndir > 0.0f) ? 0x80000000u : 0u;   // dir < 0
+        const uint32_t sg = __float_as_uint(0.0f - ndir) & 0x80000000u;   // dir < 0 (0 - (+-0) is +0)
         auto flip = [sg](float v) { return __uint_as_float(__float_as_uint(v) ^ sg); };
         const float Lxs = flip(Lx), Lys = flip(Ly), Lzs = flip(Lz);
         Edge e[3];
@@ -1964,29 +2256,26 @@ __device__ __forceinline__ void occlude_body(const FdArgs& a, const int blkIn) {
             e[k].C = dot3(nv[k][0], nv[k][1], nv[k][2], Lxs, Lys, Lzs);
             finiteC = finiteC && __builtin_isfinite(e[k].C);
         }
+        const bool allOk = !__any(known >= 0);   // then every plane is finite and small
         // a finite C = dot(n, L0 - Q) implies a finite n (an infinite
         // component makes a product infinite or NaN)
-        if (axial && !__any(!finiteC)) {
-            const float xs = flip(xd0), ys = flip(yd1);
+        const float x0 = flip(xd0), y1 = flip(yd1);
+        if (AXIAL && (allOk || !__any(!finiteC))) {
 #pragma unroll
             for (int k = 0; k < 3; ++k) {
-                e[k].A = nv[k][0] * xs;
-                e[k].B = nv[k][1] * ys;
+                e[k].A = nv[k][0] * x0;
+                e[k].B = nv[k][1] * y1;
             }
         } else {
-            const float x0 = flip(xd0), x1 = flip(xd1), x2 = flip(xd2);
-            const float y0 = flip(yd0), y1 = flip(yd1), y2 = flip(yd2);
+            // axial lights: the other components are zeros (of any sign)
+            const float x1 = AXIAL ? 0.0f : flip(xd1), x2 = AXIAL ? 0.0f : flip(xd2);
+            const float y0 = AXIAL ? 0.0f : flip(yd0), y2 = AXIAL ? 0.0f : flip(yd2);
 #pragma unroll
             for (int k = 0; k < 3; ++k) {
                 e[k].A = dot3(nv[k][0], nv[k][1], nv[k][2], x0, x1, x2);
                 e[k].B = dot3(nv[k][0], nv[k][1], nv[k][2], y0, y1, y2);
             }
         }
-        // |A|, |B| <= 2^100 for the fast mask form (a NaN dropped by fmaxf is
-        // harmless there: it makes both f1 and f2 false, as in the reference)
-        const float mAB = fmaxf(fmaxf(fmaxf(fabsf(e[0].A), fabsf(e[1].A)), fabsf(e[2].A)),
-                                fmaxf(fmaxf(fabsf(e[0].B), fabsf(e[1].B)), fabsf(e[2].B)));
-        const bool big = !(mAB <= 1.2676506e+30f);
         if (COUNT) {
             // the rows the reference visits for this pair: its row-range mask
             // minus the rows already full (general form, before any window)
@@ -2003,61 +2292,84 @@ __device__ __forceinline__ void occlude_body(const FdArgs& a, const int blkIn) {
                 DNg[k] = (e[k].B > 0 ? -g[k].nColN : 0.0f) + e[k].C;
             }
             nRefRows += Bits<T>::popc((~full) & FULL & three_edges<T, true>(g, DNg, Rf, R));
+            if (valid == (T)0) return;
         }
-        // row by row, lowest row first (:204-222)
-        auto rows = [&](T valid, auto rowMask) {
-            while (valid) {
-                if (COUNT) ++nRows;
-                const int r = Bits<T>::ctz(valid);
-                const float fr = (float)r;
-                float D[3];
-#pragma unroll
-                for (int k = 0; k < 3; ++k) D[k] = e[k].A * fr + e[k].C;
-                const T M = rowMask(D);
-                uint32_t* w0 = lds + r * 64 + lane;
-                T cur;
-                if (Bits<T>::width == 32) {
-                    if (NW > 1) {
-                        cur = (T)(atomicOr(w0, (uint32_t)M) | (uint32_t)M);
-                    } else {
-                        cur = (T)(*w0 | (uint32_t)M);
-                        *w0 = (uint32_t)cur;
-                    }
+        // row r's mask goes to the receiver's rows; full rows are noted
+        auto add_row = [&](uint32_t* w0, int r, T M) {
+            T cur;
+            if (Bits<T>::width == 32) {
+                if (NW > 1) {
+                    cur = (T)(atomicOr(w0, (uint32_t)M) | (uint32_t)M);
                 } else {
-                    uint32_t* w1 = lds + (R + r) * 64 + lane;
-                    const uint64_t mm = (uint64_t)M;
-                    uint32_t lo32, hi32;
-                    if (NW > 1) {
-                        lo32 = atomicOr(w0, (uint32_t)mm) | (uint32_t)mm;
-                        hi32 = atomicOr(w1, (uint32_t)(mm >> 32)) | (uint32_t)(mm >> 32);
-                    } else {
-                        lo32 = *w0 | (uint32_t)mm;
-                        hi32 = *w1 | (uint32_t)(mm >> 32);
-                        *w0 = lo32;
-                        *w1 = hi32;
-                    }
-                    cur = (T)(((uint64_t)hi32 << 32) | lo32);
+                    cur = (T)(*w0 | (uint32_t)M);
+                    *w0 = (uint32_t)cur;
                 }
-                if (cur == FULL) {
-                    full |= (T)1 << r;
-                    if (SHARE_FULL) {
-                        if (Bits<T>::width == 32) atomicOr((uint32_t*)(fullSh + lane), (uint32_t)1 << r);
-                        else atomicOr((unsigned long long*)(fullSh + lane), 1ull << r);
-                    }
+            } else {
+                uint32_t* w1 = w0 + R * FD_ROW_STRIDE;
+                const uint64_t mm = (uint64_t)M;
+                uint32_t lo32, hi32;
+                if (NW > 1) {
+                    lo32 = atomicOr(w0, (uint32_t)mm) | (uint32_t)mm;
+                    hi32 = atomicOr(w1, (uint32_t)(mm >> 32)) | (uint32_t)(mm >> 32);
+                } else {
+                    lo32 = *w0 | (uint32_t)mm;
+                    hi32 = *w1 | (uint32_t)(mm >> 32);
+                    *w0 = lo32;
+                    *w1 = hi32;
                 }
-                valid &= valid - (T)1;
+                cur = (T)(((uint64_t)hi32 << 32) | lo32);
+            }
+            if (cur == FULL) {
+                full |= (T)1 << r;
+                if (SHARE_FULL) {
+                    if (Bits<T>::width == 32) atomicOr((uint32_t*)(fullSh + lane), (uint32_t)1 << r);
+                    else atomicOr((unsigned long long*)(fullSh + lane), 1ull << r);
+                }
             }
         };
-        auto wave_rows = [&](T valid) {
+        // wave row iterations = max over lanes of this triangle's rows
+        auto wave_rows = [&](int nr) {
             if (COUNT) {
-                // wave row iterations = max over lanes of this triangle's rows
-                int nr = Bits<T>::popc(valid);
                 for (int o = 32; o >= 1; o >>= 1) nr = max(nr, __shfl_xor(nr, o, 64));
                 if (lane == __ffsll((unsigned long long)__ballot(1)) - 1) nWaveRows += nr;
             }
         };
-        if (!__any(big)) {
-            // fast form: finite limits in every lane of the wave.
+        if (!COUNT && onTri && point_in_tri(t.v0, t.v1, t.v2, q.q[0], q.q[1], q.q[2])) return;
+        if (!allOk) {
+            // the exact row range and the pairwise row window for every lane,
+            // then row by row, lowest row first (:204-222)
+            auto rows = [&](T valid, auto rowMask) {
+                wave_rows(Bits<T>::popc(valid));
+                while (valid) {
+                    if (COUNT) ++nRows;
+                    const int r = Bits<T>::ctz(valid);
+                    const float fr = (float)r;
+                    float D[3];
+#pragma unroll
+                    for (int k = 0; k < 3; ++k) D[k] = e[k].A * fr + e[k].C;
+                    add_row(lds + r * FD_ROW_STRIDE + lane, r, rowMask(D));
+                    valid &= valid - (T)1;
+                }
+                if (full == FULL) live = false;
+            };
+            // |A|, |B| <= 2^100 for the fast mask form (a NaN dropped by fmaxf is
+            // harmless there: it makes both f1 and f2 false, as in the reference)
+            const float mAB = fmaxf(fmaxf(fmaxf(fabsf(e[0].A), fabsf(e[1].A)), fabsf(e[2].A)),
+                                    fmaxf(fmaxf(fabsf(e[0].B), fabsf(e[1].B)), fabsf(e[2].B)));
+            if (__any(!(mAB <= 1.2676506e+30f))) {
+                float DN[3];
+#pragma unroll
+                for (int k = 0; k < 3; ++k) {
+                    e[k].nRowN = -(e[k].A * nsub);
+                    e[k].nColN = -(e[k].B * nsub);
+                    e[k].rA = rcp_or_nan(e[k].A);
+                    e[k].rB = rcp_or_nan(e[k].B);
+                    DN[k] = (e[k].B > 0 ? -e[k].nColN : 0.0f) + e[k].C;
+                }
+                rows(valid & three_edges<T, true>(e, DN, Rf, R),
+                     [&](const float (&D)[3]) { return (T)(FULL & three_edges<T, false>(e, D, Rf, R)); });
+                return;
+            }
             // |A|, |B| <= 2^100 here, so only the lower end of the reciprocal
             // range is checked (NaN coefficients fail it as well);
             // DN = C + max(B (R-1), 0) equals (B > 0 ? B (R-1) : 0) + C up to
@@ -2071,50 +2383,148 @@ __device__ __forceinline__ void occlude_body(const FdArgs& a, const int blkIn) {
                 rA[k] = fabsf(e[k].A) >= 7.8886091e-31f ? __builtin_amdgcn_rcpf(e[k].A) : __builtin_nanf("");
                 DN[k] = e[k].C + fmaxf(bn[k], 0.0f);
             }
-            // rows that may hold occluded samples (:176-191), then the row
-            // window; a wave none of whose lanes keeps a row skips the
-            // triangle at either step (the cheaper test first)
-            T valid = (~full) & FULL & three_edges_fast<T>(DN, nR, rA, dA, Rs, R);
-            if (!__any(valid != (T)0)) return;
+            valid &= three_edges_fast<T>(DN, nR, rA, dA, Rs, R);
             valid &= row_window<T>(e, Rf, mAB);
             if (!__any(valid != (T)0)) return;   // no lane can gain a bit from this triangle
-            if (!COUNT && onTri && valid != (T)0 && point_in_tri(t.v0, t.v1, t.v2, q.q[0], q.q[1], q.q[2])) return;
             float nC[3], rB[3], dB[3];
 #pragma unroll
             for (int k = 0; k < 3; ++k) {
                 dB[k] = e[k].B;
                 nC[k] = -bn[k];
                 rB[k] = fabsf(e[k].B) >= 7.8886091e-31f ? __builtin_amdgcn_rcpf(e[k].B) : __builtin_nanf("");
-                asm("" : "+v"(rB[k]));   // keep the select out of the row loop
             }
-            wave_rows(valid);
             rows(valid, [&](const float (&D)[3]) { return three_edges_fast<T>(D, nC, rB, dB, Rs, R); });
-        } else {
-            if (!COUNT && onTri && point_in_tri(t.v0, t.v1, t.v2, q.q[0], q.q[1], q.q[2])) return;
-            float DN[3];
+            return;
+        }
+        // Row by row from the first to the last row of the window that is not
+        // full.  G = the least of the edges' largest values along the row,
+        // D + max(B (R-1), 0).  G < -tol: the mask is empty.  G > tol: the
+        // row is in the reference's row-range mask (its roundings
+        // and G's stay below 8u (|A| R + |B| R + |C|)) and every edge passes at its far end, so the
+        // edge's mask is the half line c >= -D/B (B > 0) or c < -D/B (B < 0)
+        // clipped to the grid; x = R - 1/2 + D rcp(B) rounds to
+        // R - ceil(-D/B) unless x is within 2^-15 of a tie (rcp, the fma and
+        // the reference's quotient are off by at most 2^-17 + 2^-19 + 2^-19
+        // while 0 <= -D/B <= R <= 64).  Edges
+        // of the other sign stand in with x = 0 (upper limits) and x = R
+        // (lower limits), the grid's own ends; planes through one vertex
+        // fan cannot all have one sign of B but by rounding, which goes the
+        // exact way, as do ties and |G| <= tol.  A zero B gives an infinite
+        // reciprocal: no limit, as every column then has the sign of G.
+        float rh[3], rl[3], Kh[3], Kl[3], bp[3];
+        const int Rm = __float_as_int(Rf - 0.5f), RmR = Rm ^ __float_as_int(Rf);
+        int sAnd = -1, sOr = 0;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            int sB = __float_as_int(e[k].B) >> 31;
+            asm("" : "+v"(sB));   // as a mask: selects run at half the rate
+            const int rB = __float_as_int(__builtin_amdgcn_rcpf(e[k].B)), bn = __float_as_int(e[k].B * nsub);
+            rh[k] = __int_as_float(rB & sB);
+            rl[k] = __int_as_float(rB ^ (rB & sB));
+            Kh[k] = __int_as_float(Rm & sB);
+            Kl[k] = __int_as_float(Rm ^ (RmR & sB));
+            bp[k] = __int_as_float(bn ^ (bn & sB));
+            sAnd &= sB;
+            sOr |= sB;
+        }
+        // tol = q / 16 >= 3u (|A| R + |B| R + |C|)
+        const int tolBits = (__float_as_int(tol) - (4 << 23)) | ((sAnd | ~sOr) & 0x7f800000);
+        const int r0 = Bits<T>::ctz(valid);
+        const int r1 = Bits<T>::last(valid);
+        wave_rows(r1 - r0 + 1);
+        float fr = (float)r0;
+        const float frEnd = (float)r1;
+        uint32_t* w0 = lds + r0 * FD_ROW_STRIDE + lane;
+        T redo = (T)0;
+        do {
+            if (COUNT) ++nRows;
+            float D[3], xh[3], xl[3], g[3];
 #pragma unroll
             for (int k = 0; k < 3; ++k) {
-                e[k].nRowN = -(e[k].A * nsub);
-                e[k].nColN = -(e[k].B * nsub);
-                e[k].rA = rcp_or_nan(e[k].A);
-                e[k].rB = rcp_or_nan(e[k].B);
-                DN[k] = (e[k].B > 0 ? -e[k].nColN : 0.0f) + e[k].C;
+                D[k] = e[k].A * fr + e[k].C;
+                xh[k] = __builtin_fmaf(D[k], rh[k], Kh[k]);
+                xl[k] = __builtin_fmaf(D[k], rl[k], Kl[k]);
+                g[k] = D[k] + bp[k];
             }
-            const T valid = (~full) & FULL & three_edges<T, true>(e, DN, Rf, R);
-            wave_rows(valid);
-            rows(valid, [&](const float (&D)[3]) { return (T)(FULL & three_edges<T, false>(e, D, Rf, R)); });
+            const float xH = fmaxf(fmaxf(xh[0], xh[1]), xh[2]), xL = fminf(fminf(xl[0], xl[1]), xl[2]);
+            const int G = __float_as_int(fminf(fminf(g[0], g[1]), g[2]));
+            const float yH = xH + WIN_MAGIC, yL = xL + WIN_MAGIC;
+            const float zH = xH - (yH - WIN_MAGIC), zL = xL - (yL - WIN_MAGIC);
+            // negative: decided (0x3efffc00 = 1/2 - 2^-15)
+            const int sure = ((__float_as_int(zH) & 0x7fffffff) - 0x3efffc00) &
+                             ((__float_as_int(zL) & 0x7fffffff) - 0x3efffc00) & (tolBits - (G & 0x7fffffff));
+            const unsigned iL = (unsigned)__float_as_int(yL);
+            const unsigned iH = (unsigned)__float_as_int(yH) | ((unsigned)G & 0x80000000u);   // G < 0: empty
+            T M = interval_bits<T>(__builtin_elementwise_sub_sat(iL, iH), (unsigned)(WIN_BASE + R) - iL);
+            if (sure >= 0) {
+                M = (T)0;
+                redo |= (T)1 << (int)fr;
+            }
+            add_row(w0, (int)fr, M);
+            fr += 1.0f;
+            w0 += FD_ROW_STRIDE;
+        } while (fr <= frEnd);
+        // the rows left open (about one in a hundred row iterations of a
+        // wave), out of the loop so that their divisions cost it no registers
+        while (redo) {
+            const int r = Bits<T>::ctz(redo);
+            add_row(lds + r * FD_ROW_STRIDE + lane, r, row_exact<T>(e, (float)r, nsub, R));
+            redo &= redo - (T)1;
         }
         if (full == FULL) live = false;
     };
-    if (COUNT) {
-        for (int ti = ts + wv; ti < te; ti += NW) {
-            const uint64_t liveMask = __ballot(live);
-            if (liveMask == 0) break;
-            nCand += __popcll(liveMask);
-            ++nWaveIt;
-            step(triList[ti]);
+    // Of a block's triangles (lane l holds the id of triangle l, cmask the ones
+    // still to do), those that can set a sample some receiver lacks.  A
+    // receiver's rows fill early: on the 1080p soup 70-80% of the pairs that
+    // pass the cull, on the sphere meshes a third, only meet full rows.  It
+    // costs about a pair and a half (all triangles at once), so it runs after
+    // FD_PRUNE_STEPS pairs and for FD_PRUNE_LEFT triangles or more.
+    auto prune = [&](uint64_t cmask, const int tidv, auto axialT) -> uint64_t {
+        uint64_t U[FD_OCC_STRIPS];
+        row_occupancy<T>(lds, R, lsw, FULL, U);
+        bool keep = (cmask >> lane) & 1;
+        if (keep) {
+            const FdTri& tr = a.tri[tidv];
+            float vf[3][3], S0 = 0.0f;
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                const float* v = k == 0 ? tr.v0 : k == 1 ? tr.v1 : tr.v2;
+                const float x = v[0] - a.L.ur[0], y = v[1] - a.L.ur[1], z = v[2] - a.L.ur[2];
+                S0 = fmaxf(S0, fabsf(x) + fabsf(y) + fabsf(z));
+                if constexpr (decltype(axialT)::value) {
+                    vf[k][0] = x * a.L.X[0];
+                    vf[k][1] = y * a.L.Y[1];
+                    vf[k][2] = z;
+                } else {
+                    vf[k][0] = dot3(x, y, z, a.L.X[0], a.L.X[1], a.L.X[2]);
+                    vf[k][1] = dot3(x, y, z, a.L.Y[0], a.L.Y[1], a.L.Y[2]);
+                    vf[k][2] = dot3(x, y, z, a.L.N[0], a.L.N[1], a.L.N[2]) * sgN;
+                }
+            }
+            int rlo, rhi, clo, chi;
+            if (tile_window(tb, vf, S0, tr.we, R - 1, rlo, rhi, clo, chi)) {
+                const int s0 = clo >> lsw, s1 = chi >> lsw;
+                T open = (T)0;
+#pragma unroll
+                for (int k = 0; k < FD_OCC_STRIPS; ++k) open |= (k >= s0 && k <= s1) ? (T)U[k] : (T)0;
+                const T rows = interval_bits<T>((unsigned)max(rhi + 1 - rlo, 0), (unsigned)rlo);
+                keep = chi >= clo && (open & rows) != (T)0;
+            }
         }
-    } else {
+        return __ballot(keep);
+    };
+    // the list, once per light class: the axial one needs fewer registers
+    auto walk = [&](auto axialT) {
+        if (COUNT) {
+            for (int ti = ts + wv; ti < te; ti += NW) {
+                const uint64_t liveMask = __ballot(live);
+                if (liveMask == 0) break;
+                nCand += __popcll(liveMask);
+                ++nWaveIt;
+                step(triList[ti], axialT);
+            }
+            return;
+        }
         // blocks of 64 of this wave's entries; the candidate loop reads the
         // block's ids from the lanes that loaded them (written once per
         // block, so any subset of lanes that runs an iteration reads the
@@ -2122,6 +2532,7 @@ __device__ __forceinline__ void occlude_body(const FdArgs& a, const int blkIn) {
         // tested and its pairs run; the box fields load unconditionally, in
         // one round trip.
         int tidNext = (ts + wv + lane * NW < te) ? listV[ts + wv + lane * NW] : -1;
+        bool stepped = false;   // some pair has run: rows may be full
         for (int blk0 = ts + wv; blk0 < te; blk0 += 64 * NW) {
             if (__ballot(live) == 0) break;
             const int tj = blk0 + lane * NW;
@@ -2136,12 +2547,19 @@ __device__ __forceinline__ void occlude_body(const FdArgs& a, const int blkIn) {
             const int tn = tj + 64 * NW;
             tidNext = tn < te ? listV[tn] : -1;
             if (okv) keep = bmn.x <= gx0 && bmn.y <= gy0 && gx1 <= bmx.x && gy1 <= bmx.y && bmn.z <= gz;
-            for (uint64_t cmask = __ballot(keep); cmask; cmask &= cmask - 1) {
-                if (__ballot(live) == 0) break;
-                step(__builtin_amdgcn_readlane(tidv, uniform(__ffsll((unsigned long long)cmask) - 1)));
+            uint64_t cmask = __ballot(keep);
+            while (cmask) {
+                if (stepped && longList && __popcll(cmask) >= FD_PRUNE_LEFT) cmask = prune(cmask, tidv, axialT);
+                for (int k = 0; k < FD_PRUNE_STEPS && cmask; ++k, cmask &= cmask - 1) {
+                    if (__ballot(live) == 0) return;
+                    step(__builtin_amdgcn_readlane(tidv, uniform(__ffsll((unsigned long long)cmask) - 1)), axialT);
+                    stepped = true;
+                }
             }
         }
-    }
+    };
+    if (axialW) walk(std::true_type{});
+    else walk(std::false_type{});
     if (COUNT) {
         // per-lane counts: nCand is wave-wide already
         unsigned long long p = nPass, r = nRows, rr = nRefRows, pl = nPlanes;
@@ -2170,8 +2588,8 @@ __device__ __forceinline__ void occlude_body(const FdArgs& a, const int blkIn) {
     if (wv == 0 && S == 1) {
         int cnt = 0;
         for (int r = 0; r < R; ++r) {
-            cnt += __popc(lds[r * 64 + lane]);
-            if (wpr == 2) cnt += __popc(lds[(R + r) * 64 + lane]);
+            cnt += __popc(lds[r * FD_ROW_STRIDE + lane]);
+            if (wpr == 2) cnt += __popc(lds[(R + r) * FD_ROW_STRIDE + lane]);
         }
         if (act) a.shadow[id] = (float)cnt / (float)a.L.resNum;
     }
@@ -2196,11 +2614,9 @@ __device__ __forceinline__ void occlude_finish_body(const FdArgs& a, const int c
     const FdState* s = a.st;
     if (s->status != FD_EXIT_OK || c >= s->totalChunks) return;
     const int nb = s->nb;
-    const int rank = chunk_rank(a, c, nb);
-    const int bin = a.binAtRank[rank];
-    if (bin == nb) return;
-    const int s0 = a.rxStart[bin] + (c - a.chunkStart[rank]) * 64;
-    const int n = min(64, a.rxEnd[bin] - s0);
+    const FdChunk ck = a.chunks[c];
+    if (ck.nbin >> 8 == nb) return;
+    const int s0 = ck.s0, n = ck.nbin & 255;
     const int lane = lane_id();
     int id = lane < n ? a.sortedId[s0 + lane] : 0;
     if ((unsigned)id >= (unsigned)a.WH) id = 0;   // defensive: ids form a permutation
@@ -2212,7 +2628,7 @@ __device__ __forceinline__ void occlude_finish_body(const FdArgs& a, const int c
     const int total = n * per;
     for (int j0 = 0; j0 < total; j0 += 64) {
         const int j = j0 + lane;
-        const int l = min(j, total - 1) / per, w = j - l * per;
+        const int l = word_receiver(min(j, total - 1), 1.0f / (float)per), w = j - l * per;
         const int idl = __shfl(id, l, 64);
         if (j < total) {
             const int b = __popc(a.masks[(size_t)idl * per + w]);
@@ -2263,10 +2679,12 @@ __global__ __launch_bounds__(64) void k_occlude_finish(FdArgs a) { occlude_finis
 // runs one wave per work item: each receiver then meets its triangles in
 // list order with the full-row state of all earlier ones, as in the
 // reference, so its work counters do not depend on the schedule.
-// 8 waves per SIMD (the most a SIMD holds): the target makes the compiler
-// keep the scalar registers within 8 waves' share (else 99-103 SGPRs, 7-8).
+// 6 waves per SIMD, 80 vector registers: at 8 (64) and 7 (72) the pair's
+// set-up spills (heightfield-1k 2944 / 2754 / 2739 us at 8 / 7 / 6 waves,
+// 1080p soup with 32 x 32 samples 2510 / 2201 / 2100 us), at 5 too few waves
+// hide the record loads.
 template <typename T, bool COUNT, int NW>
-__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(8))) void k_occlude(FdArgs a) {
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(6))) void k_occlude(FdArgs a) {
     occlude_body<T, COUNT, false, NW>(a, xcd_block(blockIdx.x, gridDim.x));
 }
 template <typename T>
@@ -2316,7 +2734,7 @@ FD_BATCHED(kb_tri_order, FD_ORDER_THREADS, tri_order_body)
 #undef FD_BATCHED
 
 template <typename T, int NW>
-__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(8))) void kb_occlude(const FdArgs* __restrict__ inst, const int* __restrict__ map, int n) {
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(6))) void kb_occlude(const FdArgs* __restrict__ inst, const int* __restrict__ map, int n) {
     const int b = xcd_block(blockIdx.x, gridDim.x);
     const int i = inst_of(map, n, b);
     const FdArgs a = inst[i];
@@ -2513,7 +2931,7 @@ hipError_t enqueue_batch(const FdBatchPlan& p, hipStream_t st) {
     for (int c = 0; c < FD_OCC_CLASSES; ++c) {   // fd_occ_class: 32 / 64-bit rows x 2 / 4 / 8 waves
         if (p.nocc[c] == 0) continue;
         const int wpr = c / 3 + 1, nw = 2 << (c % 3);
-        const size_t shm = (size_t)wpr * p.maxRes[c] * 64 * sizeof(uint32_t) + 64 * wpr * sizeof(uint32_t);
+        const size_t shm = fd_occ_lds(wpr, p.maxRes[c]);
         const dim3 g = L(FD_MAP_OCC0 + c);
         const int* mp = p.map[FD_MAP_OCC0 + c];
         const FdArgs* in = p.occ[c];
@@ -2602,7 +3020,7 @@ hipError_t enqueue_frame(const FdArgs& a, hipStream_t st, hipEvent_t* ev) {
     }
     mark(3);
     k_tables<<<1, 1024, 0, st>>>(a);
-    if (a.ntris > 0) k_tri_order<<<nb, FD_ORDER_THREADS, 0, st>>>(a);
+    if (a.ntris > 0) k_tri_order<<<nb + 1, FD_ORDER_THREADS, 0, st>>>(a);
     mark(4);
     // occlusion (or the early-exit fill); split lists zero the masks first
     // and count them after the merge
@@ -2610,13 +3028,13 @@ hipError_t enqueue_frame(const FdArgs& a, hipStream_t st, hipEvent_t* ev) {
     if (a.segs > 1) k_zero_masks<<<zero_blocks(a), 256, 0, st>>>(a);
     if (a.occVariant == FD_OCC_BIN_QUEUE) {
         const int chunks = a.chunkSlots * a.segs;
-        const size_t shmCta = (size_t)wpr * a.L.res * 64 * sizeof(uint32_t) + 64 * sizeof(uint64_t);   // + full-row flags
+        const size_t shmCta = (size_t)wpr * a.L.res * FD_ROW_STRIDE * sizeof(uint32_t) + 64 * sizeof(uint64_t);   // + full-row flags
         if (wpr == 1) k_occlude_cta<uint32_t><<<chunks, 64, shmCta, st>>>(a);
         else k_occlude_cta<uint64_t><<<chunks, 64, shmCta, st>>>(a);
     } else {
         const FdArgs& ao = a;
         const int chunks = a.chunkSlots * a.segs;
-        const size_t shm = (size_t)wpr * a.L.res * 64 * sizeof(uint32_t) + 64 * wpr * sizeof(uint32_t);
+        const size_t shm = fd_occ_lds(wpr, a.L.res);
         if (a.opCount) {
             if (wpr == 1) k_occlude<uint32_t, true, 1><<<chunks, 64, shm, st>>>(ao);
             else k_occlude<uint64_t, true, 1><<<chunks, 64, shm, st>>>(ao);

@@ -16,6 +16,9 @@ struct FdLight {
     int resNum;           // res * res
     int wpr;              // 32-bit words per mask row: 1 (res <= 32) or 2
     int pad;
+    // light-plane normal and the vectors dual to the sample steps: xd.X = yd.Y = 1,
+    // xd.Y = yd.X = X.N = Y.N = 0 (double arithmetic, rounded once)
+    float X[3], Y[3], N[3];
 };
 
 // Frame exit codes: FD_EXIT_* of the public header (the order of the early
@@ -63,7 +66,7 @@ struct FdTri {
     float v0[3], v1[3], v2[3];
     float bminx, bminy, bmaxx, bmaxy;   // projected AABB (aabb2Dmin/max)
     float minz, maxz;
-    float pad0;
+    float we;        // light_window's edge term (infinite for huge triangles)
     float n[3];      // cross(v1 - v0, v2 - v1)
     float e01[3];    // v0 - v1
     float e12[3];    // v1 - v2
