@@ -24,6 +24,7 @@ struct GbArgs {
     double eye[3], f[3], s[3], u[3];
     double tanh_, aspect, ground_half;
     int w, h, nbox, hasMat;
+    int tilesX;            // 16 x 16 pixel tiles per row; 0: one pixel after the other
     const double* boxes;   // nbox x 6
     const float* mat;      // (nbox + 1) x 10: ka, kd, ks, shininess
     float4 *g0, *g1, *g2, *g3;
@@ -37,14 +38,62 @@ __device__ __forceinline__ DV dnormalize(DV a) {
     return dmul(a, 1.0 / l);
 }
 
+// The slab test in single precision finds the boxes a ray may hit first.
+// With c = corner - eye rounded once and rcp within an ulp, a float slab
+// distance is off by less than 2^-21 of itself; GB_EPS = 2^-18 leaves room
+// for the comparisons.  Only near / far distances that stay apart by that much
+// are ordered by it: then the exact test has the same near axis, t0 <= t1, and
+// t0 is that axis's one quotient in double precision.  Everything else (close
+// distances, rays along an axis) runs the exact test of all six quotients.
+//
+// Bound: the double-precision divisions (about 100 cycles each per wave), six
+// per box and ray in the plain loop: 197 us at 1920 x 1080 with 20 boxes
+// (0.7 TB/s of the 133 MB written); with the float test 4 to 6 per ray and
+// 40 us (3.3 TB/s).
+constexpr float GB_EPS = 3.814697265625e-06f;
+constexpr int GB_TILE = 16;        // tiles of 16 x 16 pixels: a wave holds 16 x 4
+constexpr int GB_MAX_BOXES = 256;  // fd_gbuffer_boxes' limit
+
 __global__ __launch_bounds__(256) void k_gbuffer_boxes(GbArgs a) {
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (long)a.w * a.h) return;
-    const int y = (int)(i / a.w), x = (int)(i - (long)y * a.w);
+    __shared__ __align__(16) float cb[GB_MAX_BOXES * 8];   // per box: min - eye, 1 if not finite or huge, max - eye, -
+    __shared__ float mat[(GB_MAX_BOXES + 1) * 10];
+    __shared__ double nx[GB_TILE], ny[GB_TILE];
+    const int tid = threadIdx.x;
+    for (int b = tid; b < a.nbox; b += 256) {
+        float far = 0.0f;
+        for (int k = 0; k < 3; ++k) {
+            const float lo = (float)(a.boxes[6 * b + k] - a.eye[k]), hi = (float)(a.boxes[6 * b + 3 + k] - a.eye[k]);
+            cb[8 * b + k] = lo;
+            cb[8 * b + 4 + k] = hi;
+            if (!(fabsf(lo) <= 1e30f && fabsf(hi) <= 1e30f)) far = 1.0f;
+        }
+        cb[8 * b + 3] = far;
+    }
+    if (a.hasMat)
+        for (int k = tid; k < 10 * (a.nbox + 1); k += 256) mat[k] = a.mat[k];
+    int x, y;
+    double ndcx, ndcy;
+    if (a.tilesX > 0) {
+        const int ty = (int)(blockIdx.x / (unsigned)a.tilesX), tx = (int)blockIdx.x - ty * a.tilesX;
+        x = tx * GB_TILE + (tid & 15);
+        y = ty * GB_TILE + (tid >> 4);
+        if (tid < 16) nx[tid] = (2.0 * (x + 0.5) / a.w - 1.0) * a.tanh_ * a.aspect;   // row 0 of the tile: x = its column
+        else if (tid < 32) ny[tid - 16] = (1.0 - 2.0 * (ty * GB_TILE + (tid - 16) + 0.5) / a.h) * a.tanh_;
+        __syncthreads();
+        ndcx = nx[tid & 15];
+        ndcy = ny[tid >> 4];
+    } else {   // views narrower or lower than a tile
+        __syncthreads();
+        const unsigned i = blockIdx.x * 256u + tid;
+        y = (int)(i / (unsigned)a.w);
+        x = (int)(i - (unsigned)y * (unsigned)a.w);
+        ndcx = (2.0 * (x + 0.5) / a.w - 1.0) * a.tanh_ * a.aspect;
+        ndcy = (1.0 - 2.0 * (y + 0.5) / a.h) * a.tanh_;
+    }
+    if (x >= a.w || y >= a.h) return;
+    const size_t i = (size_t)y * a.w + x;
     const DV eye{a.eye[0], a.eye[1], a.eye[2]};
     const DV f{a.f[0], a.f[1], a.f[2]}, s{a.s[0], a.s[1], a.s[2]}, u{a.u[0], a.u[1], a.u[2]};
-    const double ndcx = (2.0 * (x + 0.5) / a.w - 1.0) * a.tanh_ * a.aspect;
-    const double ndcy = (1.0 - 2.0 * (y + 0.5) / a.h) * a.tanh_;
     const DV d = dnormalize(dadd(dadd(f, dmul(s, ndcx)), dmul(u, ndcy)));
     double tbest = 1e300;
     DV nbest{0, 0, 0};
@@ -55,6 +104,10 @@ __global__ __launch_bounds__(256) void k_gbuffer_boxes(GbArgs a) {
         if (fabs(p.x) <= a.ground_half && fabs(p.y) <= a.ground_half) { tbest = t; nbest = {0, 0, 1}; obj = 0; }
     }
     const double e[3] = {eye.x, eye.y, eye.z}, dd[3] = {d.x, d.y, d.z};
+    const float df[3] = {(float)d.x, (float)d.y, (float)d.z};
+    const float iv[3] = {__builtin_amdgcn_rcpf(df[0]), __builtin_amdgcn_rcpf(df[1]), __builtin_amdgcn_rcpf(df[2])};
+    const bool along = fminf(fminf(fabsf(df[0]), fabsf(df[1])), fabsf(df[2])) < 1e-30f;
+    float tbf = tbest < 1e30 ? (float)tbest * (1.0f + GB_EPS) : INFINITY;
 #if defined(__HIP_DEVICE_COMPILE__)
     typedef const __attribute__((address_space(4))) double* cdbl_p;   // uniform box records: scalar loads
 #else
@@ -62,26 +115,52 @@ __global__ __launch_bounds__(256) void k_gbuffer_boxes(GbArgs a) {
 #endif
     const cdbl_p boxes = (cdbl_p)a.boxes;
     for (int b = 0; b < a.nbox; ++b) {
+        const float4 c0 = *(const float4*)(cb + 8 * b), c1 = *(const float4*)(cb + 8 * b + 4);
+        const float ax = c0.x * iv[0], ay = c0.y * iv[1], az = c0.z * iv[2];
+        const float bx = c1.x * iv[0], by = c1.y * iv[1], bz = c1.z * iv[2];
+        const float lx = fminf(ax, bx), ly = fminf(ay, by), lz = fminf(az, bz);
+        const float t0f = fmaxf(fmaxf(lx, ly), lz);
+        const float t1f = fminf(fminf(fmaxf(ax, bx), fmaxf(ay, by)), fmaxf(az, bz));
+        // no hit: behind the eye, past the nearest hit, or out of a slab before into another
+        const bool exact = along || c0.w != 0.0f;
+        if (!exact && (t0f < 0.0f || t0f > tbf || t1f < t0f * (1.0f - GB_EPS))) continue;
         const cdbl_p bmin = boxes + 6 * b;
         const cdbl_p bmax = bmin + 3;
         double t0 = -1e300, t1 = 1e300;
         int axis = -1;
         double sgn = 0;
-        bool miss = false;
-        for (int k = 0; k < 3; ++k) {
-            if (fabs(dd[k]) < 1e-300) {
-                if (e[k] < bmin[k] || e[k] > bmax[k]) { miss = true; break; }
-                continue;
+        // one near distance clearly the last, clearly before the first far one
+        const float m = t0f * (1.0f - GB_EPS);
+        const int last = (lx > m ? 1 : 0) + (ly > m ? 2 : 0) + (lz > m ? 4 : 0);
+        if (!exact && t0f > 1e-30f && t0f < 1e30f && t1f > t0f * (1.0f + GB_EPS) &&
+            (last == 1 || last == 2 || last == 4)) {
+            axis = last >> 1;
+            // the nearer face of the slab (they are apart: the far one is not before t1f)
+            const bool first = axis == 0 ? ax < bx : axis == 1 ? ay < by : az < bz;
+            const double dk = axis == 0 ? d.x : axis == 1 ? d.y : d.z;
+            const double ek = axis == 0 ? eye.x : axis == 1 ? eye.y : eye.z;
+            const double lo = axis == 0 ? bmin[0] : axis == 1 ? bmin[1] : bmin[2];
+            const double hi = axis == 0 ? bmax[0] : axis == 1 ? bmax[1] : bmax[2];
+            t0 = ((first ? lo : hi) - ek) / dk;
+            sgn = first ? -1.0 : 1.0;
+        } else {
+            bool miss = false;
+            for (int k = 0; k < 3; ++k) {
+                if (fabs(dd[k]) < 1e-300) {
+                    if (e[k] < bmin[k] || e[k] > bmax[k]) { miss = true; break; }
+                    continue;
+                }
+                double ta = (bmin[k] - e[k]) / dd[k], tb = (bmax[k] - e[k]) / dd[k];
+                double sa = -1.0;
+                if (ta > tb) { const double tmp = ta; ta = tb; tb = tmp; sa = 1.0; }
+                if (ta > t0) { t0 = ta; axis = k; sgn = sa; }
+                if (tb < t1) t1 = tb;
             }
-            double ta = (bmin[k] - e[k]) / dd[k], tb = (bmax[k] - e[k]) / dd[k];
-            double sa = -1.0;
-            if (ta > tb) { const double tmp = ta; ta = tb; tb = tmp; sa = 1.0; }
-            if (ta > t0) { t0 = ta; axis = k; sgn = sa; }
-            if (tb < t1) t1 = tb;
+            if (miss || t0 > t1 || t0 <= 0.0 || axis < 0) continue;
         }
-        if (miss || t0 > t1 || t0 <= 0.0 || axis < 0) continue;
         if (t0 < tbest) {
             tbest = t0;
+            tbf = tbest < 1e30 ? (float)tbest * (1.0f + GB_EPS) : INFINITY;
             nbest = {0, 0, 0};
             if (axis == 0) nbest.x = sgn; else if (axis == 1) nbest.y = sgn; else nbest.z = sgn;
             obj = 1 + b;
@@ -89,10 +168,10 @@ __global__ __launch_bounds__(256) void k_gbuffer_boxes(GbArgs a) {
     }
     if (tbest < 1e299) {
         const DV p = dadd(eye, dmul(d, tbest));
-        const float* m = a.hasMat ? a.mat + 10 * obj : nullptr;
-        a.g0[i] = make_float4((float)p.x, (float)p.y, (float)p.z, m ? m[6] : 1.0f);
-        a.g1[i] = make_float4((float)nbest.x, (float)nbest.y, (float)nbest.z, m ? m[7] : 1.0f);
-        if (m) {
+        const float* m = mat + 10 * obj;
+        a.g0[i] = make_float4((float)p.x, (float)p.y, (float)p.z, a.hasMat ? m[6] : 1.0f);
+        a.g1[i] = make_float4((float)nbest.x, (float)nbest.y, (float)nbest.z, a.hasMat ? m[7] : 1.0f);
+        if (a.hasMat) {
             if (a.g2) a.g2[i] = make_float4(m[0], m[1], m[2], m[8]);
             if (a.g3) a.g3[i] = make_float4(m[3], m[4], m[5], m[9]);
         }
@@ -188,7 +267,7 @@ struct Upload {
 extern "C" {
 
 int fd_gbuffer_boxes(const fd_gbuffer_scene* sc, float* d_g0, float* d_g1, float* d_g2, float* d_g3, void* stream) {
-    if (!sc || !d_g0 || !d_g1 || sc->width <= 0 || sc->height <= 0 || sc->nbox < 0 || sc->nbox > 256 ||
+    if (!sc || !d_g0 || !d_g1 || sc->width <= 0 || sc->height <= 0 || sc->nbox < 0 || sc->nbox > GB_MAX_BOXES ||
         (sc->nbox > 0 && !sc->boxes) || (long)sc->width * sc->height > (1L << 30))
         return FD_ERR_ARG;
     if ((d_g2 || d_g3) && !sc->materials) return FD_ERR_ARG;
@@ -223,7 +302,12 @@ int fd_gbuffer_boxes(const fd_gbuffer_scene* sc, float* d_g0, float* d_g1, float
         a.boxes = (const double*)ub.p;
         a.mat = (const float*)um.p;
         const long n = (long)sc->width * sc->height;
-        hipLaunchKernelGGL(k_gbuffer_boxes, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, a);
+        long blocks = (n + 255) / 256;
+        if (sc->width >= GB_TILE && sc->height >= GB_TILE) {   // else most of a tile would be outside the view
+            a.tilesX = (sc->width + GB_TILE - 1) / GB_TILE;
+            blocks = (long)a.tilesX * ((sc->height + GB_TILE - 1) / GB_TILE);
+        }
+        hipLaunchKernelGGL(k_gbuffer_boxes, dim3((unsigned)blocks), dim3(256), 0, st, a);
         e = hipGetLastError();
     }
     ub.free(st);
