@@ -70,6 +70,16 @@ template <int CTRL, int ROWS>
 __device__ __forceinline__ int dpp_or(int old, int v) {   // old where the source lane does not exist
     return __builtin_amdgcn_update_dpp(old, v, CTRL, ROWS, 0xf, false);
 }
+// Inclusive prefix sum over the wave, every lane active.
+__device__ __forceinline__ uint32_t wave_incl_scan(uint32_t x) {
+    x += (uint32_t)dpp_or<0x111, 0xf>(0, (int)x);
+    x += (uint32_t)dpp_or<0x112, 0xf>(0, (int)x);
+    x += (uint32_t)dpp_or<0x114, 0xf>(0, (int)x);
+    x += (uint32_t)dpp_or<0x118, 0xf>(0, (int)x);
+    x += (uint32_t)dpp_or<0x142, 0xa>(0, (int)x);
+    x += (uint32_t)dpp_or<0x143, 0xc>(0, (int)x);
+    return x;
+}
 template <typename F>
 __device__ __forceinline__ int wave_reduce(int v, F&& f, bool sum) {
     v = f(v, dpp_or<0x111, 0xf>(sum ? 0 : v, v));   // row_shr:1, 2, 4, 8

@@ -205,12 +205,15 @@ size_t layout(FdArgs& a, char* base, bool countOps) {
     a.st = (FdState*)take(sizeof(FdState));
     a.rec = (float4*)take(WH * sizeof(float4));
     a.rxKey = (uint16_t*)take(WH * sizeof(uint16_t));
-    // the histograms are done with once the tables exist: the work-item records
-    // take their place (and more only where both are a few KB)
+    // the histograms and totals are done with once both scatters are: the
+    // work-item records take their place (each holds a receiver: WH at most)
     const size_t hr = ((size_t)a.nR * sizeof(uint32_t) + 255) & ~(size_t)255;
-    char* hist = (char*)take(std::max(hr + (size_t)a.nT * sizeof(uint32_t), (size_t)a.chunkSlots * sizeof(FdChunk)));
+    const size_t ht = hr + (size_t)a.nT * sizeof(uint32_t), tot = (size_t)(2 * nb + 1) * sizeof(uint32_t);
+    char* hist = (char*)take(std::max(ht + tot, std::min((size_t)a.chunkSlots, WH) * sizeof(FdChunk)));
     a.histR = (uint32_t*)hist;
     a.histT = hist ? (uint32_t*)(hist + hr) : nullptr;
+    a.rxTot = hist ? (uint32_t*)(hist + ht) : nullptr;
+    a.triTot = a.rxTot ? a.rxTot + nb + 1 : nullptr;
     a.chunks = (FdChunk*)hist;
     a.sortedId = (int*)take(WH * sizeof(int));
     a.sortedRec = (FdRxRec*)take(WH * sizeof(FdRxRec));
@@ -223,17 +226,14 @@ size_t layout(FdArgs& a, char* base, bool countOps) {
     a.triClass = (uint8_t*)take(T);
     a.pairKT = (uint32_t*)take((size_t)a.pairCap * sizeof(uint32_t));
     a.sortedTri = (int*)take((size_t)a.pairCap * sizeof(int));
-    int* tb = (int*)take((size_t)(6 * (nb + 2)) * sizeof(int));
+    // a bin's list ends where the next one starts
+    int* tb = (int*)take((size_t)(3 * (nb + 2)) * sizeof(int));
     a.rxStart = tb;
-    a.rxEnd = tb ? tb + (nb + 2) : nullptr;
-    a.triStart = tb ? tb + 2 * (nb + 2) : nullptr;
-    a.triEnd = tb ? tb + 3 * (nb + 2) : nullptr;
-    a.chunkStart = tb ? tb + 4 * (nb + 2) : nullptr;
-    a.binAtRank = tb ? tb + 5 * (nb + 2) : nullptr;
-    const long np = std::max(std::max(fdk::scan_partials_needed(a.nR), fdk::scan_partials_needed(a.nT)),
-                             fdk::scan_partials_needed(T)) + 1;
-    a.scanPart = (uint64_t*)take(np * sizeof(uint64_t));
-    a.part = (uint32_t*)take((size_t)std::max(8 * (a.nbR + a.nbV), 3 * a.nblkT) * sizeof(uint32_t));
+    a.rxEnd = tb ? tb + 1 : nullptr;
+    a.triStart = tb ? tb + (nb + 2) : nullptr;
+    a.triEnd = tb ? tb + (nb + 2) + 1 : nullptr;
+    a.chunkStart = tb ? tb + 2 * (nb + 2) : nullptr;
+    a.part = (uint32_t*)take((size_t)std::max(8 * (a.nbR + a.nbV), 2 * a.nblkT) * sizeof(uint32_t));
     a.opCount = countOps ? (unsigned long long*)take(FD_NOPS * sizeof(unsigned long long)) : nullptr;
     if (!a.masks) a.masks = (uint32_t*)take(WH * a.L.res * a.L.wpr * sizeof(uint32_t));
     return off;
@@ -770,13 +770,10 @@ size_t build_plan(const std::vector<FdArgs>& args, bool anyTris, char* devBase, 
             int blocks = 1;
             switch (m) {
                 case FD_MAP_ONE: blocks = 1; break;
-                case FD_MAP_BINS: blocks = cdiv(nb, 256); break;
                 case FD_MAP_RED: blocks = a.nbR + a.nbV; break;
                 case FD_MAP_RX: blocks = a.nblkR; break;
-                case FD_MAP_SCANR: blocks = fdk::scan_chunks(a.nR); break;
                 case FD_MAP_TRI: blocks = a.nblkT; break;
-                case FD_MAP_SCANT: blocks = fdk::scan_chunks(a.nT); break;
-                case FD_MAP_SCANO: blocks = fdk::scan_chunks(std::max(a.ntris, 1)); break;
+                case FD_MAP_SCAN: blocks = fdk::scan_blocks(a); break;
                 case FD_MAP_NB: blocks = nb + 1; break;
                 case FD_MAP_ZERO: blocks = a.segs > 1 ? fdk::zero_blocks(a) : 0; break;
                 case FD_MAP_FIN: blocks = a.segs > 1 ? a.chunkSlots : 0; break;

@@ -54,6 +54,8 @@ struct FdArgs {
     int nblkT;            // blocks of the triangle count / scatter passes
     int nbR, nbV;         // k_reduce blocks over receivers / vertices
     long nR, nT;          // lengths of the receiver / pair histograms
+    uint32_t* rxTot;      // nb + 1: receivers per key
+    uint32_t* triTot;     // nb: pairs per bin
     int* sortedId;        // WH
     FdRxRec* sortedRec;   // WH
     uint32_t* binStat;    // nb * 5 (order-preserving encodings)
@@ -69,14 +71,12 @@ struct FdArgs {
     int* sortedTri;       // pairCap
     unsigned long long pairCap;
     int* rxStart;         // nb + 1
-    int* rxEnd;           // nb + 1
+    int* rxEnd;           // nb + 1 (rxStart + 1)
     int* triStart;        // nb
-    int* triEnd;          // nb
+    int* triEnd;          // nb (triStart + 1)
     int* chunkStart;      // nb + 1: first work item of each bin (in occlusion order)
     FdChunk* chunks;      // chunkSlots: the work items (over histR / histT, done with by then)
-    int* binAtRank;       // nb + 1: occlusion order of the bins, longest triangle list first
-    uint64_t* scanPart;   // scan partial sums
-    uint32_t* part;       // per-block partials: 8 per k_reduce block (value-major), then 1 per pair-count block
+    uint32_t* part;       // per-block partials: 8 per k_reduce block (value-major), then 2 per pair-count block
     unsigned long long* opCount;  // optional occlusion counters (FD_NOPS), or null
     // occlusion work split: chunkSlots = receiver chunk slots (64 each, an upper
     // bound of the work items); each bin's triangle list is cut into segs
@@ -147,23 +147,26 @@ inline int fd_occ_class(int wpr, int occWaves) { return (wpr - 1) * 3 + (occWave
 #define FD_LDS_BINS 1024
 #define FD_BIN_LDS_BYTES 20
 
-// Pair scatter with all 16 waves of a triangle block: 16 x 16-bit per-wave
-// counts and a 32-bit block offset per bin in LDS (144 KiB at the largest
+// Scatters with all 16 waves of a block: 16 x 16-bit per-wave counts, and for
+// the pairs a 32-bit block offset, per bin in LDS (144 KiB at the largest
 // grid, 64 x 64 = 4096 bins).
+#define FD_SCATTER_RX_LDS 32
 #define FD_SCATTER_WIDE_LDS 36
+
+// Scans: rows of a histogram (nblk counts each) per block, about 4096 counts
+__host__ __device__ inline int fd_scan_rows(int nblk) { return nblk >= 4096 ? 1 : 4096 / nblk; }
 
 // Occlusion counters, in the order documented at fd_get_profile.
 #define FD_NOPS FD_PROFILE_COUNTERS
 
 // Stage boundaries recorded when profiling (events[0..FD_NSTAGES]).
-#define FD_NSTAGES 5   // light plane, receiver binning, triangle pairing, tables, occlusion
+#define FD_NSTAGES 5   // light plane, receiver keys, triangle pairing (and both scatters), list order, occlusion
 
-#define FD_FIN_THREADS 1024   // k_finalize / k_post_pairs block size
+#define FD_FIN_THREADS 1024   // k_finalize block size
 
 // Block maps of a batched launch (prefix sums over instances, n + 1 each).
-enum FdMap { FD_MAP_ONE, FD_MAP_BINS, FD_MAP_RED, FD_MAP_RX, FD_MAP_SCANR, FD_MAP_TRI, FD_MAP_SCANT, FD_MAP_OCC0,
-             FD_MAP_OCC1, FD_MAP_OCC2, FD_MAP_OCC3, FD_MAP_OCC4, FD_MAP_OCC5, FD_MAP_ZERO, FD_MAP_FIN, FD_MAP_SCANO,
-             FD_MAP_NB, FD_NMAPS };
+enum FdMap { FD_MAP_ONE, FD_MAP_RED, FD_MAP_RX, FD_MAP_TRI, FD_MAP_SCAN, FD_MAP_OCC0, FD_MAP_OCC1, FD_MAP_OCC2,
+             FD_MAP_OCC3, FD_MAP_OCC4, FD_MAP_OCC5, FD_MAP_ZERO, FD_MAP_FIN, FD_MAP_NB, FD_NMAPS };
 static_assert(FD_MAP_OCC0 + FD_OCC_CLASSES == FD_MAP_ZERO, "one block map per occlusion class");
 static_assert(FD_TRI_CLASSES < (1 << FD_WALK_KEY_BITS), "area classes and the no-entry value fit the key bits");
 
@@ -181,8 +184,7 @@ struct FdBatchPlan {
 namespace fdk {
 hipError_t enqueue_frame(const FdArgs& a, hipStream_t st, hipEvent_t* stageEvents = nullptr);
 hipError_t enqueue_batch(const FdBatchPlan& p, hipStream_t st);
-long scan_partials_needed(long n);
 int reduce_blocks(long n);
-int scan_chunks(long n);
+int scan_blocks(const FdArgs& a);
 int zero_blocks(const FdArgs& a);   // blocks of the mask-zeroing pass
 }  // namespace fdk

@@ -5,10 +5,10 @@
 //   verticesRectangleAABBcal + AABBReduce_kernel  -> k_reduce (one pass)
 //   lightPlaneParamCal host part                 -> k_finalize
 //   writeSampleAndBinPair + maxZpreBinReduce      -> k_rx_key
-//   thrust::sort_by_key (receivers) + FindStart    -> k_scan_* + k_rx_scatter
+//   thrust::sort_by_key (receivers) + FindStart    -> k_scan + k_rx_scatter
 //   triangleVertexSetup + countPairNumForPerTri    -> k_tri_count
-//   exclusive_scan + writeTriBinPair + sort_by_key -> k_scan_* + k_tri_write + k_tri_scatter_wide
-//   findTriangleStartEnd                           -> k_tables
+//   exclusive_scan + writeTriBinPair + sort_by_key -> k_scan + k_tri_scatter
+//   findTriangleStartEnd                           -> k_scan (block 0)
 //   shadowCal_per_sample_kernel                    -> k_occlude
 //
 // Every kernel reads the frame status first, so the whole frame is one
@@ -23,19 +23,16 @@ using namespace fdk;
 
 namespace {
 
-constexpr int RED_BLOCK = 256;
-constexpr int RED_ITEMS = 8;           // receivers / vertices per thread in k_reduce
-constexpr int SCAN_BLOCK = 256;
-constexpr int SCAN_ITEMS = 16;
+constexpr int RED_BLOCK = 1024;
+constexpr int RED_ITEMS = 2;           // receivers / vertices per thread in k_reduce
+constexpr int SCAN_BLOCK = 1024;
+constexpr int SCAN_ITEMS = 4;
 constexpr int SCAN_CHUNK = SCAN_BLOCK * SCAN_ITEMS;
+static_assert(SCAN_CHUNK % FD_TRB == 0, "a chunk of pair counts covers whole triangle blocks");
 
-// --------------------------------------------------------------------------
-// k_init: reset the frame state (a kernel, not a memset, so that replays of
-// a captured graph start from the same state).
-// --------------------------------------------------------------------------
-__device__ __forceinline__ void init_body(const FdArgs& a, const int blk) {
-    if (threadIdx.x != 0 || blk != 0) return;
-    FdState* s = a.st;
+// Resets the frame state (by k_finalize's first thread: nothing reads the state
+// before, and replays of a captured graph start from the same one).
+__device__ __forceinline__ void init_state(FdState* s) {
     const uint32_t encMax = fenc(FD_F32_MAX), encNegMax = fenc(-FD_F32_MAX);
     s->rxZmaxAll = encNegMax;
     s->rxMin[0] = s->rxMin[1] = s->rxMin[2] = encMax;
@@ -57,22 +54,37 @@ __device__ __forceinline__ void init_body(const FdArgs& a, const int blk) {
     s->triOrder = FD_TRI_ORDER_LIST;
 }
 
-// Bin statistics reset (maxZ, minRange) for the bins of this frame.
-__device__ __forceinline__ void init_bins_body(const FdArgs& a, const int blk) {
-    int b = blk * blockDim.x + threadIdx.x;
+// Resets the bin statistics (maxZ, minRange) and totals of this frame, dealt
+// over k_reduce's blocks.
+__device__ __forceinline__ void init_bins(const FdArgs& a, const int blk, const int blocks) {
     const int nb = 1 << (2 * a.gridLog2);
-    if (b >= nb) return;
     const uint32_t encMax = fenc(FD_F32_MAX), encNegMax = fenc(-FD_F32_MAX);
-    a.binStat[5 * b + 0] = encNegMax;  // maxZ
-    a.binStat[5 * b + 1] = encNegMax;  // max of rect min x
-    a.binStat[5 * b + 2] = encNegMax;  // max of rect min y
-    a.binStat[5 * b + 3] = encMax;     // min of rect max x
-    a.binStat[5 * b + 4] = encMax;     // min of rect max y
+    for (int b = blk * RED_BLOCK + threadIdx.x; b <= nb; b += blocks * RED_BLOCK) {
+        a.rxTot[b] = 0;
+        if (b == nb) break;
+        a.triTot[b] = 0;
+        a.binStat[5 * b + 0] = encNegMax;  // maxZ
+        a.binStat[5 * b + 1] = encNegMax;  // max of rect min x
+        a.binStat[5 * b + 2] = encNegMax;  // max of rect min y
+        a.binStat[5 * b + 3] = encMax;     // min of rect max x
+        a.binStat[5 * b + 4] = encMax;     // min of rect max y
+    }
 }
 
 // Block-level reduction of NV uint32 values with op (0 = min, 1 = max,
 // 2 = sum); the block's results go to part[k * P + blk] (no atomics: many
 // blocks updating the few words of the frame state would serialise).
+static_assert(RED_BLOCK / 64 == 16 && FD_FIN_THREADS / 64 == 16, "one 16-lane row holds a block's waves");
+// op over a 16-lane row, in lane 15 of it (every lane of the row active)
+__device__ __forceinline__ uint32_t row_reduce(uint32_t v, int op) {
+    auto f = [&](uint32_t x) { v = op == 2 ? v + x : op ? max(v, x) : min(v, x); };
+    const bool sum = op == 2;
+    f((uint32_t)dpp_or<0x111, 0xf>(sum ? 0 : (int)v, (int)v));
+    f((uint32_t)dpp_or<0x112, 0xf>(sum ? 0 : (int)v, (int)v));
+    f((uint32_t)dpp_or<0x114, 0xf>(sum ? 0 : (int)v, (int)v));
+    f((uint32_t)dpp_or<0x118, 0xf>(sum ? 0 : (int)v, (int)v));
+    return v;
+}
 template <int NV>
 __device__ void block_reduce_store(uint32_t (&v)[NV], const int (&op)[NV], uint32_t* part, int P, int blk) {
     __shared__ uint32_t sh[NV][RED_BLOCK / 64];
@@ -83,12 +95,11 @@ __device__ void block_reduce_store(uint32_t (&v)[NV], const int (&op)[NV], uint3
         if (l == 0) sh[k][w] = r;
     }
     __syncthreads();
-    if (threadIdx.x < NV) {
-        const int k = threadIdx.x;
-        uint32_t r = sh[k][0];
-        for (int i = 1; i < RED_BLOCK / 64; ++i)
-            r = op[k] == 2 ? r + sh[k][i] : op[k] ? max(r, sh[k][i]) : min(r, sh[k][i]);
-        part[(size_t)k * P + blk] = r;
+    // one 16-lane row per value: its waves' results
+    if (threadIdx.x < NV * (RED_BLOCK / 64)) {
+        const int k = threadIdx.x >> 4, j = threadIdx.x & 15;
+        const uint32_t r = row_reduce(sh[k][j], op[k]);
+        if (j == 15) part[(size_t)k * P + blk] = r;
     }
 }
 
@@ -96,7 +107,9 @@ __device__ void block_reduce_store(uint32_t (&v)[NV], const int (&op)[NV], uint3
 // k_reduce: one pass over receivers (blocks [0, nbR)) and vertices (blocks
 // [nbR, nbR + nbV)).  Receivers: z for the far plane
 // (Step2_1_samplerRectangleAABB.inl:1-34), back-face test against the four
-// light corners and the light-plane rectangle (:53-137).  The rectangle's max
+// light corners and the light-plane rectangle (:53-137).  1024 threads with two
+// elements each: a thread's chain of loads is what small frames wait for (256
+// threads with eight each: 7.8 us for 64 x 64 receivers, now 5.2).  The rectangle's max
 // corner x' + F/z - S is reduced as max(x' + F/z) - S after the frame's S is
 // known: rounding of (a - S) is monotone in a, so both give the same float.
 // Vertices: Step2_2_modelRectangleAABB.inl:1-99.
@@ -104,6 +117,7 @@ __device__ void block_reduce_store(uint32_t (&v)[NV], const int (&op)[NV], uint3
 __device__ __forceinline__ void reduce_body(const FdArgs& a, const int blk) {
     const int nbR = a.nbR;
     const float* m = a.L.m;
+    init_bins(a, blk, nbR + a.nbV);
     const uint32_t encMax = fenc(FD_F32_MAX), encNegMax = fenc(-FD_F32_MAX);
     if ((int)blk < nbR) {
         uint32_t v[7] = {encNegMax, encMax, encMax, encMax, encNegMax, encNegMax, encNegMax};
@@ -172,6 +186,8 @@ __device__ __forceinline__ void reduce_body(const FdArgs& a, const int blk) {
 // --------------------------------------------------------------------------
 // k_finalize: the host part of lightPlaneParamCal
 // (Step2_3_defineFDbuffer.inl:5-111) on the device, with its early exits.
+// Latency-bound: 16-lane rows reduce the waves' results (one thread that walked
+// all 256 of them: 10.0 us, now 4.6).
 // --------------------------------------------------------------------------
 __device__ __forceinline__ void finalize_body(const FdArgs& a, const int blk) {
     if (blk != 0) return;
@@ -196,25 +212,25 @@ __device__ __forceinline__ void finalize_body(const FdArgs& a, const int blk) {
             }
         }
         const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
+        __shared__ uint32_t o[2][8];
 #pragma unroll
         for (int g = 0; g < 2; ++g)
 #pragma unroll
             for (int k = 0; k < 8; ++k) {
-                const uint32_t x = op[k] == 2 ? (uint32_t)wave_sum_i32((int)r[g][k])
-                                              : op[k] ? wave_max_u32(r[g][k]) : wave_min_u32(r[g][k]);
+                uint32_t x = r[g][k];   // the start value where the wave has no partial
+                if (w * 64 < P)
+                    x = op[k] == 2 ? (uint32_t)wave_sum_i32((int)x) : op[k] ? wave_max_u32(x) : wave_min_u32(x);
                 if (l == 0) red[g][k][w] = x;
             }
         __syncthreads();
+        if (threadIdx.x < 256) {   // one 16-lane row per value
+            const int g = threadIdx.x >> 7, k = (threadIdx.x >> 4) & 7, j = threadIdx.x & 15;
+            const uint32_t x = row_reduce(red[g][k][j], k == 7 ? 2 : (k == 0 || k > 3) ? 1 : 0);
+            if (j == 15) o[g][k] = x;
+        }
+        __syncthreads();
         if (threadIdx.x != 0) return;
-        const int nw = (int)(blockDim.x + 63) >> 6;
-        uint32_t o[2][8];
-        for (int g = 0; g < 2; ++g)
-            for (int k = 0; k < 8; ++k) {
-                uint32_t x = red[g][k][0];
-                for (int j = 1; j < nw; ++j)
-                    x = op[k] == 2 ? x + red[g][k][j] : op[k] ? max(x, red[g][k][j]) : min(x, red[g][k][j]);
-                o[g][k] = x;
-            }
+        init_state(s);
         s->rxZmaxAll = o[0][0];
         s->rxMin[0] = o[0][1]; s->rxMin[1] = o[0][2]; s->rxMin[2] = o[0][3];
         s->rxMaxA[0] = o[0][4]; s->rxMaxA[1] = o[0][5];
@@ -264,7 +280,8 @@ __device__ __forceinline__ void finalize_body(const FdArgs& a, const int blk) {
 // Receiver key (writeSampleAndBinPair, Step3_bindSampleToBin.inl:5-59) and
 // the per-bin receiver statistics (maxZpreBinReduce_kernel, :61-104), which
 // are min/max reductions and so are folded into the same pass with atomics.
-// Each block owns RXB consecutive receivers and writes its key histogram.
+// Each block owns RXB consecutive receivers, one per thread, and writes its key
+// histogram (256 threads with four each: 15.8 us for 64 x 64 receivers, now 8.2).
 // --------------------------------------------------------------------------
 struct RxRect { float bx, by, ex, ey, z; };
 
@@ -324,8 +341,8 @@ __device__ __forceinline__ void rx_key_body(const FdArgs& a, const int blk) {
     __syncthreads();
     int nvalid = 0, noor = 0;
     const int base = blk * FD_RXB;
-    for (int it = 0; it < FD_RXB / 256; ++it) {
-        const int p = base + it * 256 + threadIdx.x;
+    {
+        const int p = base + threadIdx.x;
         const int i = p < a.npos ? tile_id(p, a.W, a.H, a.tileLog2) : -1;
         int key = nb;
         RxRect q{};
@@ -380,12 +397,13 @@ __device__ __forceinline__ void rx_key_body(const FdArgs& a, const int blk) {
     }
     __syncthreads();
     // valid receivers = binned ones (the scanned histogram) + out-of-range
-    // keys, totalled in k_post_pairs; only the rare out-of-range count is
+    // keys, totalled in k_scan; only the rare out-of-range count is
     // accumulated here
     if (threadIdx.x == 0 && blkCount[1]) atomicAdd(&a.st->keyOutOfRange, (int)blkCount[1]);
     for (int k = threadIdx.x; k <= nb; k += blockDim.x) {
         const uint32_t h = hist[k];
         a.histR[(size_t)k * a.nblkR + blk] = h;
+        if (h) atomicAdd(a.rxTot + k, h);
         if (ldsStat && k < nb && h) {
             const uint32_t* l = bstat + 5 * k;
             uint32_t* bs = a.binStat + 5 * k;
@@ -396,125 +414,136 @@ __device__ __forceinline__ void rx_key_body(const FdArgs& a, const int blk) {
 }
 
 // --------------------------------------------------------------------------
-// Device-wide exclusive scan of uint32 counts (thrust::exclusive_scan /
-// the offsets of a stable counting sort) in two launches: chunk sums, then
-// each chunk's scan offset by the sums before it.  Totals are kept in 64 bits.
+// Device-wide exclusive scans of uint32 counts (thrust::exclusive_scan / the
+// offsets of a stable counting sort), one launch for all three of a frame:
+// the blocks know what lies before them from sums that the counting passes
+// leave behind (per bin, per triangle block), so no pass over the counts comes
+// first.  Modulo 2^32; the number of pairs is totalled in 64 bits.
+//
+// Bound: latency.  Six launches (a pass of chunk sums and a pass of offsets
+// for each array) of 4 to 8 us each before, and 9 us for the exits and tables;
+// one of 7.5 us (64 x 64 receivers) to 10 us (1920 x 1080) now.
 // --------------------------------------------------------------------------
-__device__ __forceinline__ uint64_t block_excl_scan_u64(uint64_t v, uint64_t* tot) {
-    __shared__ uint64_t wsum[SCAN_BLOCK / 64];
+// the frame got past k_finalize: receivers are binned (also where no triangle
+// or no pair is found, or too many)
+__device__ __forceinline__ bool binned(int status) {
+    return status == FD_EXIT_OK || status == FD_EXIT_NO_VALID_TRI || status == FD_EXIT_NO_PAIRS ||
+           status == FD_EXIT_CAPACITY;
+}
+
+// Exclusive prefix of v over the block's 1024 threads; total: over all of them.
+__device__ __forceinline__ uint32_t block_excl_scan(uint32_t v, uint32_t (&sh)[16], uint32_t& total) {
     const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
-    uint64_t x = v;
+    const uint32_t x = wave_incl_scan(v);
+    __syncthreads();   // sh is free again
+    if (l == 63) sh[w] = x;
+    __syncthreads();
+    uint32_t off = 0, all = 0;
 #pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        uint64_t y = __shfl_up(x, o, 64);
-        if (l >= o) x += y;
+    for (int i = 0; i < 16; ++i) {
+        const uint32_t t = sh[i];
+        off += i < w ? t : 0u;
+        all += t;
     }
-    if (l == 63) wsum[w] = x;
-    __syncthreads();
-    uint64_t off = 0, all = 0;
-    for (int i = 0; i < SCAN_BLOCK / 64; ++i) {
-        if (i < w) off += wsum[i];
-        all += wsum[i];
-    }
-    __syncthreads();
-    *tot = all;
+    total = all;
     return off + x - v;
 }
 
-__device__ __forceinline__ void scan_reduce_body(const uint32_t* __restrict__ d, long n, uint64_t* __restrict__ part,
-                                                 const int* status, const int blk) {
-    if (status && *status != FD_EXIT_OK) return;
-    const long base = (long)blk * SCAN_CHUNK + threadIdx.x * SCAN_ITEMS;
-    uint64_t sum = 0;
+__device__ __forceinline__ uint32_t block_sum(uint32_t v, uint32_t (&sh)[16]) {
+    const uint32_t x = (uint32_t)wave_sum_i32((int)v);
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = x;
+    __syncthreads();
+    uint32_t all = 0;
 #pragma unroll
-    for (int k = 0; k < SCAN_ITEMS; ++k)
-        if (base + k < n) sum += d[base + k];
-    uint64_t tot;
-    block_excl_scan_u64(sum, &tot);
-    if (threadIdx.x == 0) part[blk] = tot;
+    for (int i = 0; i < 16; ++i) all += sh[i];
+    return all;
 }
 
-// Second pass: each chunk adds the sum of the chunk sums before it (read
-// from part[], at most a few hundred values, by the whole block) to its own
-// exclusive scan; block 0 also writes the grand total.
-__device__ __forceinline__ void scan_apply_body(uint32_t* __restrict__ d, long n, const uint64_t* __restrict__ part,
-                                                unsigned long long* total, const int* status, const int blk) {
-    if (status && *status != FD_EXIT_OK) return;
-    const int np = (int)((n + SCAN_CHUNK - 1) / SCAN_CHUNK);
-    uint64_t pre = 0, all = 0;
-    for (int i = threadIdx.x; i < np; i += SCAN_BLOCK) {
-        const uint64_t x = part[i];
-        if (i < blk) pre += x;
-        all += x;
-    }
-    uint64_t preTot, allTot;
-    block_excl_scan_u64(pre, &preTot);
-    block_excl_scan_u64(all, &allTot);
-    if (blk == 0 && threadIdx.x == 0 && total) *total = allTot;
-    const long base = (long)blk * SCAN_CHUNK + threadIdx.x * SCAN_ITEMS;
-    uint32_t v[SCAN_ITEMS];
-    uint64_t sum = 0;
+// d[e0 .. e1), in place, by one block; base: the sum of what comes before
+__device__ __forceinline__ void scan_range(uint32_t* __restrict__ d, long e0, long e1, uint32_t base, uint32_t (&sh)[16]) {
+    for (long c = e0; c < e1; c += SCAN_CHUNK) {
+        const long i0 = c + threadIdx.x * SCAN_ITEMS;
+        uint32_t v[SCAN_ITEMS], sum = 0;
 #pragma unroll
-    for (int k = 0; k < SCAN_ITEMS; ++k) {
-        v[k] = (base + k < n) ? d[base + k] : 0u;
-        sum += v[k];
-    }
-    uint64_t tot;
-    uint64_t off = block_excl_scan_u64(sum, &tot) + preTot;
+        for (int k = 0; k < SCAN_ITEMS; ++k) v[k] = i0 + k < e1 ? d[i0 + k] : 0u;
 #pragma unroll
-    for (int k = 0; k < SCAN_ITEMS; ++k) {
-        if (base + k < n) d[base + k] = (uint32_t)off;
-        off += v[k];
+        for (int k = 0; k < SCAN_ITEMS; ++k) sum += v[k];
+        uint32_t tot;
+        uint32_t off = base + block_excl_scan(sum, sh, tot);
+        base += tot;
+#pragma unroll
+        for (int k = 0; k < SCAN_ITEMS; ++k) {
+            if (i0 + k < e1) d[i0 + k] = off;
+            off += v[k];
+        }
     }
+}
+
+// rows [r0, r1) of a histogram, nblk counts each; tot: the rows' sums
+__device__ __forceinline__ void scan_rows(uint32_t* d, const uint32_t* __restrict__ tot, int r0, int r1, int nblk,
+                                          uint32_t (&sh)[16]) {
+    uint32_t pre = 0;
+    for (int k = threadIdx.x; k < r0; k += SCAN_BLOCK) pre += tot[k];
+    const uint32_t base = block_sum(pre, sh);
+    scan_range(d, (long)r0 * nblk, (long)r1 * nblk, base, sh);
 }
 
 // --------------------------------------------------------------------------
-// Stable receiver scatter: one wave per block walks its RXB receivers in
-// order, 64 at a time; lanes holding equal keys are matched with ballots
-// over the key bits and ranked with mbcnt, so the result equals a stable
-// sort_by_key (Step3_bindSampleToBin.inl:125-127).  Binned receivers also
-// get their 32-byte occlusion record written in sorted order.
+// Stable receiver scatter: each of the block's 16 waves takes 64 of its
+// receivers; lanes holding equal keys are matched with ballots over the key
+// bits and ranked with mbcnt, and the counts of the waves before (16-bit, a row
+// of 16 per key in LDS) place the wave within the block, so the result equals a
+// stable sort_by_key (Step3_bindSampleToBin.inl:125-127).  Binned receivers
+// also get their 32-byte occlusion record written in sorted order.
+//
+// Bound: latency for small views, then memory (134 MB at 1920 x 1080).  One
+// wave that walked a block's receivers 64 at a time took 18 us for 64 x 64 and
+// 27 us for 1920 x 1080 receivers; 16 waves take 4.5 and 21.6.
 // --------------------------------------------------------------------------
 __device__ __forceinline__ void rx_scatter_body(const FdArgs& a, const int blk) {
-    extern __shared__ int cnt[];  // nb + 1, -1 = not loaded yet
+    extern __shared__ __align__(16) uint32_t rcnt[];  // (nb + 1) x 16 counts of 16 bits
     const FdState* s = a.st;
-    if (s->status != FD_EXIT_OK) return;
+    if (!binned(s->status)) return;
     const int nb = s->nb;
-    int kbits = 1;
-    while ((1 << kbits) <= nb) ++kbits;
-    for (int k = threadIdx.x; k <= nb; k += 64) cnt[k] = -1;
+    const int kbits = 2 * s->log2G + 1;   // keys 0 .. nb
+    const int w = threadIdx.x >> 6;
+    for (int k = threadIdx.x; k < (nb + 1) * 2; k += FD_RXB) ((uint4*)rcnt)[k] = make_uint4(0u, 0u, 0u, 0u);
+    const int p = blk * FD_RXB + threadIdx.x;
+    const int i = p < a.npos ? tile_id(p, a.W, a.H, a.tileLog2) : -1;
+    const bool act = i >= 0;
+    const int key = act ? (int)a.rxKey[i] : 0;
+    const uint32_t base = act ? a.histR[(size_t)key * a.nblkR + blk] : 0u;
+    float4 r = make_float4(0.f, 0.f, 0.f, 0.f), ps = r;
+    if (act && key < nb) {
+        r = a.rec[i];
+        ps = a.pos[i];
+    }
+    uint64_t eq = __ballot(act);
+    for (int b = 0; b < kbits; ++b) {
+        const bool bit = (key >> b) & 1;
+        const uint64_t bal = __ballot(act && bit);
+        eq &= bit ? bal : ~bal;
+    }
+    const int rank = mbcnt(eq);
     __syncthreads();
-    const int base = blk * FD_RXB;
-    for (int it = 0; it < FD_RXB / 64; ++it) {
-        const int pp = base + it * 64 + lane_id();
-        const int i = pp < a.npos ? tile_id(pp, a.W, a.H, a.tileLog2) : -1;
-        const bool act = i >= 0;
-        const int key = act ? (int)a.rxKey[i] : 0;
-        uint64_t eq = __ballot(act);
-        for (int b = 0; b < kbits; ++b) {
-            const bool bit = (key >> b) & 1;
-            const uint64_t bal = __ballot(act && bit);
-            eq &= bit ? bal : ~bal;
-        }
-        if (act) {
-            const int rank = mbcnt(eq);
-            const int gcount = __popcll(eq);
-            int b0 = cnt[key];
-            if (b0 < 0) b0 = (int)a.histR[(size_t)key * a.nblkR + blk];
-            const int p = b0 + rank;
-            if (rank == gcount - 1) cnt[key] = b0 + gcount;
-            if ((unsigned)p < (unsigned)a.WH) a.sortedId[p] = i;
-            if (key < nb && (unsigned)p < (unsigned)a.WH) {
-                const float4 r = a.rec[i];
-                const RxRect q = rx_rect(r, s, a.L);
-                const float4 ps = a.pos[i];
-                FdRxRec o;
-                o.q[0] = ps.x; o.q[1] = ps.y; o.q[2] = ps.z;
-                o.rminx = q.bx; o.rminy = q.by; o.rmaxx = q.ex; o.rmaxy = q.ey; o.z = q.z;
-                a.sortedRec[p] = o;
-            }
-        }
-        __syncthreads();
+    if (act && rank == 0) ((uint16_t*)rcnt)[16 * key + w] = (uint16_t)__popcll(eq);
+    __syncthreads();
+    if (!act) return;
+    // counts of the waves before this one: two per word, at most 1024 in all
+    uint32_t sum = 0;
+    for (int j = 0; j < (w >> 1); ++j) sum += rcnt[8 * key + j];
+    sum = (sum & 0xffffu) + (sum >> 16);
+    if (w & 1) sum += rcnt[8 * key + (w >> 1)] & 0xffffu;
+    const uint32_t d = base + sum + (uint32_t)rank;
+    if (d >= (uint32_t)a.WH) return;
+    a.sortedId[d] = i;
+    if (key < nb) {
+        const RxRect q = rx_rect(r, s, a.L);
+        FdRxRec o;
+        o.q[0] = ps.x; o.q[1] = ps.y; o.q[2] = ps.z;
+        o.rminx = q.bx; o.rminy = q.by; o.rmaxx = q.ex; o.rmaxy = q.ey; o.z = q.z;
+        a.sortedRec[d] = o;
     }
 }
 
@@ -635,7 +664,7 @@ __device__ __forceinline__ void tri_count_body(const FdArgs& a, const int blk) {
     // nb counters, then the staged bin statistics (float4 + float per bin);
     // 16-byte aligned behind the block's static counters, for the float4s
     extern __shared__ __align__(16) uint32_t thist[];
-    __shared__ uint32_t blkValid, blkPairs, blkOverlaps;
+    __shared__ uint32_t blkStat, blkSum;   // valid | neighbours << 11 | overlaps << 21; pairs
     const FdState* s = a.st;
     if (s->status != FD_EXIT_OK) return;
     const int nb = s->nb, log2G = s->log2G;
@@ -643,7 +672,7 @@ __device__ __forceinline__ void tri_count_body(const FdArgs& a, const int blk) {
     float4* binQ = (float4*)(thist + nb);
     float* binW = (float*)(binQ + nb);
     for (int k = threadIdx.x; k < nb; k += blockDim.x) thist[k] = 0;
-    if (threadIdx.x == 0) blkValid = blkPairs = blkOverlaps = 0;
+    if (threadIdx.x == 0) blkStat = blkSum = 0;
     if (staged) stage_bins(a, nb, binQ, binW);
     __syncthreads();
     const int t = blk * FD_TRB + threadIdx.x;
@@ -728,8 +757,7 @@ __device__ __forceinline__ void tri_count_body(const FdArgs& a, const int blk) {
         a.triClass[t] = (uint8_t)(valid ? area_class(px, py, s) : FD_TRI_CLASSES - 1);
     }
     {
-        const int nv = wave_sum_i32(valid);
-        if (lane_id() == 0 && nv) atomicAdd(&blkValid, (uint32_t)nv);
+        const int nv = __popcll(__ballot(valid));
         // list coherence: how often a valid triangle's culling box overlaps
         // the next triangle's (the next lane's; the wave's last lane has none)
         const float nx0 = __shfl_down(mn.x, 1, 64), ny0 = __shfl_down(mn.y, 1, 64);
@@ -738,10 +766,7 @@ __device__ __forceinline__ void tri_count_body(const FdArgs& a, const int blk) {
         const bool pair = valid && nvld && lane_id() < 63;
         const bool over = pair && mn.x <= nx1 && nx0 <= mx.x && mn.y <= ny1 && ny0 <= mx.y;
         const int np = __popcll(__ballot(pair)), no = __popcll(__ballot(over));
-        if (lane_id() == 0 && np) {
-            atomicAdd(&blkPairs, (uint32_t)np);
-            atomicAdd(&blkOverlaps, (uint32_t)no);
-        }
+        if (lane_id() == 0 && nv) atomicAdd(&blkStat, (uint32_t)(nv | np << 11 | no << 21));
     }
     // count pass
     TriClamp c = tri_clamp(mn, mx, s);
@@ -791,13 +816,18 @@ __device__ __forceinline__ void tri_count_body(const FdArgs& a, const int blk) {
         a.triOff[t] = (uint32_t)count;
         a.triRange[t] = make_uint2((uint32_t)tsx | ((uint32_t)tsy << 16), (uint32_t)tex | ((uint32_t)tey << 16));
     }
+    const int sum = wave_sum_i32(count);
+    if (lane_id() == 0 && sum) atomicAdd(&blkSum, (uint32_t)sum);
     __syncthreads();
-    if (threadIdx.x == 0) {   // totalled in k_post_pairs
-        a.part[blk] = blkValid;
-        a.part[a.nblkT + blk] = blkPairs;
-        a.part[2 * a.nblkT + blk] = blkOverlaps;
+    if (threadIdx.x == 0) {
+        a.part[blk] = blkStat;
+        a.part[a.nblkT + blk] = blkSum;
     }
-    for (int k = threadIdx.x; k < nb; k += blockDim.x) a.histT[(size_t)k * a.nblkT + blk] = thist[k];
+    for (int k = threadIdx.x; k < nb; k += blockDim.x) {
+        const uint32_t h = thist[k];
+        a.histT[(size_t)k * a.nblkT + blk] = h;
+        if (h) atomicAdd(a.triTot + k, h);
+    }
 }
 
 // The large rectangles of the write pass, walked by the whole wave; a pair's
@@ -829,25 +859,47 @@ __device__ __forceinline__ void tri_write_big(const FdArgs& a, int log2G, bool s
 }
 
 // Stable pair scatter (writeTriBinPair_kernel + sort_by_key,
-// Step4_RasterizeTriangleToBin.inl:161-223): per bin, triangles ascending.
-// Pair write: every triangle writes its (bin) pairs at its triangle-major
-// offset (scanned pair counts), bins ascending within the triangle -- the
-// order in which the reference's writeTriBinPair_kernel emits them
-// (Step4_RasterizeTriangleToBin.inl:161-204), with the count pass's test.
-__device__ __forceinline__ void tri_write_body(const FdArgs& a, const int blk) {
-    extern __shared__ uint32_t lds[];   // staged bin statistics
+// Step4_RasterizeTriangleToBin.inl:161-223): per bin, triangles ascending, one
+// block of 1024 triangles at a time.
+//
+// First every triangle writes its (bin) pairs at its triangle-major offset
+// (scanned pair counts), bins ascending within the triangle -- the order in
+// which the reference's writeTriBinPair_kernel emits them (:161-204), with the
+// count pass's test.  The block's pairs then are one stretch of that list, and
+// its 16 waves sort equal slices of the stretch by bin: a pair of a bin means a
+// triangle of its own, so a block has at most 1024 pairs of a bin and the 16
+// per-wave counts of a bin fit 16-bit halves of LDS words (two waves per word,
+// counted with 32-bit LDS adds).  After a barrier every bin's counts become
+// exclusive prefixes over the waves, and each wave ranks its slice from base +
+// prefix: lanes with equal bins are matched by ballots over the key bits and
+// ranked with mbcnt, the last lane of a group advances the running offset.
+// Result: bin-major, ascending triangle id within a bin.  LDS:
+// FD_SCATTER_WIDE_LDS bytes per bin (bins <= 4096: grids up to 64 x 64), and
+// before them the staged bin statistics.
+//
+// Bound: the ranking's chain of ballots, 64 pairs a step.  Slices of equal
+// length keep the 16 waves alike: one slice per 64 triangles, in a launch of its
+// own after the write, took 11 + 32 us for 512 x 512 receivers and 40 k
+// triangles, and 29 + 69 us for 970 k; now 20 and 87 us.
+__device__ __forceinline__ int wide_half(int w, int k, int nb) { return (((w >> 1) * nb + k) << 1) | (w & 1); }
+
+__device__ __forceinline__ void tri_scatter_body(const FdArgs& a, const int blk) {
+    extern __shared__ __align__(16) uint32_t wlds[];
     const FdState* s = a.st;
     if (s->status != FD_EXIT_OK) return;
     const int nb = s->nb, log2G = s->log2G;
     const bool staged = a.binLds && nb <= FD_LDS_BINS;
-    float4* binQ = (float4*)lds;
+    float4* binQ = (float4*)wlds;
     float* binW = (float*)(binQ + nb);
-    if (staged) {
-        stage_bins(a, nb, binQ, binW);
-        __syncthreads();
-    }
-    const int t = blk * FD_TRB + threadIdx.x;
-    if (uniform(blk * FD_TRB + (int)(threadIdx.x & ~63u)) >= a.ntris) return;   // whole wave past the end
+    uint32_t* cnt32 = wlds + (staged ? nb * (FD_BIN_LDS_BYTES / 4) : 0);   // 8 * nb words
+    uint16_t* cnt16 = (uint16_t*)cnt32;
+    uint32_t* base = cnt32 + 8 * nb;                                       // nb block offsets
+    if (staged) stage_bins(a, nb, binQ, binW);
+    for (int k = threadIdx.x; k < 8 * nb; k += FD_TRB) cnt32[k] = 0u;
+    for (int k = threadIdx.x; k < nb; k += FD_TRB) base[k] = a.histT[(size_t)k * a.nblkT + blk];
+    const unsigned long long cap = a.pairCap;
+    const int t0 = blk * FD_TRB;
+    const int t = t0 + threadIdx.x;
     // the walk over the pair range (bins with pairs) of the count pass
     bool has = t < a.ntris;
     int sx = 0, sy = 0, ex = 0, ey = 0;
@@ -855,87 +907,62 @@ __device__ __forceinline__ void tri_write_body(const FdArgs& a, const int blk) {
     unsigned long long o = 0;
     if (has) {
         const uint2 rg = a.triRange[t];
+        const float4 mn = a.triAABB[2 * t], mx = a.triAABB[2 * t + 1];
+        o = a.triOff[t];
         sx = rg.x & 0xffff; sy = rg.x >> 16; ex = rg.y & 0xffff; ey = rg.y >> 16;
         has = sx < ex && sy < ey;
         if (has) {
-            c = tri_clamp(a.triAABB[2 * t], a.triAABB[2 * t + 1], s);
+            c = tri_clamp(mn, mx, s);
             has = c.ok;
-            o = a.triOff[t];
         }
     }
+    __syncthreads();
     const bool big = has && (ex - sx) * (ey - sy) > FD_BIG_AREA;
     if (has && !big) {
-        const unsigned long long cap = a.pairCap;
+        unsigned long long q = o;
         const uint32_t tag = (uint32_t)threadIdx.x << 16;
         for (int j = sy; j < ey; ++j)
             for (int i = sx; i < ex; ++i) {
                 const int bp = j << log2G | i;
                 if (bin_test(bin_at(a, staged, binQ, binW, bp), c.bx, c.by, c.bz, c.ex, c.ey)) {
-                    if (o < cap) a.pairKT[o] = tag | (uint32_t)bp;
-                    ++o;
+                    if (q < cap) a.pairKT[q] = tag | (uint32_t)bp;
+                    ++q;
                 }
             }
     }
     tri_write_big(a, log2G, staged, binQ, binW, big, sx, sy, ex, ey, c, o);
-}
-
-// Stable counting scatter of one triangle block's pairs (the reference's
-// stable sort_by_key by bin, Step4_RasterizeTriangleToBin.inl:206-223), by
-// the block's 16 waves at once: wave w owns triangles t0 + 64w .. t0 + 64w + 63 and with them a contiguous slice
-// of the triangle-major pair list.  A triangle has at most one pair per bin,
-// so a wave holds at most 64 pairs of a bin and the 16 per-wave counts of a
-// bin fit 16-bit halves of LDS words (two waves per word, counted with 32-bit
-// LDS adds).  After a barrier every bin's counts become exclusive prefixes
-// over the waves (at most 1024, still 16 bits), and each wave ranks its
-// slice from base + prefix: lanes with equal bins are matched by ballots
-// over the key bits and ranked with mbcnt, the last lane of a group advances
-// the running offset.  Result: bin-major, ascending triangle id within a
-// bin.  LDS: FD_SCATTER_WIDE_LDS bytes per bin (bins <= 4096: grids up to
-// 64 x 64).
-__device__ __forceinline__ int wide_half(int w, int k, int nb) { return (((w >> 1) * nb + k) << 1) | (w & 1); }
-
-__device__ __forceinline__ void tri_scatter_wide_body(const FdArgs& a, const int blk) {
-    extern __shared__ uint32_t wlds[];
-    const FdState* s = a.st;
-    if (s->status != FD_EXIT_OK) return;
-    const int nb = s->nb;
-    uint32_t* cnt32 = wlds;                                   // 8 * nb words
-    uint16_t* cnt16 = (uint16_t*)wlds;
-    uint32_t* base = wlds + 8 * nb;                           // nb block offsets
-    int kbits = 1;
-    while ((1 << kbits) < nb) ++kbits;
-    for (int k = threadIdx.x; k < 8 * nb; k += FD_TRB) cnt32[k] = 0u;
-    for (int k = threadIdx.x; k < nb; k += FD_TRB) base[k] = a.histT[(size_t)k * a.nblkT + blk];
-    __syncthreads();
+    __syncthreads();   // the block's pairs are written
+    // this wave's slice of them: whole steps of 64 pairs
     const int w = (int)(threadIdx.x >> 6);
-    const int ta = blk * FD_TRB + w * 64;
-    const int tb = min(ta + 64, a.ntris);
-    unsigned long long p0 = 0, p1 = 0;
-    if (ta < a.ntris) {
-        p0 = a.triOff[ta];
-        p1 = tb < a.ntris ? (unsigned long long)a.triOff[tb] : s->pairs;
-    }
-    const unsigned long long cap = a.pairCap;
-    const unsigned long long e = p1 < cap ? p1 : cap;
+    const unsigned long long b0 = a.triOff[t0];
+    const unsigned long long b1 = t0 + FD_TRB < a.ntris ? (unsigned long long)a.triOff[t0 + FD_TRB] : s->pairs;
+    const unsigned long long e1 = b1 < cap ? b1 : cap;
+    const unsigned steps = b0 < e1 ? (unsigned)((e1 - b0 + 63) >> 6) : 0u;
+    const unsigned per = (steps + 15) >> 4;
+    const unsigned long long p0 = b0 + 64ull * per * w;
+    const unsigned long long p1 = p0 + 64ull * per < e1 ? p0 + 64ull * per : e1;
     const uint32_t inc = (w & 1) ? 0x10000u : 1u;
-    for (unsigned long long p = p0 + lane_id(); p < e; p += 64)
+#pragma unroll 4
+    for (unsigned long long p = p0 + lane_id(); p < p1; p += 64)
         atomicAdd(&cnt32[(w >> 1) * nb + (int)(a.pairKT[p] & 0xffffu)], inc);
     __syncthreads();
     for (int k = threadIdx.x; k < nb; k += FD_TRB) {
         uint32_t run = 0;
-        for (int v = 0; v < 16; ++v) {
-            const int h = wide_half(v, k, nb);
-            const uint32_t c = cnt16[h];
-            cnt16[h] = (uint16_t)run;
-            run += c;
+#pragma unroll
+        for (int v = 0; v < 8; ++v) {
+            const uint32_t x = cnt32[v * nb + k], lo = x & 0xffffu;
+            cnt32[v * nb + k] = run | (run + lo) << 16;
+            run += lo + (x >> 16);
         }
     }
     __syncthreads();
-    const int t0 = blk * FD_TRB;
+    const int kbits = 2 * log2G;
+    uint32_t nxt = p0 + lane_id() < p1 ? a.pairKT[p0 + lane_id()] : 0u;
     for (unsigned long long c0 = p0; c0 < p1; c0 += 64) {
         const unsigned long long p = c0 + lane_id();
-        const bool act = p < e;
-        const uint32_t v = act ? a.pairKT[p] : 0u;
+        const bool act = p < p1;
+        const uint32_t v = nxt;
+        if (p + 64 < p1) nxt = a.pairKT[p + 64];
         const int key = (int)(v & 0xffffu);
         uint64_t eq = __ballot(act);
         for (int b = 0; b < kbits; ++b) {
@@ -947,73 +974,123 @@ __device__ __forceinline__ void tri_scatter_wide_body(const FdArgs& a, const int
             const int rank = mbcnt(eq);
             const int gcount = __popcll(eq);
             const int h = wide_half(w, key, nb);
-            const uint32_t b0 = cnt16[h];
-            const unsigned long long dst = (unsigned long long)base[key] + b0 + (unsigned)rank;
-            if (rank == gcount - 1) cnt16[h] = (uint16_t)(b0 + gcount);
+            const uint32_t r0 = cnt16[h];
+            const unsigned long long dst = (unsigned long long)base[key] + r0 + (unsigned)rank;
+            if (rank == gcount - 1) cnt16[h] = (uint16_t)(r0 + gcount);
             if (dst < cap) a.sortedTri[dst] = t0 + (int)(v >> 16);
         }
     }
 }
 
 // --------------------------------------------------------------------------
-// Per-bin tables (FindStart_kernel, binRaster.inl:5-59) and the occlusion
-// work list: one work item per 64 sorted receivers of a bin (the invalid key
+// Exit bookkeeping once the counts are known, the per-bin tables
+// (FindStart_kernel, binRaster.inl:5-59) and the occlusion work list, by one
+// block, from the bins' totals.
+//
+// Exits: setupTriangleVertex returns 1 when no triangle reached the light plane
+// (Step0_triangleSetup.inl:224-225); FDLaunch skips the rest when there are no
+// pairs (FD/api.cpp:522).
+//
+// Work list: one work item per 64 sorted receivers of a bin (the invalid key
 // included, so every receiver's output is written exactly once).  Work items
 // are issued bin by bin, longest triangle list first (by power-of-two class
 // of the list length; the invalid key, with no list, last), so that the
 // launch does not end on a few long-running waves.  The order only schedules
 // work: every receiver's result is the same in any order.
 // --------------------------------------------------------------------------
-__device__ __forceinline__ void tables_body(const FdArgs& a, const int blk) {
-    __shared__ int wsum[16];
+__device__ __forceinline__ void tables_body(const FdArgs& a, uint32_t (&sh)[16]) {
     __shared__ int classCount[33], classBase[33];
+    __shared__ int waveCount[16][33];
+    __shared__ uint16_t binAt[4097];     // per rank: the bin and its number of work items
+    __shared__ uint32_t itemsAt[4097];
     FdState* s = a.st;
-    const int status = s->status;
+    const int nb = s->nb;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    // totals; the counting blocks' results (no count pass without triangles)
+    unsigned long long pairs = 0;
+    uint32_t nv = 0, np = 0, no = 0, rxIn = 0;
+    for (int k = threadIdx.x; k < nb; k += SCAN_BLOCK) {
+        pairs += a.triTot[k];
+        rxIn += a.rxTot[k];
+    }
+    if (a.ntris > 0)
+        for (int i = threadIdx.x; i < a.nblkT; i += SCAN_BLOCK) {
+            const uint32_t x = a.part[i];
+            nv += x & 0x7ffu;
+            np += (x >> 11) & 0x3ffu;
+            no += x >> 21;
+        }
+    nv = block_sum(nv, sh);
+    np = block_sum(np, sh);
+    no = block_sum(no, sh);
+    rxIn = block_sum(rxIn, sh);
+    // each bin has at most 2^31 pairs and a thread at most four bins
+    const unsigned long long lo = block_sum((uint32_t)(pairs & 0xffffu), sh), mi = block_sum((uint32_t)(pairs >> 16) & 0xffffu, sh),
+                             hi = block_sum((uint32_t)(pairs >> 32), sh);
+    pairs = lo + (mi << 16) + (hi << 32);
+    int status = FD_EXIT_OK;
+    if (nv == 0) status = FD_EXIT_NO_VALID_TRI;
+    else if (pairs == 0) status = FD_EXIT_NO_PAIRS;
+    else if (pairs > a.pairCap || pairs >= 0x7fffffffull) status = FD_EXIT_CAPACITY;
+    if (threadIdx.x == 0) {
+        s->pairs = pairs;
+        s->rxTotal = (unsigned long long)rxIn + a.rxTot[nb];
+        s->validTris = (int)nv;
+        // walk order of the bins' lists.  A triangle soup (neighbouring
+        // triangles mostly apart): largest projected triangles first, big
+        // occluders fill receivers early.  A connected mesh: the mesh order,
+        // largest first except those covering 1/512 of the light plane or more,
+        // which come last in list order (mostly triangles near the light; first,
+        // they would scatter each object's triangles, which a receiver often
+        // needs together) -- unless the lists are long (many objects overlap:
+        // a receiver fills from whichever object comes first in the list, so
+        // the list order, which keeps every object together, wins)
+        const bool mesh = 2 * no >= np;
+        const bool dense = pairs > (unsigned long long)FD_MESH_MAX_LIST16 * 256ull;
+        s->triOrder = a.triOrder != FD_TRI_ORDER_AUTO ? a.triOrder
+                      : !mesh ? FD_TRI_ORDER_AREA : dense ? FD_TRI_ORDER_LIST : FD_TRI_ORDER_MESH;
+        // valid receivers: binned (keys < nb) plus keys out of range
+        s->validSamples = (int)rxIn + s->keyOutOfRange;
+        if (status == FD_EXIT_CAPACITY) s->capacityHit = 1;
+        s->status = status;
+    }
     // the receivers' start / end table exists once they are sorted: FDLaunch
     // binds the samples before it pairs the triangles (FD/api.cpp:505-522),
     // so a frame that ends without pairs (or over the pair arena) has it too
-    if (status != FD_EXIT_OK && status != FD_EXIT_NO_PAIRS && status != FD_EXIT_CAPACITY) return;
-    const int nb = s->nb;
-    if (status != FD_EXIT_OK) {
-        for (int k = threadIdx.x; k <= nb; k += blockDim.x) {
-            a.rxStart[k] = (int)a.histR[(size_t)k * a.nblkR];
-            a.rxEnd[k] = (k < nb) ? (int)a.histR[(size_t)(k + 1) * a.nblkR] : a.WH;
-        }
-        return;
-    }
+    if (status == FD_EXIT_NO_VALID_TRI) return;
     if (threadIdx.x < 33) classCount[threadIdx.x] = 0;
     __syncthreads();
-    // bin tables and the cost class of every bin (0 = longest lists)
-    for (int k = threadIdx.x; k <= nb; k += blockDim.x) {
-        const int rs = (int)a.histR[(size_t)k * a.nblkR];
-        const int re = (k < nb) ? (int)a.histR[(size_t)(k + 1) * a.nblkR] : a.WH;
-        a.rxStart[k] = rs;
-        a.rxEnd[k] = re;
-        int cls = 32;
-        if (k < nb) {
-            const int ts = (int)a.histT[(size_t)k * a.nblkT];
-            const int te = (k < nb - 1) ? (int)a.histT[(size_t)(k + 1) * a.nblkT] : (int)s->pairs;
-            a.triStart[k] = ts;
-            a.triEnd[k] = te;
-            cls = __clz(te - ts + 1);   // 31 - floor(log2(len + 1)): longer lists, smaller class
-        }
-        atomicAdd(&classCount[cls], 1);
-    }
+    // the cost class of every bin (0 = longest lists): 31 - floor(log2(len + 1))
+    for (int k = threadIdx.x; k <= nb; k += SCAN_BLOCK)
+        atomicAdd(&classCount[k < nb ? __clz((int)a.triTot[k] + 1) : 32], 1);
     __syncthreads();
-    if (threadIdx.x == 0) {
-        int c = 0;
-        for (int i = 0; i < 33; ++i) { classBase[i] = c; c += classCount[i]; }
+    if (w == 0) {
+        const int c = lane < 33 ? classCount[lane] : 0;
+        const int x = (int)wave_incl_scan((uint32_t)c);
+        if (lane < 33) classBase[lane] = x - c;
     }
     __syncthreads();
     // stable within a class (ascending bin index, so that neighbouring bins,
     // which share triangles, stay close in the issue order): ranks from wave
     // ballots, then a prefix over the waves of each 1024-bin slice
-    __shared__ int waveCount[16][33];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    for (int k0 = 0; k0 <= nb; k0 += 1024) {
+    uint32_t rxCarry = 0, triCarry = 0;
+    for (int k0 = 0; k0 <= nb; k0 += SCAN_BLOCK) {
         const int k = k0 + threadIdx.x;
         const bool in = k <= nb;
-        const int cls = !in ? 0 : (k < nb) ? __clz(a.triEnd[k] - a.triStart[k] + 1) : 32;
+        const uint32_t rx = in ? a.rxTot[k] : 0u, tr = k < nb ? a.triTot[k] : 0u;
+        uint32_t rxAll, trAll;
+        const uint32_t rs = rxCarry + block_excl_scan(rx, sh, rxAll), ts = triCarry + block_excl_scan(tr, sh, trAll);
+        rxCarry += rxAll;
+        triCarry += trAll;
+        if (in) {
+            a.rxStart[k] = (int)rs;
+            if (k == nb) a.rxStart[nb + 1] = a.WH;
+            if (status == FD_EXIT_OK) {
+                a.triStart[k] = (int)ts;   // triStart[nb]: the number of pairs
+            }
+        }
+        if (status != FD_EXIT_OK) continue;
+        const int cls = !in ? 0 : (k < nb) ? __clz((int)tr + 1) : 32;
         for (int i = lane; i < 33; i += 64) waveCount[w][i] = 0;
         int rankInWave = 0;
         for (uint64_t pending = __ballot(in); pending;) {
@@ -1027,6 +1104,7 @@ __device__ __forceinline__ void tables_body(const FdArgs& a, const int blk) {
         __syncthreads();
         if (threadIdx.x < 33) {   // per class: exclusive prefix over the waves, then advance the class base
             int run = classBase[threadIdx.x];
+#pragma unroll
             for (int j = 0; j < 16; ++j) {
                 const int c = waveCount[j][threadIdx.x];
                 waveCount[j][threadIdx.x] = run;
@@ -1035,37 +1113,55 @@ __device__ __forceinline__ void tables_body(const FdArgs& a, const int blk) {
             classBase[threadIdx.x] = run;
         }
         __syncthreads();
-        if (in) a.binAtRank[waveCount[w][cls] + rankInWave] = k;
+        if (in) {
+            const int r = waveCount[w][cls] + rankInWave;
+            binAt[r] = (uint16_t)k;
+            itemsAt[r] = ((k == nb ? (uint32_t)a.WH - rs : rx) + 63) >> 6;
+        }
         __syncthreads();
     }
+    if (status != FD_EXIT_OK) return;
     // work-item prefix in rank order
-    int carry = 0;
-    for (int k0 = 0; k0 <= nb; k0 += 1024) {
+    uint32_t carry = 0;
+    for (int k0 = 0; k0 <= nb; k0 += SCAN_BLOCK) {
         const int r = k0 + threadIdx.x;
-        int nch = 0;
-        if (r <= nb) {
-            const int k = a.binAtRank[r];
-            nch = (a.rxEnd[k] - a.rxStart[k] + 63) >> 6;
-        }
-        // block exclusive scan of nch
-        int x = nch;
-        const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
-        for (int o = 1; o < 64; o <<= 1) {
-            int y = __shfl_up(x, o, 64);
-            if (l >= o) x += y;
-        }
-        if (l == 63) wsum[w] = x;
-        __syncthreads();
-        int off = carry, all = 0;
-        for (int i = 0; i < 16; ++i) {
-            if (i < w) off += wsum[i];
-            all += wsum[i];
-        }
-        if (r <= nb) a.chunkStart[a.binAtRank[r]] = off + x - nch;
+        uint32_t all;
+        const uint32_t off = carry + block_excl_scan(r <= nb ? itemsAt[r] : 0u, sh, all);
+        if (r <= nb) a.chunkStart[binAt[r]] = (int)off;
         carry += all;
-        __syncthreads();
     }
-    if (threadIdx.x == 0) s->totalChunks = carry;
+    if (threadIdx.x == 0) s->totalChunks = (int)carry;
+}
+
+// All that follows from the counts in one launch: block 0 the exits and tables,
+// the others the scans of the receiver histogram, the pair histogram and the
+// triangles' pair counts.  Nothing here depends on the status that block 0 sets.
+__device__ __forceinline__ void scan_body(const FdArgs& a, int blk) {
+    __shared__ uint32_t sh[16];
+    const FdState* s = a.st;
+    if (!binned(s->status)) return;
+    if (blk == 0) {
+        tables_body(a, sh);
+        return;
+    }
+    --blk;
+    const int nb = 1 << (2 * a.gridLog2);
+    const int rr = fd_scan_rows(a.nblkR), nr = (nb + rr) / rr;   // rows per block; blocks of nb + 1 rows
+    if (blk < nr) {
+        scan_rows(a.histR, a.rxTot, blk * rr, min((blk + 1) * rr, nb + 1), a.nblkR, sh);
+        return;
+    }
+    blk -= nr;
+    const int rt = fd_scan_rows(a.nblkT), nt = (nb + rt - 1) / rt;
+    if (blk < nt) {
+        scan_rows(a.histT, a.triTot, blk * rt, min((blk + 1) * rt, nb), a.nblkT, sh);
+        return;
+    }
+    blk -= nt;
+    uint32_t pre = 0;
+    for (int i = threadIdx.x; i < blk * (SCAN_CHUNK / FD_TRB); i += SCAN_BLOCK) pre += a.part[a.nblkT + i];
+    const uint32_t base = block_sum(pre, sh);
+    scan_range(a.triOff, (long)blk * SCAN_CHUNK, min((long)(blk + 1) * SCAN_CHUNK, (long)a.ntris), base, sh);
 }
 
 // Area order of one bin's triangle list (frames whose walk order is
@@ -1161,62 +1257,6 @@ __device__ __forceinline__ void tri_order_body(const FdArgs& a, const int bin) {
         if (key < K) out[ts + waveCount[w][key] + rank] = tri;
         __syncthreads();
     }
-}
-
-// Exit bookkeeping after the scans (setupTriangleVertex returns 1 when no
-// triangle reached the light plane, Step0_triangleSetup.inl:224-225;
-// FDLaunch skips the rest when there are no pairs, FD/api.cpp:522).
-__device__ __forceinline__ void post_pairs_body(const FdArgs& a, const int blk) {
-    if (blk != 0) return;
-    FdState* s = a.st;
-    if (s->status != FD_EXIT_OK) return;
-    // valid triangles: the pair-count blocks' totals (no count pass without
-    // triangles)
-    __shared__ int wsum[3][FD_FIN_THREADS / 64];
-    int v = 0, np = 0, no = 0;
-    if (a.ntris > 0)
-        for (int i = threadIdx.x; i < a.nblkT; i += blockDim.x) {
-            v += (int)a.part[i];
-            np += (int)a.part[a.nblkT + i];
-            no += (int)a.part[2 * a.nblkT + i];
-        }
-    v = wave_sum_i32(v);
-    np = wave_sum_i32(np);
-    no = wave_sum_i32(no);
-    if ((threadIdx.x & 63) == 0) {
-        wsum[0][threadIdx.x >> 6] = v;
-        wsum[1][threadIdx.x >> 6] = np;
-        wsum[2][threadIdx.x >> 6] = no;
-    }
-    __syncthreads();
-    if (threadIdx.x != 0) return;
-    int nv = 0;
-    long pairsAdj = 0, overlaps = 0;
-    for (int j = 0; j < (int)(blockDim.x + 63) >> 6; ++j) {
-        nv += wsum[0][j];
-        pairsAdj += wsum[1][j];
-        overlaps += wsum[2][j];
-    }
-    s->validTris = nv;
-    // walk order of the bins' lists.  A triangle soup (neighbouring
-    // triangles mostly apart): largest projected triangles first, big
-    // occluders fill receivers early.  A connected mesh: the mesh order,
-    // largest first except those covering 1/512 of the light plane or more,
-    // which come last in list order (mostly triangles near the light; first,
-    // they would scatter each object's triangles, which a receiver often
-    // needs together) -- unless the lists are long (many objects overlap:
-    // a receiver fills from whichever object comes first in the list, so
-    // the list order, which keeps every object together, wins)
-    const bool mesh = 2 * overlaps >= pairsAdj;
-    const bool dense = s->pairs > (unsigned long long)FD_MESH_MAX_LIST16 * 256ull;
-    s->triOrder = a.triOrder != FD_TRI_ORDER_AUTO ? a.triOrder
-                  : !mesh ? FD_TRI_ORDER_AREA : dense ? FD_TRI_ORDER_LIST : FD_TRI_ORDER_MESH;
-    // valid receivers: binned (keys < nb, the scanned histogram at key nb)
-    // plus keys out of range
-    s->validSamples = (int)a.histR[(size_t)s->nb * a.nblkR] + s->keyOutOfRange;
-    if (s->validTris == 0) s->status = FD_EXIT_NO_VALID_TRI;
-    else if (s->pairs == 0) s->status = FD_EXIT_NO_PAIRS;
-    else if (s->pairs > a.pairCap || s->pairs >= 0x7fffffffull) { s->status = FD_EXIT_CAPACITY; s->capacityHit = 1; }
 }
 
 // --------------------------------------------------------------------------
@@ -2645,17 +2685,13 @@ __device__ __forceinline__ void occlude_finish_body(const FdArgs& a, const int c
 // belongs to instance i with map[i] <= b < map[i+1] (host-built prefix), and
 // the instance's FdArgs is read from the device-resident instance table.
 // ==========================================================================
-__global__ void k_init(FdArgs a) { init_body(a, blockIdx.x); }
-__global__ void k_init_bins(FdArgs a) { init_bins_body(a, blockIdx.x); }
 __global__ __launch_bounds__(RED_BLOCK) void k_reduce(FdArgs a) { reduce_body(a, blockIdx.x); }
 __global__ __launch_bounds__(FD_FIN_THREADS) void k_finalize(FdArgs a) { finalize_body(a, blockIdx.x); }
-__global__ __launch_bounds__(256) void k_rx_key(FdArgs a) { rx_key_body(a, blockIdx.x); }
-__global__ __launch_bounds__(64) void k_rx_scatter(FdArgs a) { rx_scatter_body(a, blockIdx.x); }
+__global__ __launch_bounds__(FD_RXB) void k_rx_key(FdArgs a) { rx_key_body(a, blockIdx.x); }
+__global__ __launch_bounds__(FD_RXB) void k_rx_scatter(FdArgs a) { rx_scatter_body(a, blockIdx.x); }
 __global__ __launch_bounds__(FD_TRB) void k_tri_count(FdArgs a) { tri_count_body(a, blockIdx.x); }
-__global__ __launch_bounds__(FD_TRB) void k_tri_write(FdArgs a) { tri_write_body(a, blockIdx.x); }
-__global__ __launch_bounds__(FD_TRB) void k_tri_scatter_wide(FdArgs a) { tri_scatter_wide_body(a, blockIdx.x); }
-__global__ __launch_bounds__(1024) void k_tables(FdArgs a) { tables_body(a, blockIdx.x); }
-__global__ __launch_bounds__(FD_FIN_THREADS) void k_post_pairs(FdArgs a) { post_pairs_body(a, blockIdx.x); }
+__global__ __launch_bounds__(SCAN_BLOCK) void k_scan(FdArgs a) { scan_body(a, blockIdx.x); }
+__global__ __launch_bounds__(FD_TRB) void k_tri_scatter(FdArgs a) { tri_scatter_body(a, blockIdx.x); }
 __global__ __launch_bounds__(FD_ORDER_THREADS) void k_tri_order(FdArgs a) { tri_order_body(a, blockIdx.x); }
 // Workgroups are dealt to the 8 XCDs round-robin (block b runs on XCD
 // b % 8).  Work items of one bin share that bin's triangle list, so the
@@ -2691,16 +2727,6 @@ template <typename T>
 __global__ __launch_bounds__(64) void k_occlude_cta(FdArgs a) {
     occlude_body<T, false, true>(a, xcd_block(blockIdx.x, gridDim.x));
 }
-__global__ __launch_bounds__(SCAN_BLOCK) void k_scan_reduce(const uint32_t* __restrict__ d, long n,
-                                                            uint64_t* __restrict__ part, const int* status) {
-    scan_reduce_body(d, n, part, status, blockIdx.x);
-}
-__global__ __launch_bounds__(SCAN_BLOCK) void k_scan_apply(uint32_t* __restrict__ d, long n,
-                                                           const uint64_t* __restrict__ part,
-                                                           unsigned long long* total, const int* status) {
-    scan_apply_body(d, n, part, total, status, blockIdx.x);
-}
-
 // instance of block b: map[i] <= b < map[i+1] (wave-uniform binary search)
 __device__ __forceinline__ int inst_of(const int* __restrict__ map, int n, int b) {
     int lo = 0, hi = n;
@@ -2719,17 +2745,13 @@ __device__ __forceinline__ int inst_of(const int* __restrict__ map, int n, int b
         const FdArgs a = inst[i];                                                              \
         BODY(a, b - map[i]);                                                                   \
     }
-FD_BATCHED(kb_init, 64, init_body)
-FD_BATCHED(kb_init_bins, 256, init_bins_body)
 FD_BATCHED(kb_reduce, RED_BLOCK, reduce_body)
 FD_BATCHED(kb_finalize, FD_FIN_THREADS, finalize_body)
-FD_BATCHED(kb_rx_key, 256, rx_key_body)
-FD_BATCHED(kb_rx_scatter, 64, rx_scatter_body)
+FD_BATCHED(kb_rx_key, FD_RXB, rx_key_body)
 FD_BATCHED(kb_tri_count, FD_TRB, tri_count_body)
-FD_BATCHED(kb_tri_write, FD_TRB, tri_write_body)
-FD_BATCHED(kb_tri_scatter_wide, FD_TRB, tri_scatter_wide_body)
-FD_BATCHED(kb_tables, 1024, tables_body)
-FD_BATCHED(kb_post_pairs, FD_FIN_THREADS, post_pairs_body)
+FD_BATCHED(kb_scan, SCAN_BLOCK, scan_body)
+FD_BATCHED(kb_rx_scatter, FD_RXB, rx_scatter_body)
+FD_BATCHED(kb_tri_scatter, FD_TRB, tri_scatter_body)
 FD_BATCHED(kb_tri_order, FD_ORDER_THREADS, tri_order_body)
 #undef FD_BATCHED
 
@@ -2751,31 +2773,6 @@ __global__ __launch_bounds__(64) void kb_occlude_finish(const FdArgs* __restrict
     const int b = blockIdx.x;
     const int i = inst_of(map, n, b);
     occlude_finish_body(inst[i], b - map[i]);
-}
-
-// which = 0: receiver key histogram, 1: pair histogram
-// The three scanned arrays of a frame: 0 receiver histogram, 1 pair
-// histogram, 2 per-triangle pair counts (the last two have the same total).
-__device__ __forceinline__ uint32_t* scan_data(const FdArgs& a, int which) {
-    return which == 0 ? a.histR : which == 1 ? a.histT : a.triOff;
-}
-__device__ __forceinline__ long scan_len(const FdArgs& a, int which) {
-    return which == 0 ? a.nR : which == 1 ? a.nT : (long)a.ntris;
-}
-__global__ __launch_bounds__(SCAN_BLOCK) void kb_scan_reduce(const FdArgs* __restrict__ inst, const int* __restrict__ map,
-                                                             int n, int which) {
-    const int b = blockIdx.x;
-    const int i = inst_of(map, n, b);
-    const FdArgs a = inst[i];
-    scan_reduce_body(scan_data(a, which), scan_len(a, which), a.scanPart, &a.st->status, b - map[i]);
-}
-__global__ __launch_bounds__(SCAN_BLOCK) void kb_scan_apply(const FdArgs* __restrict__ inst, const int* __restrict__ map,
-                                                            int n, int which) {
-    const int b = blockIdx.x;
-    const int i = inst_of(map, n, b);
-    const FdArgs a = inst[i];
-    scan_apply_body(scan_data(a, which), scan_len(a, which), a.scanPart, which ? &a.st->pairs : &a.st->rxTotal,
-                    &a.st->status, b - map[i]);
 }
 
 // Verification of the row-mask primitive on given (D, B) pairs (n = R - 1),
@@ -2887,17 +2884,12 @@ namespace fdk {
 
 static inline int cdiv(long a, long b) { return (int)((a + b - 1) / b); }
 
-static hipError_t scan_u32(uint32_t* d, long n, uint64_t* part, unsigned long long* total, const int* status,
-                           hipStream_t st) {
-    const int nch = cdiv(n, SCAN_CHUNK);
-    k_scan_reduce<<<nch, SCAN_BLOCK, 0, st>>>(d, n, part, status);
-    k_scan_apply<<<nch, SCAN_BLOCK, 0, st>>>(d, n, part, total, status);
-    return hipGetLastError();
-}
-
-long scan_partials_needed(long n) { return cdiv(n, SCAN_CHUNK); }
 int reduce_blocks(long n) { return cdiv(n, RED_BLOCK * RED_ITEMS); }
-int scan_chunks(long n) { return cdiv(n, SCAN_CHUNK); }
+int scan_blocks(const FdArgs& a) {
+    const int nb = 1 << (2 * a.gridLog2);
+    return 1 + cdiv(nb + 1, fd_scan_rows(a.nblkR)) +
+           (a.ntris > 0 ? cdiv(nb, fd_scan_rows(a.nblkT)) + cdiv(a.ntris, SCAN_CHUNK) : 0);
+}
 int zero_blocks(const FdArgs& a) { return (int)cdiv((long)a.WH * a.L.res * a.L.wpr, ZERO_WORDS); }
 
 hipError_t enqueue_batch(const FdBatchPlan& p, hipStream_t st) {
@@ -2905,28 +2897,17 @@ hipError_t enqueue_batch(const FdBatchPlan& p, hipStream_t st) {
     auto L = [&](int m) { return dim3((unsigned)(p.total[m] > 0 ? p.total[m] : 1)); };
     const int nb = p.maxNb;
     const size_t binLds = nb <= FD_LDS_BINS ? (size_t)nb * FD_BIN_LDS_BYTES : 0;
-    kb_init<<<L(FD_MAP_ONE), 64, 0, st>>>(p.inst, p.map[FD_MAP_ONE], n);
-    kb_init_bins<<<L(FD_MAP_BINS), 256, 0, st>>>(p.inst, p.map[FD_MAP_BINS], n);
     kb_reduce<<<L(FD_MAP_RED), RED_BLOCK, 0, st>>>(p.inst, p.map[FD_MAP_RED], n);
     kb_finalize<<<L(FD_MAP_ONE), FD_FIN_THREADS, 0, st>>>(p.inst, p.map[FD_MAP_ONE], n);
-    kb_rx_key<<<L(FD_MAP_RX), 256, (nb + 1) * sizeof(uint32_t) + binLds, st>>>(p.inst, p.map[FD_MAP_RX], n);
-    kb_scan_reduce<<<L(FD_MAP_SCANR), SCAN_BLOCK, 0, st>>>(p.inst, p.map[FD_MAP_SCANR], n, 0);
-    kb_scan_apply<<<L(FD_MAP_SCANR), SCAN_BLOCK, 0, st>>>(p.inst, p.map[FD_MAP_SCANR], n, 0);
-    kb_rx_scatter<<<L(FD_MAP_RX), 64, (nb + 1) * sizeof(int), st>>>(p.inst, p.map[FD_MAP_RX], n);
-    if (p.anyTris) {
+    kb_rx_key<<<L(FD_MAP_RX), FD_RXB, (nb + 1) * sizeof(uint32_t) + binLds, st>>>(p.inst, p.map[FD_MAP_RX], n);
+    if (p.anyTris)
         kb_tri_count<<<L(FD_MAP_TRI), FD_TRB, nb * sizeof(uint32_t) + binLds, st>>>(p.inst, p.map[FD_MAP_TRI], n);
-        kb_scan_reduce<<<L(FD_MAP_SCANT), SCAN_BLOCK, 0, st>>>(p.inst, p.map[FD_MAP_SCANT], n, 1);
-        kb_scan_apply<<<L(FD_MAP_SCANT), SCAN_BLOCK, 0, st>>>(p.inst, p.map[FD_MAP_SCANT], n, 1);
-    }
-    kb_post_pairs<<<L(FD_MAP_ONE), FD_FIN_THREADS, 0, st>>>(p.inst, p.map[FD_MAP_ONE], n);
+    kb_scan<<<L(FD_MAP_SCAN), SCAN_BLOCK, 0, st>>>(p.inst, p.map[FD_MAP_SCAN], n);
+    kb_rx_scatter<<<L(FD_MAP_RX), FD_RXB, (size_t)(nb + 1) * FD_SCATTER_RX_LDS, st>>>(p.inst, p.map[FD_MAP_RX], n);
     if (p.anyTris) {
-        kb_scan_reduce<<<L(FD_MAP_SCANO), SCAN_BLOCK, 0, st>>>(p.inst, p.map[FD_MAP_SCANO], n, 2);
-        kb_scan_apply<<<L(FD_MAP_SCANO), SCAN_BLOCK, 0, st>>>(p.inst, p.map[FD_MAP_SCANO], n, 2);
-        kb_tri_write<<<L(FD_MAP_TRI), FD_TRB, binLds, st>>>(p.inst, p.map[FD_MAP_TRI], n);
-        kb_tri_scatter_wide<<<L(FD_MAP_TRI), FD_TRB, (size_t)nb * FD_SCATTER_WIDE_LDS, st>>>(p.inst, p.map[FD_MAP_TRI], n);
+        kb_tri_scatter<<<L(FD_MAP_TRI), FD_TRB, (size_t)nb * FD_SCATTER_WIDE_LDS + binLds, st>>>(p.inst, p.map[FD_MAP_TRI], n);
+        kb_tri_order<<<L(FD_MAP_NB), FD_ORDER_THREADS, 0, st>>>(p.inst, p.map[FD_MAP_NB], n);
     }
-    kb_tables<<<L(FD_MAP_ONE), 1024, 0, st>>>(p.inst, p.map[FD_MAP_ONE], n);
-    if (p.anyTris) kb_tri_order<<<L(FD_MAP_NB), FD_ORDER_THREADS, 0, st>>>(p.inst, p.map[FD_MAP_NB], n);
     if (p.total[FD_MAP_ZERO] > 0) kb_zero_masks<<<L(FD_MAP_ZERO), 256, 0, st>>>(p.occ[0], p.map[FD_MAP_ZERO], n);
     for (int c = 0; c < FD_OCC_CLASSES; ++c) {   // fd_occ_class: 32 / 64-bit rows x 2 / 4 / 8 waves
         if (p.nocc[c] == 0) continue;
@@ -2990,36 +2971,20 @@ hipError_t debug_rect(const FdArgs& a, float* out8, hipStream_t st) {
 hipError_t enqueue_frame(const FdArgs& a, hipStream_t st, hipEvent_t* ev) {
     const int nb = 1 << (2 * a.gridLog2);
     const size_t binLds = a.binLds ? (size_t)nb * FD_BIN_LDS_BYTES : 0;
-    const int nbR = a.nbR, nbV = a.nbV;
-    FdState* s = a.st;
     auto mark = [&](int i) { if (ev) (void)hipEventRecord(ev[i], st); };
     mark(0);
-    k_init<<<1, 64, 0, st>>>(a);
-    k_init_bins<<<cdiv(nb, 256), 256, 0, st>>>(a);
-    k_reduce<<<nbR + nbV, RED_BLOCK, 0, st>>>(a);
+    k_reduce<<<a.nbR + a.nbV, RED_BLOCK, 0, st>>>(a);
     k_finalize<<<1, FD_FIN_THREADS, 0, st>>>(a);
     mark(1);
-    // receivers: key + bin statistics, stable counting sort
-    k_rx_key<<<a.nblkR, 256, (nb + 1) * sizeof(uint32_t) + binLds, st>>>(a);
-    hipError_t e = scan_u32(a.histR, a.nR, a.scanPart, &s->rxTotal, &s->status, st);
-    if (e != hipSuccess) return e;
-    k_rx_scatter<<<a.nblkR, 64, (nb + 1) * sizeof(int), st>>>(a);
+    // receivers: key + bin statistics; triangles: setup + pair count (needs the statistics)
+    k_rx_key<<<a.nblkR, FD_RXB, (nb + 1) * sizeof(uint32_t) + binLds, st>>>(a);
     mark(2);
-    // triangles: setup + pair count, stable pair scatter
-    if (a.ntris > 0) {
-        k_tri_count<<<a.nblkT, FD_TRB, nb * sizeof(uint32_t) + binLds, st>>>(a);
-        e = scan_u32(a.histT, a.nT, a.scanPart, &s->pairs, &s->status, st);
-        if (e != hipSuccess) return e;
-        k_post_pairs<<<1, FD_FIN_THREADS, 0, st>>>(a);
-        e = scan_u32(a.triOff, a.ntris, a.scanPart, &s->pairs, &s->status, st);
-        if (e != hipSuccess) return e;
-        k_tri_write<<<a.nblkT, FD_TRB, binLds, st>>>(a);
-        k_tri_scatter_wide<<<a.nblkT, FD_TRB, (size_t)nb * FD_SCATTER_WIDE_LDS, st>>>(a);
-    } else {
-        k_post_pairs<<<1, FD_FIN_THREADS, 0, st>>>(a);
-    }
+    if (a.ntris > 0) k_tri_count<<<a.nblkT, FD_TRB, nb * sizeof(uint32_t) + binLds, st>>>(a);
+    // offsets and tables, then both stable scatters
+    k_scan<<<scan_blocks(a), SCAN_BLOCK, 0, st>>>(a);
+    k_rx_scatter<<<a.nblkR, FD_RXB, (size_t)(nb + 1) * FD_SCATTER_RX_LDS, st>>>(a);
+    if (a.ntris > 0) k_tri_scatter<<<a.nblkT, FD_TRB, (size_t)nb * FD_SCATTER_WIDE_LDS + binLds, st>>>(a);
     mark(3);
-    k_tables<<<1, 1024, 0, st>>>(a);
     if (a.ntris > 0) k_tri_order<<<nb + 1, FD_ORDER_THREADS, 0, st>>>(a);
     mark(4);
     // occlusion (or the early-exit fill); split lists zero the masks first

@@ -361,7 +361,8 @@ int fd_autotune(fd_ctx* ctx, const fd_instance* inst, fd_tune_entry* cands, int 
 
 /* No counterpart (the reference times the whole FDLaunch with cudaEvents,
  * FD/api.cpp:405-409,574-581): per-stage device times of the next frames
- * (light plane, receiver binning, triangle pairing, tables, occlusion) and,
+ * (light plane, receiver keys, triangle pairing with the offsets and both
+ * scatters, list order and work items, occlusion) and,
  * with count_ops, FD_PROFILE_COUNTERS occlusion work counters (a slower
  * counting variant of the occlusion kernel runs):
  *   [0] candidate (receiver, triangle) tests   [1] cull passes
