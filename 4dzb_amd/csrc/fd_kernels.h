@@ -120,23 +120,29 @@ struct FdArgs {
 inline int fd_default_waves(int wpr, long items) { return (wpr == 2 || items <= FD_WAVES8_ITEMS) ? 8 : 4; }
 inline bool fd_valid_waves(int w) { return w == 2 || w == 4 || w == 8; }
 
-// LDS of an occlusion work item: its light rows ([row][receiver], a stride of
+// LDS of an occlusion work item: the tile windows of each wave's block (64
+// float4; nw = 0: none), its light rows ([row][receiver], a stride of
 // 65 words, so that lanes that walk one receiver's rows, or one lane per row,
 // use different banks: the write-out and the prefilter's occupancy pass), the
 // full-row masks (one row word per receiver) and the receivers' rectangles and
 // depths (5 floats).
 #define FD_ROW_STRIDE 65
-inline size_t fd_occ_lds(int wpr, int res) {
-    return (size_t)wpr * res * FD_ROW_STRIDE * sizeof(uint32_t) + 64 * (wpr * sizeof(uint32_t) + 5 * sizeof(float));
+#define FD_TILE_WORDS 256
+inline size_t fd_occ_lds(int wpr, int res, int nw) {
+    return (size_t)nw * FD_TILE_WORDS * sizeof(uint32_t) + (size_t)wpr * res * FD_ROW_STRIDE * sizeof(uint32_t) + 64 * (wpr * sizeof(uint32_t) + 5 * sizeof(float));
 }
 // Column strips of the light grid in the occlusion prefilter
 #define FD_OCC_STRIPS 8
-// The prefilter's test against the receivers' rows: for lists of FD_PRUNE_LIST
-// entries per wave and more, on a block's remaining triangles (FD_PRUNE_LEFT or
-// more) before every FD_PRUNE_STEPS pairs.
-#define FD_PRUNE_LIST 64
-#define FD_PRUNE_LEFT 4
-#define FD_PRUNE_STEPS 24
+// The prefilter's windows for all receivers at once: for lists of FD_TILE_LIST
+// entries per wave and more, on blocks of FD_TILE_MIN triangles and more that
+// pass the boxes.  Its test against the receivers' rows: on a block's remaining
+// triangles (FD_PRUNE_LEFT or more) before every FD_PRUNE_STEPS pairs.
+// Measured flat around these (16 / 4 / 4 and 32 / 6 / 6: within 1%; rows tested
+// every 8 or 24 pairs: 1 to 3% slower on the soup or the meshes).
+#define FD_TILE_LIST 32
+#define FD_TILE_MIN 6
+#define FD_PRUNE_LEFT 6
+#define FD_PRUNE_STEPS 16
 
 // Occlusion classes of a batched launch: 32-bit / 64-bit rows x 2 / 4 / 8
 // waves per work item (one launch each).
