@@ -254,7 +254,8 @@ int frame_args(fd_ctx* c, FdArgs& a) {
               c->masks, c->pairCap);
     a.occVariant = c->occVariant;
     a.triOrder = c->triOrder;
-    a.occWaves = c->occWaves ? c->occWaves : fd_default_waves(a.L.wpr, a.chunkSlots);
+    a.wavesReq = c->occWaves;
+    a.occWaves = a.wavesReq ? a.wavesReq : fd_default_waves(a.L.wpr, a.chunkSlots);
     apply_split(a, c->listSplit);
     return FD_OK;
 }
@@ -718,9 +719,14 @@ size_t build_plan(const std::vector<FdArgs>& args, bool anyTris, char* devBase, 
     P.maxNb = 0;
     P.anyTris = anyTris;
     std::vector<int> occIdx[FD_OCC_CLASSES];
+    long slots = 0;   // work items of the batch
+    for (int i = 0; i < n; ++i) slots += args[i].chunkSlots;
+    auto waves = [&](const FdArgs& q) {
+        return !q.wavesReq && q.L.wpr == 1 && slots > FD_WAVES8_ITEMS ? 4 : q.occWaves;
+    };
     for (int i = 0; i < n; ++i) {
         P.maxNb = std::max(P.maxNb, 1 << (2 * args[i].gridLog2));
-        occIdx[fd_occ_class(args[i].L.wpr, args[i].occWaves)].push_back(i);
+        occIdx[fd_occ_class(args[i].L.wpr, waves(args[i]))].push_back(i);
     }
     for (int cl = 0; cl < FD_OCC_CLASSES; ++cl) {  // largest work first: shorter tail
         auto cost = [&](int i) { return (double)args[i].WH * args[i].L.res * args[i].L.res; };
@@ -734,10 +740,9 @@ size_t build_plan(const std::vector<FdArgs>& args, bool anyTris, char* devBase, 
     FdArgs* hArgs = (FdArgs*)image.data();
     // a batch that fills the GPU with whole-list work items does not split the
     // triangle lists of its small instances (the merge would only cost)
-    long slots = 0;
-    for (int i = 0; i < n; ++i) slots += args[i].chunkSlots;
     for (int i = 0; i < n; ++i) {
         hArgs[i] = args[i];
+        hArgs[i].occWaves = waves(args[i]);
         if (slots > FD_SPLIT_ITEMS && !hArgs[i].splitReq) hArgs[i].segs = 1;
         hArgs[i].binLds = P.maxNb <= FD_LDS_BINS;   // the batched launch sizes LDS for the largest grid
     }
@@ -840,8 +845,9 @@ extern "C" int fd_batch_create(fd_ctx* c, const fd_instance* in, int n, fd_batch
         fill_args(b->args[i], md, (const float4*)q.d_position4, (const float4*)q.d_normal4, q.width, q.height, L,
                   c->eps, c->cull, g, tl, q.d_shadow, q.d_masks, cap);
         b->args[i].triOrder = q.tri_order ? q.tri_order : c->triOrder;
-        b->args[i].occWaves = q.occ_waves ? q.occ_waves : c->occWaves ? c->occWaves
-                                                     : fd_default_waves(L.wpr, b->args[i].chunkSlots);
+        const int waves = q.occ_waves ? q.occ_waves : c->occWaves;
+        b->args[i].wavesReq = waves;
+        b->args[i].occWaves = waves ? waves : fd_default_waves(L.wpr, b->args[i].chunkSlots);
         apply_split(b->args[i], q.list_split ? q.list_split : c->listSplit);   // after occWaves
         FdArgs probe = b->args[i];
         off[i + 1] = off[i] + ((layout(probe, nullptr, false) + 255) & ~(size_t)255);

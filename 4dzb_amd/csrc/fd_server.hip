@@ -319,6 +319,7 @@ long long fd_server_submit(fd_server* s, const fd_request* r) {
     if ((1 << g) != bins || g < 3 || g > 6 || (1 << tl) != tw || tl < 3 || tl > 6) return FD_ERR_ARG;
     fill_args(q.args, md, (const float4*)r->d_position4, (const float4*)r->d_normal4, r->width,
               r->height, L, s->cfg.eps, s->cfg.backface_cull, g, tl, r->d_shadow, r->d_masks, s->cfg.max_pairs);
+    q.args.wavesReq = waves;
     q.args.occWaves = waves ? waves : fd_default_waves(L.wpr, q.args.chunkSlots);
     q.args.triOrder = order;
     apply_split(q.args, split);
