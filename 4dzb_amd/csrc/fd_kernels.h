@@ -104,12 +104,24 @@ struct FdArgs {
 // up to FD_LIST_SPLIT_MAX (fd4d.h).  The automatic rule: a frame of at
 // most FD_SPLIT_ITEMS work items and fewer than FD_SPLIT_MIN_WAVES waves in
 // all (work items x waves per item) splits its lists into about
-// FD_SPLIT_WAVES waves, at most 16 stretches; larger frames keep whole
-// lists.  Each stretch merges its masks into the output by atomic OR, which
-// only pays where the GPU would otherwise idle.
+// FD_SPLIT_WAVES waves, at most fd_split_max stretches; larger frames keep
+// whole lists.  Each stretch merges its masks into the output by atomic OR,
+// which only pays where the GPU would otherwise idle.
 #define FD_SPLIT_ITEMS 2048
 #define FD_SPLIT_MIN_WAVES 6144
 #define FD_SPLIT_WAVES 49152
+// Most stretches by the triangles per bin (the host does not know the lists):
+// a stretch of a few entries costs more than it takes off, and a long whole
+// list lets the prefilter leave out what meets full rows.  Measured on evenly
+// spread triangles and on spheres, 32 x 32 to 160 x 160 receivers and 8 x 8 to
+// 64 x 64 samples, us with 16 stretches / with this rule: 8 per bin 108 / 91 and
+// 81 / 77, 78 per bin 176 / 161 and 129 / 123, 781 per bin 515 / 374 (spheres;
+// at 390 per bin whole lists are still up to 10% slower there).  Whole lists
+// need work items enough: with 64 of them 117 / 181.
+inline int fd_split_max(long ntris, int nb, long items) {
+    const long e = ntris / nb;
+    return e < 16 ? 4 : e < 512 ? 8 : items >= 256 ? 1 : 16;
+}
 
 // Waves per occlusion work item (per-sample kernel) unless a frame asks for
 // another count (2, 4 or 8): the waves share a work item's receivers, LDS
