@@ -48,13 +48,18 @@ def work_items(w, h, bins=16):
 
 
 def default_waves(res, w=None, h=None, bins=16):
-    """The library's default waves per occlusion work item for a res x res
-    light grid (fd_set_occlusion_waves): 8 for 64-bit rows and for frames of
-    up to WAVES8_ITEMS work items, else 4 (a frame of unknown size counts
-    as large)."""
+    """Waves per occlusion work item of a class without a tuned count: 8 for
+    64-bit rows and for frames of up to WAVES8_ITEMS work items, else 4 (a
+    frame of unknown size counts as large).  Left to choose, the library takes
+    4 for large frames of 64-bit rows too (library_waves)."""
     if res > 32:
         return 8
     return 8 if w is not None and h is not None and work_items(w, h, bins) <= WAVES8_ITEMS else 4
+
+
+def library_waves(w, h, bins=16):
+    """The library's own default (fd_set_occlusion_waves 0) for a plain frame."""
+    return 8 if work_items(w, h, bins) <= WAVES8_ITEMS else 4
 
 
 def default_layout(res, w=None, h=None):

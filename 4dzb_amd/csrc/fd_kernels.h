@@ -125,15 +125,16 @@ inline int fd_split_max(long ntris, int nb, long items) {
 
 // Waves per occlusion work item (per-sample kernel) unless a frame asks for
 // another count (2, 4 or 8): the waves share a work item's receivers, LDS
-// rows and full-row masks and split its triangle list.  8 for 64-bit rows
-// (32 KiB of rows per work item: LDS holds 4 work items per CU, so 8 waves
-// each fill it) and for frames of up to FD_WAVES8_ITEMS work items (too few
-// to fill the GPU with 4 waves each); 4 for larger frames of 32-bit rows.
+// rows and full-row masks and split its triangle list.  8 for frames of up to
+// FD_WAVES8_ITEMS work items (too few to fill the GPU with 4 waves each); 4
+// for larger frames: 64-bit rows leave LDS for 4 work items of 4 waves per CU,
+// or 3 of 8, and the fewer waves share a work item the less they walk past
+// one another (us, 8 / 4 waves: heightfield-1k 4021 / 3580 with 48 x 48
+// samples, 4780 / 4590 with 64 x 64; 1080p soup 2863 / 2529 and 3204 / 3114).
 #define FD_WAVES8_ITEMS 8192
-// In a batch of more work items in all, its small frames of 32-bit rows take 4
-// as well: the others fill the GPU beside them (24 frames, 300 k work items:
-// 29.3 -> 28.5 ms).
-inline int fd_default_waves(int wpr, long items) { return (wpr == 2 || items <= FD_WAVES8_ITEMS) ? 8 : 4; }
+// In a batch of more work items in all, its small frames take 4 as well: the
+// others fill the GPU beside them (24 frames, 300 k work items: 29.3 -> 28.5 ms).
+inline int fd_default_waves(long items) { return items <= FD_WAVES8_ITEMS ? 8 : 4; }
 inline bool fd_valid_waves(int w) { return w == 2 || w == 4 || w == 8; }
 
 // LDS of an occlusion work item: the tile windows of each wave's block (64

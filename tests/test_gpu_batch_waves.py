@@ -1,6 +1,6 @@
 """Waves per work item in a batch that fills the GPU (more than 8192 work
-items): small frames of 32-bit rows by the batch's rule, 64-bit rows and frames
-that ask for a count as alone, every instance bit for bit as alone (MI355X
+items): small frames by the batch's rule, frames
+that ask for a count by theirs, every instance bit for bit as alone (MI355X
 only)."""
 import numpy as np
 import pytest
