@@ -758,10 +758,10 @@ size_t build_plan(const std::vector<FdArgs>& args, bool anyTris, char* devBase, 
     for (int cl = 0, base = n; cl < FD_OCC_CLASSES; base += P.nocc[cl++]) P.occ[cl] = dArgs + base;
     for (int m = 0; m < FD_NMAPS; ++m) {
         const bool occCls = m >= FD_MAP_OCC0 && m < FD_MAP_OCC0 + FD_OCC_CLASSES;
-        const bool occ = occCls || m == FD_MAP_ZERO || m == FD_MAP_FIN;
+        const bool occ = occCls || m == FD_MAP_FIN;
         const std::vector<int>* order = occCls ? &occIdx[m - FD_MAP_OCC0] : nullptr;
-        std::vector<int> all;   // zero / finish maps: every instance, in occlusion-table order
-        if (m == FD_MAP_ZERO || m == FD_MAP_FIN) {
+        std::vector<int> all;   // finish map: every instance, in occlusion-table order
+        if (m == FD_MAP_FIN) {
             for (int cl = 0; cl < FD_OCC_CLASSES; ++cl) all.insert(all.end(), occIdx[cl].begin(), occIdx[cl].end());
             order = &all;
         }
@@ -772,7 +772,6 @@ size_t build_plan(const std::vector<FdArgs>& args, bool anyTris, char* devBase, 
         mp[0] = 0;
         for (int q = 0; q < cnt; ++q) {
             const FdArgs& a = hArgs[occ ? (*order)[q] : q];
-            const int nb = 1 << (2 * a.gridLog2);
             int blocks = 1;
             switch (m) {
                 case FD_MAP_ONE: blocks = 1; break;
@@ -780,8 +779,7 @@ size_t build_plan(const std::vector<FdArgs>& args, bool anyTris, char* devBase, 
                 case FD_MAP_RX: blocks = a.nblkR; break;
                 case FD_MAP_TRI: blocks = a.nblkT; break;
                 case FD_MAP_SCAN: blocks = fdk::scan_blocks(a); break;
-                case FD_MAP_NB: blocks = nb + 1; break;
-                case FD_MAP_ZERO: blocks = a.segs > 1 ? fdk::zero_blocks(a) : 0; break;
+                case FD_MAP_NB: blocks = fdk::order_blocks(a); break;
                 case FD_MAP_FIN: blocks = a.segs > 1 ? a.chunkSlots : 0; break;
                 default: blocks = a.chunkSlots * a.segs; break;
             }

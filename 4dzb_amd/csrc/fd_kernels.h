@@ -189,8 +189,8 @@ __host__ __device__ inline int fd_scan_rows(int nblk) { return nblk >= 4096 ? 1 
 
 // Block maps of a batched launch (prefix sums over instances, n + 1 each).
 enum FdMap { FD_MAP_ONE, FD_MAP_RED, FD_MAP_RX, FD_MAP_TRI, FD_MAP_SCAN, FD_MAP_OCC0, FD_MAP_OCC1, FD_MAP_OCC2,
-             FD_MAP_OCC3, FD_MAP_OCC4, FD_MAP_OCC5, FD_MAP_ZERO, FD_MAP_FIN, FD_MAP_NB, FD_NMAPS };
-static_assert(FD_MAP_OCC0 + FD_OCC_CLASSES == FD_MAP_ZERO, "one block map per occlusion class");
+             FD_MAP_OCC3, FD_MAP_OCC4, FD_MAP_OCC5, FD_MAP_FIN, FD_MAP_NB, FD_NMAPS };
+static_assert(FD_MAP_OCC0 + FD_OCC_CLASSES == FD_MAP_FIN, "one block map per occlusion class");
 static_assert(FD_TRI_CLASSES < (1 << FD_WALK_KEY_BITS), "area classes and the no-entry value fit the key bits");
 
 struct FdBatchPlan {
@@ -209,5 +209,5 @@ hipError_t enqueue_frame(const FdArgs& a, hipStream_t st, hipEvent_t* stageEvent
 hipError_t enqueue_batch(const FdBatchPlan& p, hipStream_t st);
 int reduce_blocks(long n);
 int scan_blocks(const FdArgs& a);
-int zero_blocks(const FdArgs& a);   // blocks of the mask-zeroing pass
+int order_blocks(const FdArgs& a);   // one per bin and the invalid key, and the mask-zeroing ones
 }  // namespace fdk

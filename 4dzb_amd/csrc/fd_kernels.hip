@@ -1164,6 +1164,17 @@ __device__ __forceinline__ void scan_body(const FdArgs& a, int blk) {
     scan_range(a.triOff, (long)blk * SCAN_CHUNK, min((long)(blk + 1) * SCAN_CHUNK, (long)a.ntris), base, sh);
 }
 
+// Split lists only: zeroes the mask output before the occlusion merges into
+// it (by blocks of k_tri_order, which waits for nothing of theirs; no memset, so
+// that the sequence stays graph-capturable).  A launch of its own took 2.9 us.
+constexpr int ZERO_WORDS = 4096;   // words per block
+__device__ __forceinline__ void zero_masks_body(const FdArgs& a, const int blk) {
+    const size_t n = (size_t)a.WH * a.L.res * a.L.wpr;
+    const size_t base = (size_t)blk * ZERO_WORDS;
+    for (int k = threadIdx.x; k < ZERO_WORDS; k += blockDim.x)
+        if (base + k < n) a.masks[base + k] = 0u;
+}
+
 // Area order of one bin's triangle list (frames whose walk order is
 // FD_TRI_ORDER_AREA): a stable counting sort of triStart..triEnd of the
 // reference-order list by the triangles' area classes, into the same range
@@ -1178,8 +1189,13 @@ __device__ __forceinline__ void tri_order_body(const FdArgs& a, const int bin) {
     __shared__ int waveCount[NWV][K];
     __shared__ int keyBase[K];
     __shared__ uint8_t keyCache[FD_ORDER_CACHE];
+    const int nb = 1 << (2 * a.gridLog2);
+    if (bin > nb) {
+        zero_masks_body(a, bin - nb - 1);
+        return;
+    }
     const FdState* s = a.st;
-    if (s->status != FD_EXIT_OK || bin > s->nb) return;
+    if (s->status != FD_EXIT_OK) return;
     const int ts = bin < s->nb ? a.triStart[bin] : 0, te = bin < s->nb ? a.triEnd[bin] : 0;
     {   // the bin's work items: one record each, so that the occlusion finds its own in one load
         const int c0 = a.chunkStart[bin], rs = a.rxStart[bin], re = a.rxEnd[bin];
@@ -2793,16 +2809,6 @@ __device__ __forceinline__ void occlude_body(const FdArgs& a, const int blkIn) {
     else or_masks(a, lds, id, n, R, wpr, wv, NW);
 }
 
-// Split lists only: zeroes the mask output before the occlusion merges into
-// it (a fill kernel, so that the sequence stays graph-capturable).
-constexpr int ZERO_WORDS = 4096;   // words per block
-__device__ __forceinline__ void zero_masks_body(const FdArgs& a, const int blk) {
-    const size_t n = (size_t)a.WH * a.L.res * a.L.wpr;
-    const size_t base = (size_t)blk * ZERO_WORDS;
-    for (int k = threadIdx.x; k < ZERO_WORDS; k += blockDim.x)
-        if (base + k < n) a.masks[base + k] = 0u;
-}
-
 // Split lists: shadow value of every receiver of a
 // real bin from its merged mask (popcount / samples, :226-231).
 __device__ __forceinline__ void occlude_finish_body(const FdArgs& a, const int c) {
@@ -2863,7 +2869,6 @@ __device__ __forceinline__ int xcd_block(int b, int n) {
     return b - j + (j & 7) * G + (j >> 3);
 }
 
-__global__ __launch_bounds__(256) void k_zero_masks(FdArgs a) { zero_masks_body(a, blockIdx.x); }
 __global__ __launch_bounds__(64) void k_occlude_finish(FdArgs a) { occlude_finish_body(a, blockIdx.x); }
 
 // NW waves per occlusion work item (they share its receivers and LDS rows):
@@ -2917,12 +2922,6 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(6))) vo
     const int i = inst_of(map, n, b);
     const FdArgs a = inst[i];
     occlude_body<T, false, false, NW>(a, b - map[i]);
-}
-__global__ __launch_bounds__(256) void kb_zero_masks(const FdArgs* __restrict__ inst, const int* __restrict__ map,
-                                                     int n) {
-    const int b = blockIdx.x;
-    const int i = inst_of(map, n, b);
-    zero_masks_body(inst[i], b - map[i]);
 }
 __global__ __launch_bounds__(64) void kb_occlude_finish(const FdArgs* __restrict__ inst, const int* __restrict__ map,
                                                         int n) {
@@ -3046,7 +3045,9 @@ int scan_blocks(const FdArgs& a) {
     return 1 + cdiv(nb + 1, fd_scan_rows(a.nblkR)) +
            (a.ntris > 0 ? cdiv(nb, fd_scan_rows(a.nblkT)) + cdiv(a.ntris, SCAN_CHUNK) : 0);
 }
-int zero_blocks(const FdArgs& a) { return (int)cdiv((long)a.WH * a.L.res * a.L.wpr, ZERO_WORDS); }
+int order_blocks(const FdArgs& a) {
+    return (1 << (2 * a.gridLog2)) + 1 + (a.segs > 1 ? cdiv((long)a.WH * a.L.res * a.L.wpr, ZERO_WORDS) : 0);
+}
 
 hipError_t enqueue_batch(const FdBatchPlan& p, hipStream_t st) {
     const int n = p.n;
@@ -3064,7 +3065,6 @@ hipError_t enqueue_batch(const FdBatchPlan& p, hipStream_t st) {
         kb_tri_scatter<<<L(FD_MAP_TRI), FD_TRB, (size_t)nb * FD_SCATTER_WIDE_LDS + binLds, st>>>(p.inst, p.map[FD_MAP_TRI], n);
         kb_tri_order<<<L(FD_MAP_NB), FD_ORDER_THREADS, 0, st>>>(p.inst, p.map[FD_MAP_NB], n);
     }
-    if (p.total[FD_MAP_ZERO] > 0) kb_zero_masks<<<L(FD_MAP_ZERO), 256, 0, st>>>(p.occ[0], p.map[FD_MAP_ZERO], n);
     for (int c = 0; c < FD_OCC_CLASSES; ++c) {   // fd_occ_class: 32 / 64-bit rows x 2 / 4 / 8 waves
         if (p.nocc[c] == 0) continue;
         const int wpr = c / 3 + 1, nw = 2 << (c % 3);
@@ -3141,12 +3141,11 @@ hipError_t enqueue_frame(const FdArgs& a, hipStream_t st, hipEvent_t* ev) {
     k_rx_scatter<<<a.nblkR, FD_RXB, (size_t)(nb + 1) * FD_SCATTER_RX_LDS, st>>>(a);
     if (a.ntris > 0) k_tri_scatter<<<a.nblkT, FD_TRB, (size_t)nb * FD_SCATTER_WIDE_LDS + binLds, st>>>(a);
     mark(3);
-    if (a.ntris > 0) k_tri_order<<<nb + 1, FD_ORDER_THREADS, 0, st>>>(a);
+    if (a.ntris > 0) k_tri_order<<<order_blocks(a), FD_ORDER_THREADS, 0, st>>>(a);
     mark(4);
-    // occlusion (or the early-exit fill); split lists zero the masks first
-    // and count them after the merge
+    // occlusion (or the early-exit fill); split lists count the masks after the
+    // merge
     const int wpr = a.L.wpr;
-    if (a.segs > 1) k_zero_masks<<<zero_blocks(a), 256, 0, st>>>(a);
     if (a.occVariant == FD_OCC_BIN_QUEUE) {
         const int chunks = a.chunkSlots * a.segs;
         const size_t shmCta = (size_t)wpr * a.L.res * FD_ROW_STRIDE * sizeof(uint32_t) + 64 * sizeof(uint64_t);   // + full-row flags
