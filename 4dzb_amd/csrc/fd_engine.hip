@@ -187,7 +187,7 @@ void apply_split(FdArgs& a, int req) {
     } else {
         const long waves = (long)a.chunkSlots * std::max(a.occWaves, 1);
         a.segs = (a.chunkSlots <= FD_SPLIT_ITEMS && waves < FD_SPLIT_MIN_WAVES)
-                     ? (int)std::max(1L, std::min((long)fd_split_max(a.ntris, 1 << (2 * a.gridLog2), a.chunkSlots),
+                     ? (int)std::max(1L, std::min((long)fd_split_max(a.ntris, 1 << (2 * a.gridLog2)),
                                                   FD_SPLIT_WAVES / waves)) : 1;
     }
 }

@@ -111,16 +111,20 @@ struct FdArgs {
 #define FD_SPLIT_MIN_WAVES 6144
 #define FD_SPLIT_WAVES 49152
 // Most stretches by the triangles per bin (the host does not know the lists):
-// a stretch of a few entries costs more than it takes off, and a long whole
-// list lets the prefilter leave out what meets full rows.  Measured on evenly
-// spread triangles and on spheres, 32 x 32 to 160 x 160 receivers and 8 x 8 to
-// 64 x 64 samples, us with 16 stretches / with this rule: 8 per bin 108 / 91 and
-// 81 / 77, 78 per bin 176 / 161 and 129 / 123, 781 per bin 515 / 374 (spheres;
-// at 390 per bin whole lists are still up to 10% slower there).  Whole lists
-// need work items enough: with 64 of them 117 / 181.
-inline int fd_split_max(long ntris, int nb, long items) {
+// a stretch of a few entries costs more than it takes off.  Measured at 8 x 8
+// and 16 x 16 bins, 16 x 16 to 200 x 200 receivers, 16 x 16 and 64 x 64
+// samples, on soups, spheres and boxes: frames as at 64 x 64 receivers, us with
+// 16 stretches / with this rule: 7 triangles per bin 115 / 96, 78 per bin 153 /
+// 139 (evenly spread triangles); at 234 per bin and more single frames would
+// take 16 rather than 8 (soup 196 / 226, 20 finely tessellated spheres 189 /
+// 221).  Whole lists are up to 2.1 times faster where many objects overlap
+// (968 k triangles of 500 spheres, 176 x 176 receivers: 2278 / 1068) and up to
+// 4.3 times slower elsewhere (1 M triangles of 20 spheres 1674 / 7271, soup 1717
+// / 2817), which the counts at hand do not tell apart: never chosen for dense
+// lists.
+inline int fd_split_max(long ntris, int nb) {
     const long e = ntris / nb;
-    return e < 16 ? 4 : e < 512 ? 8 : items >= 256 ? 1 : 16;
+    return e < 16 ? 4 : e < 512 ? 8 : 16;
 }
 
 // Waves per occlusion work item (per-sample kernel) unless a frame asks for

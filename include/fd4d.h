@@ -184,12 +184,11 @@ int fd_set_occlusion_waves(fd_ctx* ctx, int waves);
  * does not depend on the order, so the bits are the same for every S.
  * 0 (the default): a frame of up to 2048 work items with fewer than 6144
  * waves in all (work items x waves per item) splits into about 49152
- * waves (at most 4, 8 or 16 stretches, by the triangles per bin; whole lists
- * from 512 triangles per bin on); larger ones do not (nor does a batch whose
- * instances total more than 2048 work items); 1..64: that many
- * stretches.  The
- * batched form takes it per instance (fd_instance.list_split), the serving
- * form per class (fd_tune_entry.list_split). */
+ * waves (at most 4 stretches below 16 triangles per bin, 8 below 512, else
+ * 16); larger ones do not (nor does a batch whose instances total more than
+ * 2048 work items); 1..64: that many stretches.  The batched form takes it
+ * per instance (fd_instance.list_split), the serving form per class
+ * (fd_tune_entry.list_split). */
 #define FD_LIST_SPLIT_MAX 64
 int fd_set_list_split(fd_ctx* ctx, int segs);
 
