@@ -39,6 +39,7 @@ SPLITS = (1, 2, 4, 8, 16)       # stretches per bin list tried against the autom
 
 
 WAVES8_ITEMS = 8192   # FD_WAVES8_ITEMS: frames of up to this many work items default to 8 waves
+WAVES8_ITEMS64 = 28672   # FD_WAVES8_ITEMS64: the same with light grids above 32x32
 
 
 def work_items(w, h, bins=16):
@@ -57,9 +58,9 @@ def default_waves(res, w=None, h=None, bins=16):
     return 8 if w is not None and h is not None and work_items(w, h, bins) <= WAVES8_ITEMS else 4
 
 
-def library_waves(w, h, bins=16):
+def library_waves(res, w, h, bins=16):
     """The library's own default (fd_set_occlusion_waves 0) for a plain frame."""
-    return 8 if work_items(w, h, bins) <= WAVES8_ITEMS else 4
+    return 8 if work_items(w, h, bins) <= (WAVES8_ITEMS64 if res > 32 else WAVES8_ITEMS) else 4
 
 
 def default_layout(res, w=None, h=None):

@@ -130,15 +130,21 @@ inline int fd_split_max(long ntris, int nb) {
 // Waves per occlusion work item (per-sample kernel) unless a frame asks for
 // another count (2, 4 or 8): the waves share a work item's receivers, LDS
 // rows and full-row masks and split its triangle list.  8 for frames of up to
-// FD_WAVES8_ITEMS work items (too few to fill the GPU with 4 waves each); 4
-// for larger frames: 64-bit rows leave LDS for 4 work items of 4 waves per CU,
-// or 3 of 8, and the fewer waves share a work item the less they walk past
-// one another (us, 8 / 4 waves: heightfield-1k 4021 / 3580 with 48 x 48
-// samples, 4780 / 4590 with 64 x 64; 1080p soup 2863 / 2529 and 3204 / 3114).
+// FD_WAVES8_ITEMS work items (too few to fill the GPU with 4 waves each), 4 for
+// larger frames: the fewer waves share a work item the less they walk past one
+// another.  64-bit rows leave LDS for 4 work items of 4 waves per CU at 64 x 64
+// samples, or 3 of 8, so that 4 waves also leave fewer of them in flight, and
+// what outlasts the frame, its longest lists, is walked by fewer: 4 only from
+// FD_WAVES8_ITEMS64 items on (us, 8 / 4 waves, 48 x 48 samples: 1 M triangle
+// soup 817 / 1252 at 720 x 720 receivers, 940 / 1106 at 960 x 960, 1697 / 1406
+// at 1920 x 1080; 300 k triangles of 20 spheres 2071 / 3275, 2865 / 3214 and
+// 5421 / 5236; 500 spheres of 200 k triangles 1254 / 1147 and 3933 / 3315; with
+// 64 x 64 samples at 1920 x 1080 1938 / 1784, 5790 / 6118 and 4641 / 4270).
 #define FD_WAVES8_ITEMS 8192
+#define FD_WAVES8_ITEMS64 28672
 // In a batch of more work items in all, its small frames take 4 as well: the
 // others fill the GPU beside them (24 frames, 300 k work items: 29.3 -> 28.5 ms).
-inline int fd_default_waves(long items) { return items <= FD_WAVES8_ITEMS ? 8 : 4; }
+inline int fd_default_waves(int wpr, long items) { return items <= (wpr == 2 ? FD_WAVES8_ITEMS64 : FD_WAVES8_ITEMS) ? 8 : 4; }
 inline bool fd_valid_waves(int w) { return w == 2 || w == 4 || w == 8; }
 
 // LDS of an occlusion work item: the tile windows of each wave's block (64

@@ -194,8 +194,8 @@ def plain_leg(pkg, frame, workload, steps, warmup, quick):
                config=dict(workload=workload, receivers=f"{W}x{H}", light_samples=f"{R}x{R}",
                            triangles=frame.scene.ntris, bins=f"{1 << frame.grid_log2}x{1 << frame.grid_log2}",
                            tile_width=frame.tile_width,
-                           occ_waves=frame.occ_waves or pkg.autotune.library_waves(frame.rx.w, frame.rx.h,
-                                                                                   1 << frame.grid_log2),
+                           occ_waves=frame.occ_waves or pkg.autotune.library_waves(frame.light.res_w, frame.rx.w,
+                                                                                   frame.rx.h, 1 << frame.grid_log2),
                            path="plain per-frame"),
                p50_ms=round(pctl(g["lat"], 50), 3), p99_ms=round(pctl(g["lat"], 99), 3),
                stage_ms=dict(zip(["light_plane", "receiver_binning", "triangle_pairing", "tables", "occlusion"],
@@ -791,7 +791,8 @@ def main():
     ap.add_argument("--bins", type=int, default=0, help="bins per light-plane side (default: the workload's, 16)")
     ap.add_argument("--tile", type=int, default=0, help="receiver tile width (default 8)")
     ap.add_argument("--waves", type=int, default=0, choices=[0, 2, 4, 8],
-                    help="waves per occlusion work item (default: 8 for frames of up to 8192 work items, else 4)")
+                    help="waves per occlusion work item (default: 8 for frames of up to 8192 work items, 28672 above 32x32 light "
+                         "samples, else 4)")
     ap.add_argument("--leg", choices=["batched", "served", "target", "app_pipeline", "shard_tile"], default=None,
                     help="run only this leg and print its JSON (for profiler runs)")
     args = ap.parse_args()
