@@ -723,7 +723,7 @@ size_t build_plan(const std::vector<FdArgs>& args, bool anyTris, char* devBase, 
     long slots = 0;   // work items of the batch
     for (int i = 0; i < n; ++i) slots += args[i].chunkSlots;
     auto waves = [&](const FdArgs& q) {
-        return !q.wavesReq && slots > FD_WAVES8_ITEMS ? 4 : q.occWaves;
+        return !q.wavesReq && q.L.wpr == 1 && slots > FD_BATCH_WAVES4_ITEMS ? 4 : q.occWaves;
     };
     for (int i = 0; i < n; ++i) {
         P.maxNb = std::max(P.maxNb, 1 << (2 * args[i].gridLog2));

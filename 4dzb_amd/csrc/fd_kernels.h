@@ -13,7 +13,7 @@
 // where a receiver fills from whichever object comes first in the list)
 #define FD_MESH_MAX_LIST16 7168
 #define FD_WALK_KEY_BITS 5     // bits of an area class or of the no-entry value FD_TRI_CLASSES
-#define FD_ORDER_CACHE 32768   // list entries whose walk keys the area-order pass keeps in LDS
+#define FD_ORDER_CACHE 28672   // list entries whose walk keys the area-order pass keeps in LDS
 #define FD_ORDER_THREADS 1024  // threads per bin in the area-order pass
 
 // One occlusion work item: receivers s0 .. s0 + n - 1 of the sorted order and
@@ -142,8 +142,15 @@ inline int fd_split_max(long ntris, int nb) {
 // 64 x 64 samples at 1920 x 1080 1938 / 1784, 5790 / 6118 and 4641 / 4270).
 #define FD_WAVES8_ITEMS 8192
 #define FD_WAVES8_ITEMS64 28672
-// In a batch of more work items in all, its small frames take 4 as well: the
-// others fill the GPU beside them (24 frames, 300 k work items: 29.3 -> 28.5 ms).
+// In a batch of more than FD_BATCH_WAVES4_ITEMS work items in all, its small
+// frames of 32-bit rows take 4 as well: the others fill the GPU beside them (us, 8
+// / 4 waves: 24 frames of 300 k work items 29306 / 28560; 24 of 256 x 256
+// receivers, 31 k items, 16 x 16 samples: spheres of 200 k triangles 12% less,
+// soup of 300 k 5%).  Below, their longest lists outlast the batch (two frames of
+// 512 x 512 receivers, 9 k items: soup of 300 k triangles 608 / 800, 300 k
+// triangles of 20 spheres 3009 / 4038; six, 26 k: 8396 / 9181), and 64-bit rows
+// lose there and at 31 k items (0 to 12% with 64 x 64 samples).
+#define FD_BATCH_WAVES4_ITEMS 28672
 inline int fd_default_waves(int wpr, long items) { return items <= (wpr == 2 ? FD_WAVES8_ITEMS64 : FD_WAVES8_ITEMS) ? 8 : 4; }
 inline bool fd_valid_waves(int w) { return w == 2 || w == 4 || w == 8; }
 

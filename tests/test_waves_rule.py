@@ -14,6 +14,23 @@ extern "C" int waves(int w, int h, int res, int grid_log2) {
     fdh::fill_args(a, md, nullptr, nullptr, w, h, FdLight{}, 0.0f, 0, grid_log2, 3, nullptr, nullptr, 1);
     return fd_default_waves(res > 32 ? 2 : 1, a.chunkSlots);
 }
+// instances per occlusion class (32 / 64-bit rows x 2 / 4 / 8 waves) of a batch of n frames
+extern "C" void batch(int n, int w, int h, int res, int asked, int* classes) {
+    std::vector<FdArgs> args(n);
+    const fdh::Model md{nullptr, 4, 3, nullptr, 1};
+    FdLight L{};
+    L.res = res;
+    L.wpr = res > 32 ? 2 : 1;
+    for (FdArgs& a : args) {
+        fdh::fill_args(a, md, nullptr, nullptr, w, h, L, 0.0f, 0, 4, 3, nullptr, nullptr, 1);
+        a.wavesReq = asked;
+        a.occWaves = asked ? asked : fd_default_waves(L.wpr, a.chunkSlots);
+    }
+    std::vector<char> image;
+    FdBatchPlan P;
+    fdh::build_plan(args, true, nullptr, image, P);
+    for (int c = 0; c < FD_OCC_CLASSES; ++c) classes[c] = P.nocc[c];
+}
 """
 
 
@@ -42,3 +59,20 @@ def test_frames(shim, w, h, narrow, wide):
         want = wide if res > 32 else narrow
         assert shim.waves(w, h, res, 4) == want
         assert at.library_waves(res, w, h) == want
+
+
+@pytest.mark.parametrize("n,w,h,res,asked,waves", [
+    (2, 512, 512, 8, 0, 8), (16, 256, 256, 32, 0, 8),      # 8706 and 20496 work items: too few to fill the GPU with 4
+    (6, 512, 512, 16, 0, 8), (25, 256, 256, 16, 0, 8),     # 26118, 32025
+    (26, 256, 256, 16, 0, 4), (8, 512, 512, 32, 0, 4),     # 33306, 34824
+    (26, 256, 256, 64, 0, 8), (300, 256, 256, 33, 0, 8),   # 64-bit rows: by the frame
+    (2, 1920, 1080, 64, 0, 4), (2, 720, 720, 16, 0, 4), (26, 256, 256, 16, 2, 2), (26, 256, 256, 16, 8, 8)])
+def test_batches(shim, n, w, h, res, asked, waves):
+    """Small frames of 32-bit rows take 4 waves in batches that fill the GPU
+    with that (soup of 300 k triangles, two 512 x 512 frames with 8 x 8
+    samples: 800 us with 4, 608 with 8); an asked count stays."""
+    got = (ctypes.c_int * 6)()
+    shim.batch(n, w, h, res, asked, got)
+    want = [0] * 6
+    want[(3 if res > 32 else 0) + {2: 0, 4: 1, 8: 2}[waves]] = n
+    assert list(got) == want
