@@ -13,7 +13,7 @@
 // where a receiver fills from whichever object comes first in the list)
 #define FD_MESH_MAX_LIST16 7168
 #define FD_WALK_KEY_BITS 5     // bits of an area class or of the no-entry value FD_TRI_CLASSES
-#define FD_ORDER_CACHE 28672   // list entries whose walk keys the area-order pass keeps in LDS
+#define FD_ORDER_CACHE 32768   // list entries whose walk keys the area-order pass keeps in LDS
 #define FD_ORDER_THREADS 1024  // threads per bin in the area-order pass
 
 // One occlusion work item: receivers s0 .. s0 + n - 1 of the sorted order and
