@@ -266,13 +266,26 @@ H3 hnormalize(H3 a) {
     return {a.x * k, a.y * k, a.z * k};
 }
 
-// A table goes by value if it is small and the stream does not capture (a
-// captured call copies the table from the caller's memory at every replay).
+// Memory that HIP knows (page-locked, managed, device): an upload reads it in
+// stream order, when earlier work of the stream may have filled it.
+bool known_to_hip(const void* p) {
+    if (!p) return false;
+    const hipError_t before = hipPeekAtLastError();
+    hipPointerAttribute_t at{};
+    const bool known = hipPointerGetAttributes(&at, p) == hipSuccess && at.type != hipMemoryTypeUnregistered;
+    if (before == hipSuccess) (void)hipGetLastError();   // ordinary memory: an error here
+    return known;
+}
+
+// Tables go by value if they are small, the stream does not capture (a captured
+// call copies them from the caller's memory at every replay) and they lie in
+// ordinary memory (else uploaded, which reads ordinary memory during the call).
 // The allocations, copies and frees of the uploads: fd_shade at 1920 x 1080 41.6
 // us with, 34.4 without; fd_gbuffer_boxes 57 and 38.
-bool by_value(hipStream_t st) {
+bool by_value(hipStream_t st, const void* table, const void* table2 = nullptr) {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(st, &cs) == hipSuccess) return cs == hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &cs) == hipSuccess)
+        return cs == hipStreamCaptureStatusNone && !known_to_hip(table) && !known_to_hip(table2);
     (void)hipGetLastError();
     return false;
 }
@@ -327,7 +340,7 @@ int fd_gbuffer_boxes(const fd_gbuffer_scene* sc, float* d_g0, float* d_g1, float
         a.tilesX = (sc->width + GB_TILE - 1) / GB_TILE;
         blocks = (long)a.tilesX * ((sc->height + GB_TILE - 1) / GB_TILE);
     }
-    if (sc->nbox <= GB_INLINE_BOXES && by_value(st)) {
+    if (sc->nbox <= GB_INLINE_BOXES && by_value(st, sc->nbox ? sc->boxes : nullptr, sc->materials)) {
         GbTables t;
         if (sc->nbox) std::memcpy(t.boxes, sc->boxes, (size_t)sc->nbox * 6 * sizeof(double));
         if (sc->materials) std::memcpy(t.mat, sc->materials, (size_t)(sc->nbox + 1) * sizeof(fd_material));
@@ -370,7 +383,7 @@ int fd_shade(const fd_shade_params* p, const float* d_shadow, const float* d_g0,
     a.g3 = (const float4*)d_g3;
     a.out = (float4*)d_rgba;
     const unsigned blocks = (unsigned)((a.n + 255) / 256);
-    if (p->nsamples <= SH_INLINE_SAMPLES && by_value(st)) {
+    if (p->nsamples <= SH_INLINE_SAMPLES && by_value(st, p->samples)) {
         ShTables t;
         std::memcpy(t.samples, p->samples, (size_t)p->nsamples * 3 * sizeof(float));
         hipLaunchKernelGGL(k_shade_inline, dim3(blocks), dim3(256), 0, st, a, t);
