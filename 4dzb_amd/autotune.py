@@ -48,23 +48,25 @@ def work_items(w, h, bins=16):
     return (w * h + 63) // 64 + bins * bins + 1
 
 
+def library_waves(res, w, h, bins=16):
+    """The library's own default waves per occlusion work item of a plain w x h
+    frame with a res x res light grid (fd_set_occlusion_waves 0)."""
+    return 8 if work_items(w, h, bins) <= (WAVES8_ITEMS64 if res > 32 else WAVES8_ITEMS) else 4
+
+
 def default_waves(res, w=None, h=None, bins=16):
-    """Waves per occlusion work item of a class without a tuned count: 8 for
-    64-bit rows and for frames of up to WAVES8_ITEMS work items, else 4 (a
-    frame of unknown size counts as large).  Left to choose, the library takes
-    4 for large frames of 64-bit rows too (library_waves)."""
+    """A count by the light grid first: 8 for 64-bit rows and for frames of up
+    to WAVES8_ITEMS work items, else 4 (a frame of unknown size counts as
+    large).  The library itself takes 4 for the largest frames of 64-bit rows
+    too (library_waves), which the layouts below follow where the size is known."""
     if res > 32:
         return 8
     return 8 if w is not None and h is not None and work_items(w, h, bins) <= WAVES8_ITEMS else 4
 
 
-def library_waves(res, w, h, bins=16):
-    """The library's own default (fd_set_occlusion_waves 0) for a plain frame."""
-    return 8 if work_items(w, h, bins) <= (WAVES8_ITEMS64 if res > 32 else WAVES8_ITEMS) else 4
-
-
 def default_layout(res, w=None, h=None):
-    return (16, 8, default_waves(res, w, h))
+    known = w is not None and h is not None
+    return (16, 8, library_waves(res, w, h) if known else default_waves(res))
 
 
 def class_key(scene, w, h, res):
@@ -140,7 +142,7 @@ def tune_classes(ctx, scene, items, cache=None, candidates=CANDIDATES, reps=3, o
 def layout(cache, scene, w, h, res):
     """(bins, tile, waves) of a class, or the default layout."""
     e = cache.get(class_key(scene, w, h, res))
-    return (e["bins"], e["tile"], e.get("waves", default_waves(res, w, h, e["bins"]))) if e else default_layout(res, w, h)
+    return (e["bins"], e["tile"], e.get("waves", library_waves(res, w, h, e["bins"]))) if e else default_layout(res, w, h)
 
 
 def order(cache, scene, w, h, res):
@@ -156,13 +158,15 @@ def split(cache, scene, w, h, res):
 
 
 def server_table(cache):
-    """The cache as the server's per-class table (fd_server_config.tune)."""
+    """The cache as the server's per-class table (fd_server_config.tune); a
+    class without a tuned wave count asks for none (0: the library's rules, by
+    frame and by batch)."""
     out = []
     for key, e in cache.items():
         scene, wh, res = key.split(":")
         w, h = wh.split("x")
         out.append(dict(scene=int(scene), w=int(w), h=int(h), res=int(res), bins=e["bins"], tile=e["tile"],
-                        waves=e.get("waves", default_waves(int(res), int(w), int(h), e["bins"])), order=e.get("order", 0),
+                        waves=e.get("waves", 0), order=e.get("order", 0),
                         split=e.get("split", 0), ms=e["ms"] or 0.0))
     return out
 

@@ -76,3 +76,16 @@ def test_batches(shim, n, w, h, res, asked, waves):
     want = [0] * 6
     want[(3 if res > 32 else 0) + {2: 0, 4: 1, 8: 2}[waves]] = n
     assert list(got) == want
+
+
+def test_untuned_classes_take_the_librarys_default():
+    """Where no count was tuned the tables ask for none, and the layouts name
+    the library's own (a large frame of 64-bit rows: 4)."""
+    at = importlib.import_module("4dzb_amd.autotune")
+    assert at.default_layout(64, 1920, 1080) == (16, 8, 4) and at.default_layout(64, 1024, 1024) == (16, 8, 8)
+    assert at.default_layout(64, 1920, 1080) in at.CANDIDATES
+    cache = {at.class_key(0, 1920, 1080, 64): dict(bins=16, tile=8, ms=1.0, default_ms=1.0, candidates={}),
+             at.class_key(0, 256, 256, 16): dict(bins=16, tile=8, waves=4, ms=1.0, default_ms=1.0, candidates={})}
+    assert at.layout(cache, 0, 1920, 1080, 64) == (16, 8, 4) and at.layout({}, 0, 1920, 1080, 64) == (16, 8, 4)
+    assert at.layout(cache, 0, 256, 256, 16) == (16, 8, 4)
+    assert sorted((t["w"], t["waves"]) for t in at.server_table(cache)) == [(256, 4), (1920, 0)]
