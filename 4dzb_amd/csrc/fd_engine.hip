@@ -1003,20 +1003,33 @@ namespace fdk {
 hipError_t debug_rect(const FdArgs& a, float* out8, hipStream_t st);
 hipError_t selftest_rowmask(const float* D, const float* B, int n, int R, int mode, unsigned long long* out);
 hipError_t selftest_rowwindow(const float* coef, int n, int R, unsigned long long* out);
+hipError_t selftest_rows(const float* coef, int n, int R, unsigned long long* out);
 }
 
-extern "C" int fd_selftest_rowwindow(const float* hcoef, int n, int R, unsigned long long* hout) {
+namespace {
+// host triples in, `words` words per triple out, through a self-test kernel
+int selftest_triples(const float* hcoef, int n, int R, int words, unsigned long long* hout,
+                     hipError_t (*run)(const float*, int, int, unsigned long long*)) {
     if (!hcoef || !hout || n <= 0 || R < 1 || R > 64) return FD_ERR_ARG;
     float* dC = nullptr;
     unsigned long long* dO = nullptr;
     hipError_t e = hipMalloc(&dC, (size_t)n * 9 * sizeof(float));
-    if (e == hipSuccess) e = hipMalloc(&dO, (size_t)n * 4 * sizeof(unsigned long long));
+    if (e == hipSuccess) e = hipMalloc(&dO, (size_t)n * words * sizeof(unsigned long long));
     if (e == hipSuccess) e = hipMemcpy(dC, hcoef, (size_t)n * 9 * sizeof(float), hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = fdk::selftest_rowwindow(dC, n, R, dO);
-    if (e == hipSuccess) e = hipMemcpy(hout, dO, (size_t)n * 4 * sizeof(unsigned long long), hipMemcpyDeviceToHost);
+    if (e == hipSuccess) e = run(dC, n, R, dO);
+    if (e == hipSuccess) e = hipMemcpy(hout, dO, (size_t)n * words * sizeof(unsigned long long), hipMemcpyDeviceToHost);
     if (dC) (void)hipFree(dC);
     if (dO) (void)hipFree(dO);
     return hip_status(e);
+}
+}  // namespace
+
+extern "C" int fd_selftest_rowwindow(const float* hcoef, int n, int R, unsigned long long* hout) {
+    return selftest_triples(hcoef, n, R, 4, hout, fdk::selftest_rowwindow);
+}
+
+extern "C" int fd_selftest_rows(const float* hcoef, int n, int R, unsigned long long* hout) {
+    return selftest_triples(hcoef, n, R, 3, hout, fdk::selftest_rows);
 }
 
 extern "C" int fd_selftest_rowmask(const float* hD, const float* hB, int n, int R, int mode, unsigned long long* hout) {

@@ -1762,6 +1762,75 @@ __device__ __forceinline__ void row_occupancy(const uint32_t* lds, int R, int ls
         U[s] = (s << lsw) < R ? __ballot((a & (T)(strip << (s << lsw))) != (T)0) & rows : 0ull;
 }
 
+// One row of a pair with finite planes without a division, where that decides
+// it.  G = the least of the edges' largest values along the row,
+// D + max(B (R-1), 0).  G < -tol: the mask is empty.  G > tol: the
+// row is in the reference's row-range mask (its roundings
+// and G's stay below 8u (|A| R + |B| R + |C|)) and every edge passes at its far end, so the
+// edge's mask is the half line c >= -D/B (B > 0) or c < -D/B (B < 0)
+// clipped to the grid; x = R - 1/2 + D rcp(B) rounds to
+// R - ceil(-D/B) unless x is within 2^-15 of a tie (rcp, the fma and
+// the reference's quotient are off by at most 2^-17 + 2^-19 + 2^-19
+// while 0 <= -D/B <= R <= 64).  Edges
+// of the other sign stand in with x = 0 (upper limits) and x = R
+// (lower limits), the grid's own ends; planes through one vertex
+// fan cannot all have one sign of B but by rounding, which goes the
+// exact way, as do ties and |G| <= tol.  A zero B gives an infinite
+// reciprocal: no limit, as every column then has the sign of G.
+struct RowEdges {
+    float rh[3], rl[3], Kh[3], Kl[3], bp[3];
+    int tolBits;
+};
+// tolB: the bits of a tol >= 3u (|A| R + |B| R + |C|)
+__device__ __forceinline__ RowEdges row_edges(const Edge (&e)[3], float Rf, float nsub, const int tolB) {
+    RowEdges w;
+    const int Rm = __float_as_int(Rf - 0.5f), RmR = Rm ^ __float_as_int(Rf);
+    int sAnd = -1, sOr = 0;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        int sB = __float_as_int(e[k].B) >> 31;
+        asm("" : "+v"(sB));   // as a mask: selects run at half the rate
+        const int rB = __float_as_int(__builtin_amdgcn_rcpf(e[k].B)), bn = __float_as_int(e[k].B * nsub);
+        w.rh[k] = __int_as_float(rB & sB);
+        w.rl[k] = __int_as_float(rB ^ (rB & sB));
+        w.Kh[k] = __int_as_float(Rm & sB);
+        w.Kl[k] = __int_as_float(Rm ^ (RmR & sB));
+        w.bp[k] = __int_as_float(bn ^ (bn & sB));
+        sAnd &= sB;
+        sOr |= sB;
+    }
+    w.tolBits = tolB | ((sAnd | ~sOr) & 0x7f800000);
+    return w;
+}
+// row fr's mask where sure is all ones; sure 0: undecided
+template <typename T>
+__device__ __forceinline__ T row_fast(const Edge (&e)[3], const RowEdges& w, float fr, int R, T& sureT) {
+    float D[3], xh[3], xl[3], g[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        D[k] = e[k].A * fr + e[k].C;
+        xh[k] = __builtin_fmaf(D[k], w.rh[k], w.Kh[k]);
+        xl[k] = __builtin_fmaf(D[k], w.rl[k], w.Kl[k]);
+        g[k] = D[k] + w.bp[k];
+    }
+    const float xH = fmaxf(fmaxf(xh[0], xh[1]), xh[2]), xL = fminf(fminf(xl[0], xl[1]), xl[2]);
+    const int G = __float_as_int(fminf(fminf(g[0], g[1]), g[2]));
+    const float yH = -WIN_MAGIC - xH, yL = xL + WIN_MAGIC;
+    const float zH = xH + (yH + WIN_MAGIC), zL = xL - (yL - WIN_MAGIC);
+    // negative: decided (0x3efffc00 = 1/2 - 2^-15)
+    const int sure = ((__float_as_int(zH) & 0x7fffffff) - 0x3efffc00) &
+                     ((__float_as_int(zL) & 0x7fffffff) - 0x3efffc00) & (w.tolBits - (G & 0x7fffffff));
+    // as unsigned integers: iH has the sign bit, iL gets it unless yL
+    // (a limit far below the grid) or G (empty) is negative
+    const unsigned iL = (unsigned)__float_as_int(yL), iH = (unsigned)__float_as_int(yH);
+    const unsigned iS = (iL & 0x7fffffffu) | (~(iL | (unsigned)G) & 0x80000000u);
+    const T M = interval_bits<T>(__builtin_elementwise_sub_sat(iS, iH), (unsigned)(WIN_BASE + R) - iL);
+    int sm = sure >> 31;
+    asm("" : "+v"(sm));
+    sureT = (T)(int64_t)sm;
+    return M;
+}
+
 // One row of a pair with finite planes, decided with exact quotients: the AND
 // of the three edge masks, empty when the row is not in the reference's
 // row-range mask (three_edges<T, true>).  The reference only visits rows of
@@ -2342,40 +2411,9 @@ __device__ __forceinline__ void occlude_body(const FdArgs& a, const int blkIn) {
             if (lane == __ffsll((unsigned long long)__ballot(1)) - 1) nWaveRows += nr;
         }
     };
-    // Row by row from the first to the last row of the window that is not
-    // full.  G = the least of the edges' largest values along the row,
-    // D + max(B (R-1), 0).  G < -tol: the mask is empty.  G > tol: the
-    // row is in the reference's row-range mask (its roundings
-    // and G's stay below 8u (|A| R + |B| R + |C|)) and every edge passes at its far end, so the
-    // edge's mask is the half line c >= -D/B (B > 0) or c < -D/B (B < 0)
-    // clipped to the grid; x = R - 1/2 + D rcp(B) rounds to
-    // R - ceil(-D/B) unless x is within 2^-15 of a tie (rcp, the fma and
-    // the reference's quotient are off by at most 2^-17 + 2^-19 + 2^-19
-    // while 0 <= -D/B <= R <= 64).  Edges
-    // of the other sign stand in with x = 0 (upper limits) and x = R
-    // (lower limits), the grid's own ends; planes through one vertex
-    // fan cannot all have one sign of B but by rounding, which goes the
-    // exact way, as do ties and |G| <= tol.  A zero B gives an infinite
-    // reciprocal: no limit, as every column then has the sign of G.
-    // (tolBits: q / 16 >= 3u (|A| R + |B| R + |C|))
+    // row by row from the first to the last row of the window that is not full
     auto rows_fast = [&](const Edge (&e)[3], const T valid, const int tolB) {
-        float rh[3], rl[3], Kh[3], Kl[3], bp[3];
-        const int Rm = __float_as_int(Rf - 0.5f), RmR = Rm ^ __float_as_int(Rf);
-        int sAnd = -1, sOr = 0;
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            int sB = __float_as_int(e[k].B) >> 31;
-            asm("" : "+v"(sB));   // as a mask: selects run at half the rate
-            const int rB = __float_as_int(__builtin_amdgcn_rcpf(e[k].B)), bn = __float_as_int(e[k].B * nsub);
-            rh[k] = __int_as_float(rB & sB);
-            rl[k] = __int_as_float(rB ^ (rB & sB));
-            Kh[k] = __int_as_float(Rm & sB);
-            Kl[k] = __int_as_float(Rm ^ (RmR & sB));
-            bp[k] = __int_as_float(bn ^ (bn & sB));
-            sAnd &= sB;
-            sOr |= sB;
-        }
-        const int tolBits = tolB | ((sAnd | ~sOr) & 0x7f800000);
+        const RowEdges re = row_edges(e, Rf, nsub, tolB);
         const int r0 = Bits<T>::ctz(valid);
         const int r1 = Bits<T>::last(valid);
         wave_rows(r1 - r0 + 1);
@@ -2385,31 +2423,10 @@ __device__ __forceinline__ void occlude_body(const FdArgs& a, const int blkIn) {
         T bit = (T)1 << r0, redo = (T)0;
         do {
             if (COUNT) ++nRows;
-            float D[3], xh[3], xl[3], g[3];
-#pragma unroll
-            for (int k = 0; k < 3; ++k) {
-                D[k] = e[k].A * fr + e[k].C;
-                xh[k] = __builtin_fmaf(D[k], rh[k], Kh[k]);
-                xl[k] = __builtin_fmaf(D[k], rl[k], Kl[k]);
-                g[k] = D[k] + bp[k];
-            }
-            const float xH = fmaxf(fmaxf(xh[0], xh[1]), xh[2]), xL = fminf(fminf(xl[0], xl[1]), xl[2]);
-            const int G = __float_as_int(fminf(fminf(g[0], g[1]), g[2]));
-            const float yH = -WIN_MAGIC - xH, yL = xL + WIN_MAGIC;
-            const float zH = xH + (yH + WIN_MAGIC), zL = xL - (yL - WIN_MAGIC);
-            // negative: decided (0x3efffc00 = 1/2 - 2^-15)
-            const int sure = ((__float_as_int(zH) & 0x7fffffff) - 0x3efffc00) &
-                             ((__float_as_int(zL) & 0x7fffffff) - 0x3efffc00) & (tolBits - (G & 0x7fffffff));
-            // as unsigned integers: iH has the sign bit, iL gets it unless yL
-            // (a limit far below the grid) or G (empty) is negative
-            const unsigned iL = (unsigned)__float_as_int(yL), iH = (unsigned)__float_as_int(yH);
-            const unsigned iS = (iL & 0x7fffffffu) | (~(iL | (unsigned)G) & 0x80000000u);
-            const T M = interval_bits<T>(__builtin_elementwise_sub_sat(iS, iH), (unsigned)(WIN_BASE + R) - iL);
-            int sm = sure >> 31;
-            asm("" : "+v"(sm));
-            const T sureT = (T)(int64_t)sm;
-            redo |= bit & ~sureT;
-            add_row(w0, bit, M & sureT);
+            T sure;
+            const T M = row_fast<T>(e, re, fr, R, sure);
+            redo |= bit & ~sure;
+            add_row(w0, bit, M & sure);
             fr += 1.0f;
             bit += bit;
             w0 += FD_ROW_STRIDE;
@@ -3032,6 +3049,64 @@ __global__ void k_selftest_rowwindow(const float* coef, int n, int R, unsigned l
     else selftest_rowwindow_one<uint64_t>(coef + 9 * (size_t)i, R, out + 4 * (size_t)i);
 }
 
+// Verification of the row loop's decisions: for edge-plane triple i over an R x R
+// grid, out[3i] = the rows that row_fast decides (none where a coefficient is not
+// finite or above 2^78, where the kernel does not use it), out[3i + 1] = those
+// decided otherwise than by the general form on the reference's row range,
+// out[3i + 2] = the rows where row_exact is.  tol is the least that the windows
+// may give, 1/16 of max(52u (|A| R + |B| R + |C|), 2^-100).
+template <typename T>
+__device__ __forceinline__ void selftest_rows_one(const float* coef, int R, unsigned long long* out) {
+    Edge e[3];
+    const float nsub = (float)(unsigned)(R - 1);
+    const float Rf = (float)R;
+    float q = 7.8886091e-31f, DN[3];
+    bool ok = true;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        e[k].A = coef[3 * k];
+        e[k].B = coef[3 * k + 1];
+        e[k].C = coef[3 * k + 2];
+        e[k].nRowN = -(e[k].A * nsub);
+        e[k].nColN = -(e[k].B * nsub);
+        e[k].rA = rcp_or_nan(e[k].A);
+        e[k].rB = rcp_or_nan(e[k].B);
+        DN[k] = (e[k].B > 0 ? -e[k].nColN : 0.0f) + e[k].C;
+        const float a = fabsf(e[k].A), b = fabsf(e[k].B), c = fabsf(e[k].C);
+        ok = ok && a <= 3.0223145e+23f && b <= 3.0223145e+23f && c <= 3.0223145e+23f;   // 2^78; false for NaN
+        q = fmaxf(q, 3.0994415e-06f * (a * Rf + b * Rf + c));   // 52u
+    }
+    uint64_t decided = 0, wrong = 0, wrongExact = 0;
+    if (ok) {
+        const T FULL = (R >= Bits<T>::width) ? ~(T)0 : (((T)1 << R) - (T)1);
+        const T range = three_edges<T, true>(e, DN, Rf, R);
+        const RowEdges re = row_edges(e, Rf, nsub, __float_as_int(q) - (4 << 23));
+        for (int r = 0; r < R; ++r) {
+            float D[3];
+#pragma unroll
+            for (int k = 0; k < 3; ++k) D[k] = e[k].A * (float)r + e[k].C;
+            const T ref = ((range >> r) & (T)1) ? (T)(FULL & three_edges<T, false>(e, D, Rf, R)) : (T)0;
+            T sure;
+            const T M = row_fast<T>(e, re, (float)r, R, sure);
+            if (sure) {
+                decided |= 1ull << r;
+                if (M != ref) wrong |= 1ull << r;
+            }
+            if ((row_exact<T>(e, (float)r, nsub, R) & FULL) != ref) wrongExact |= 1ull << r;
+        }
+    }
+    out[0] = decided;
+    out[1] = wrong;
+    out[2] = wrongExact;
+}
+
+__global__ void k_selftest_rows(const float* coef, int n, int R, unsigned long long* out) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    if (R <= 32) selftest_rows_one<uint32_t>(coef + 9 * (size_t)i, R, out + 3 * (size_t)i);
+    else selftest_rows_one<uint64_t>(coef + 9 * (size_t)i, R, out + 3 * (size_t)i);
+}
+
 // Stage read-back of the receiver rectangles in the reference's 2-layer
 // layout (Step2_1_samplerRectangleAABB.inl:122-123); verification only.
 __global__ void k_debug_rect(FdArgs a, float* out) {
@@ -3128,6 +3203,13 @@ hipError_t selftest_rowmask(const float* D, const float* B, int n, int R, int mo
 
 hipError_t selftest_rowwindow(const float* coef, int n, int R, unsigned long long* out) {
     k_selftest_rowwindow<<<cdiv(n, 256), 256>>>(coef, n, R, out);
+    hipError_t e = hipGetLastError();
+    if (e == hipSuccess) e = hipDeviceSynchronize();
+    return e;
+}
+
+hipError_t selftest_rows(const float* coef, int n, int R, unsigned long long* out) {
+    k_selftest_rows<<<cdiv(n, 256), 256>>>(coef, n, R, out);
     hipError_t e = hipGetLastError();
     if (e == hipSuccess) e = hipDeviceSynchronize();
     return e;

@@ -154,6 +154,7 @@ def lib():
             "fd_set_profiling": ([vp, ip, ip], ip),
             "fd_selftest_rowmask": ([vp, vp, ip, ip, ip, vp], ip),
             "fd_selftest_rowwindow": ([vp, ip, ip, vp], ip),
+            "fd_selftest_rows": ([vp, ip, ip, vp], ip),
             "fd_device_count": ([ctypes.POINTER(ip)], ip),
             "fd_batch_create": ([vp, ctypes.c_void_p, ip, ctypes.POINTER(vp)], ip),
             "fd_batch_capture": ([vp, vp], ip),
@@ -211,6 +212,17 @@ def selftest_rowwindow(coef, res):
     out = np.empty((coef.shape[0], 4), np.uint64)
     _check(lib().fd_selftest_rowwindow(coef.ctypes.data, coef.shape[0], res, out.ctypes.data),
            "fd_selftest_rowwindow")
+    return out
+
+
+def selftest_rows(coef, res):
+    """Device row decisions on host edge-plane triples (n, 9) float32
+    (verification only).  Returns (n, 3) uint64: the rows decided without a
+    division, those decided otherwise than by the general form, and the rows
+    where the exact form differs from it."""
+    coef = np.ascontiguousarray(coef, np.float32).reshape(-1, 9)
+    out = np.empty((coef.shape[0], 3), np.uint64)
+    _check(lib().fd_selftest_rows(coef.ctypes.data, coef.shape[0], res, out.ctypes.data), "fd_selftest_rows")
     return out
 
 

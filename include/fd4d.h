@@ -477,6 +477,14 @@ int fd_selftest_rowmask(const float* D, const float* B, int n, int res, int mode
  * mask (the rows the reference visits). */
 int fd_selftest_rowwindow(const float* coef, int n, int res, unsigned long long* out);
 
+/* Verification only: the row loop's decisions without a division.  For n
+ * edge-plane triples (as above) out receives 3 row masks per triple: the rows
+ * decided (none where a coefficient is not finite or above 2^78: the kernel
+ * takes the general form there), those of them whose mask differs from the
+ * general form's on the reference's row range, and the rows where the exact
+ * form, which takes the others, differs from it. */
+int fd_selftest_rows(const float* coef, int n, int res, unsigned long long* out);
+
 const char* fd_status_string(int code);
 
 #ifdef __cplusplus
