@@ -177,7 +177,10 @@ void fill_args(FdArgs& a, const Model& md, const float4* pos, const float4* nrm,
 // item walks its bin's whole list: their lists split into about
 // FD_SPLIT_WAVES waves in all.  Larger frames fill the GPU already, and
 // splitting would only cost the merge and the early exit on full rows.  A
-// frame without triangles has no lists to split.  Needs a.occWaves.
+// frame without triangles has no lists to split.  Needs a.occWaves and
+// a.occVariant: the bin-queue variant runs one wave per stretch, nothing is
+// shared along a list, and fewer stretches only leave the GPU idle (96 x 96
+// receivers, 40 k evenly spread triangles: 1274 us with 8, 764 with 16).
 void apply_split(FdArgs& a, int req) {
     a.splitReq = req > 0 ? req : 0;
     if (a.ntris <= 0) {
@@ -186,9 +189,9 @@ void apply_split(FdArgs& a, int req) {
         a.segs = std::min(req, FD_LIST_SPLIT_MAX);
     } else {
         const long waves = (long)a.chunkSlots * std::max(a.occWaves, 1);
+        const long most = a.occVariant == FD_OCC_BIN_QUEUE ? 16 : fd_split_max(a.ntris, 1 << (2 * a.gridLog2));
         a.segs = (a.chunkSlots <= FD_SPLIT_ITEMS && waves < FD_SPLIT_MIN_WAVES)
-                     ? (int)std::max(1L, std::min((long)fd_split_max(a.ntris, 1 << (2 * a.gridLog2)),
-                                                  FD_SPLIT_WAVES / waves)) : 1;
+                     ? (int)std::max(1L, std::min(most, FD_SPLIT_WAVES / waves)) : 1;
     }
 }
 

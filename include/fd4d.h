@@ -187,7 +187,7 @@ int fd_set_occlusion_waves(fd_ctx* ctx, int waves);
  * 0 (the default): a frame of up to 2048 work items with fewer than 6144
  * waves in all (work items x waves per item) splits into about 49152
  * waves (at most 4 stretches below 16 triangles per bin, 8 below 512, else
- * 16); larger ones do not (nor does a batch whose instances total more than
+ * 16; the bin-queue variant 16); larger ones do not (nor does a batch whose instances total more than
  * 2048 work items); 1..64: that many stretches.  The batched form takes it
  * per instance (fd_instance.list_split), the serving form per class
  * (fd_tune_entry.list_split). */
