@@ -144,13 +144,13 @@ inline int fd_split_max(long ntris, int nb) {
 #define FD_WAVES8_ITEMS64 28672
 // In a batch of more than FD_BATCH_WAVES4_ITEMS work items in all, its small
 // frames of 32-bit rows take 4 as well: the others fill the GPU beside them (us, 8
-// / 4 waves: 24 frames of 300 k work items 29306 / 28560; four of 700 x 700
-// receivers, 32 k items, 16 x 16 samples: spheres of 200 k triangles 3863 / 3254,
-// soup of 300 k 1496 / 1524, 300 k triangles of 20 spheres 8615 / 8657).  Below,
-// the longest lists outlast the batch (two of 512 x 512, 9 k items, 8 x 8
-// samples: that soup 608 / 800, those 20 spheres 3009 / 4038; three of 700 x 700,
-// 24 k items, 16 x 16: soup of 1 M 1922 / 2217), and 64-bit rows lose there and at
-// 31 k items (0 to 12% with 64 x 64 samples).
+// / 4 waves: four of 700 x 700 receivers, 32 k items, 16 x 16 samples: spheres of
+// 200 k triangles 3549 / 3052, soup of 300 k 1310 / 1340, 300 k triangles of 20
+// spheres 7896 / 7938; 24 of 256 x 256, 31 k items: 4652 / 4143, 2889 / 2721 and
+// 13704 / 13455).  Below, the longest lists outlast the batch (two of 512 x 512, 9
+// k items, 8 x 8 samples: that soup 545 / 726, those 20 spheres 3065 / 3539; three
+// of 700 x 700, 24 k items, 16 x 16: soup of 1 M 1702 / 1979), and 64-bit rows lose
+// there and at 31 k items (0 to 11% with 64 x 64 samples).
 #define FD_BATCH_WAVES4_ITEMS 28672
 inline int fd_default_waves(int wpr, long items) { return items <= (wpr == 2 ? FD_WAVES8_ITEMS64 : FD_WAVES8_ITEMS) ? 8 : 4; }
 inline bool fd_valid_waves(int w) { return w == 2 || w == 4 || w == 8; }

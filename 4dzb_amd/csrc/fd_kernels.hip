@@ -2103,9 +2103,10 @@ __device__ __forceinline__ void cta_tris(const FdArgs& a, uint32_t* lds, T* full
     }
 }
 
-// NW waves per work item (1 or 2): with 2, the waves share the work item's
-// receivers and LDS rows and take alternate triangles of the list (rows
-// merged with LDS atomics), so a CU holds twice the waves for the same LDS.
+// NW waves per work item (2, 4 or 8; 1 in the counting and bin-queue variants):
+// they share the work item's receivers and LDS rows and take interleaved
+// triangles of the list (rows merged with LDS atomics), so a CU holds NW times
+// the waves for the same LDS.
 template <typename T, bool COUNT, bool CTA = false, int NW = 1>
 __device__ __forceinline__ void occlude_body(const FdArgs& a, const int blkIn) {
     // per wave 64 tile windows (timed variants), then wpr * R rows of
@@ -2889,14 +2890,14 @@ __device__ __forceinline__ int xcd_block(int b, int n) {
 __global__ __launch_bounds__(64) void k_occlude_finish(FdArgs a) { occlude_finish_body(a, blockIdx.x); }
 
 // NW waves per occlusion work item (they share its receivers and LDS rows):
-// 4 (the default) or 2 per frame (FdArgs::occWaves).  The counting variant
+// 2, 4 or 8 per frame (FdArgs::occWaves; fd_default_waves).  The counting variant
 // runs one wave per work item: each receiver then meets its triangles in
 // list order with the full-row state of all earlier ones, as in the
 // reference, so its work counters do not depend on the schedule.
 // 6 waves per SIMD, 80 vector registers, of which 26 to 38 spill in the timed
-// variants; at 8 (64) and 7 (72) more do (heightfield-1k 2944 / 2754 / 2739 us at 8 / 7 / 6 waves,
-// 1080p soup with 32 x 32 samples 2510 / 2201 / 2100 us), at 5 too few waves
-// hide the record loads.
+// variants; at 8 (64) and 7 (72) more do (heightfield-1k 2944 / 2754 / 2739 us at
+// 8 / 7 / 6 waves, 1080p soup with 32 x 32 samples 2510 / 2201 / 2100 us when the
+// projected window came in), at 5 too few waves hide the record loads.
 template <typename T, bool COUNT, int NW>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(6))) void k_occlude(FdArgs a) {
     occlude_body<T, COUNT, false, NW>(a, xcd_block(blockIdx.x, gridDim.x));
@@ -3250,23 +3251,22 @@ hipError_t enqueue_frame(const FdArgs& a, hipStream_t st, hipEvent_t* ev) {
         if (wpr == 1) k_occlude_cta<uint32_t><<<chunks, 64, shmCta, st>>>(a);
         else k_occlude_cta<uint64_t><<<chunks, 64, shmCta, st>>>(a);
     } else {
-        const FdArgs& ao = a;
         const int chunks = a.chunkSlots * a.segs;
         if (a.opCount) {
             const size_t shm = fd_occ_lds(wpr, a.L.res, 0);
-            if (wpr == 1) k_occlude<uint32_t, true, 1><<<chunks, 64, shm, st>>>(ao);
-            else k_occlude<uint64_t, true, 1><<<chunks, 64, shm, st>>>(ao);
+            if (wpr == 1) k_occlude<uint32_t, true, 1><<<chunks, 64, shm, st>>>(a);
+            else k_occlude<uint64_t, true, 1><<<chunks, 64, shm, st>>>(a);
         } else {
             const int nw = fd_valid_waves(a.occWaves) ? a.occWaves : fd_default_waves(wpr, a.chunkSlots);
             const int c = fd_occ_class(wpr, nw);
             const size_t shm = fd_occ_lds(wpr, a.L.res, nw);
             switch (c) {
-                case 0: k_occlude<uint32_t, false, 2><<<chunks, 64 * nw, shm, st>>>(ao); break;
-                case 1: k_occlude<uint32_t, false, 4><<<chunks, 64 * nw, shm, st>>>(ao); break;
-                case 2: k_occlude<uint32_t, false, 8><<<chunks, 64 * nw, shm, st>>>(ao); break;
-                case 3: k_occlude<uint64_t, false, 2><<<chunks, 64 * nw, shm, st>>>(ao); break;
-                case 4: k_occlude<uint64_t, false, 4><<<chunks, 64 * nw, shm, st>>>(ao); break;
-                default: k_occlude<uint64_t, false, 8><<<chunks, 64 * nw, shm, st>>>(ao); break;
+                case 0: k_occlude<uint32_t, false, 2><<<chunks, 64 * nw, shm, st>>>(a); break;
+                case 1: k_occlude<uint32_t, false, 4><<<chunks, 64 * nw, shm, st>>>(a); break;
+                case 2: k_occlude<uint32_t, false, 8><<<chunks, 64 * nw, shm, st>>>(a); break;
+                case 3: k_occlude<uint64_t, false, 2><<<chunks, 64 * nw, shm, st>>>(a); break;
+                case 4: k_occlude<uint64_t, false, 4><<<chunks, 64 * nw, shm, st>>>(a); break;
+                default: k_occlude<uint64_t, false, 8><<<chunks, 64 * nw, shm, st>>>(a); break;
             }
         }
     }

@@ -623,7 +623,7 @@ LIGHT_DTYPE = np.dtype([("m", "<f4", 16), ("xd", "<f4", 3), ("yd", "<f4", 3), ("
                         ("wpr", "<i4"), ("pad", "<i4")])
 
 TRI_DTYPE = np.dtype([("v0", "<f4", 3), ("v1", "<f4", 3), ("v2", "<f4", 3), ("bminx", "<f4"), ("bminy", "<f4"),
-                      ("bmaxx", "<f4"), ("bmaxy", "<f4"), ("minz", "<f4"), ("maxz", "<f4"), ("pad0", "<f4"),
+                      ("bmaxx", "<f4"), ("bmaxy", "<f4"), ("minz", "<f4"), ("maxz", "<f4"), ("we", "<f4"),
                       ("n", "<f4", 3), ("e01", "<f4", 3), ("e12", "<f4", 3), ("e20", "<f4", 3), ("pad1", "<f4", 4)])
 
 

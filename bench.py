@@ -198,7 +198,7 @@ def plain_leg(pkg, frame, workload, steps, warmup, quick):
                                                                                    frame.rx.h, 1 << frame.grid_log2),
                            path="plain per-frame"),
                p50_ms=round(pctl(g["lat"], 50), 3), p99_ms=round(pctl(g["lat"], 99), 3),
-               stage_ms=dict(zip(["light_plane", "receiver_binning", "triangle_pairing", "tables", "occlusion"],
+               stage_ms=dict(zip(["light_plane", "receiver_keys", "pairing_and_scatters", "list_order", "occlusion"],
                                  [round(x, 4) for x in g["stage"]])),
                frame_stats=dict(valid_receivers=g["stats"]["valid_receivers"], pairs=g["stats"]["pairs"],
                                 valid_triangles=g["stats"]["valid_triangles"]),

@@ -419,7 +419,9 @@ typedef struct fd_gbuffer_scene {
  * reference clears to NaN, Render.cpp:423-426).  g0 / g1 are the visibility
  * path's receiver buffers (fd_set_sample_buffers); g2 / g3 may be NULL
  * (then, without materials, g0.w = g1.w = 1).  Double-precision ray cast,
- * stream-ordered on hip_stream (no host synchronisation). */
+ * stream-ordered on hip_stream (no host synchronisation).  Host tables in
+ * ordinary memory are read during the call; in page-locked or managed memory,
+ * and under stream capture, in stream order. */
 int fd_gbuffer_boxes(const fd_gbuffer_scene* scene, float* d_g0, float* d_g1, float* d_g2, float* d_g3,
                      void* hip_stream);
 
@@ -439,7 +441,8 @@ typedef struct fd_shade_params {
  * each light sample, ambient + (diffuse + specular) * intensity, summed and
  * divided by the sample count.  Float arithmetic with IEEE division and
  * square root (normalize(v) = v / sqrt(dot(v, v)), pow = powf).  Writes
- * float4 x width*height; stream-ordered. */
+ * float4 x width*height; stream-ordered (the sample table as in
+ * fd_gbuffer_boxes). */
 int fd_shade(const fd_shade_params* params, const float* d_shadow, const float* d_g0, const float* d_g1,
              const float* d_g2, const float* d_g3, float* d_rgba, void* hip_stream);
 
