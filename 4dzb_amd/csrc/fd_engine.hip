@@ -1032,7 +1032,7 @@ extern "C" int fd_selftest_rowwindow(const float* hcoef, int n, int R, unsigned 
 }
 
 extern "C" int fd_selftest_rows(const float* hcoef, int n, int R, unsigned long long* hout) {
-    return selftest_triples(hcoef, n, R, 3, hout, fdk::selftest_rows);
+    return selftest_triples(hcoef, n, R, 4, hout, fdk::selftest_rows);
 }
 
 extern "C" int fd_selftest_rowmask(const float* hD, const float* hB, int n, int R, int mode, unsigned long long* hout) {

@@ -178,6 +178,8 @@ inline size_t fd_occ_lds(int wpr, int res, int nw) {
 #define FD_TILE_MIN 6
 #define FD_PRUNE_LEFT 6
 #define FD_PRUNE_STEPS 16
+// Rows of a pair (last - first) from which the row loop takes row_range first
+#define FD_RANGE_ROWS 6
 
 // Occlusion classes of a batched launch: 32-bit / 64-bit rows x 2 / 4 / 8
 // waves per work item (one launch each).

@@ -217,11 +217,12 @@ def selftest_rowwindow(coef, res):
 
 def selftest_rows(coef, res):
     """Device row decisions on host edge-plane triples (n, 9) float32
-    (verification only).  Returns (n, 3) uint64: the rows decided without a
-    division, those decided otherwise than by the general form, and the rows
-    where the exact form differs from it."""
+    (verification only).  Returns (n, 4) uint64: the rows decided without a
+    division, those decided otherwise than by the general form, the rows where
+    the exact form differs from it, and those with a sample that the row range
+    leaves out."""
     coef = np.ascontiguousarray(coef, np.float32).reshape(-1, 9)
-    out = np.empty((coef.shape[0], 3), np.uint64)
+    out = np.empty((coef.shape[0], 4), np.uint64)
     _check(lib().fd_selftest_rows(coef.ctypes.data, coef.shape[0], res, out.ctypes.data), "fd_selftest_rows")
     return out
 

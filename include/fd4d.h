@@ -481,11 +481,12 @@ int fd_selftest_rowmask(const float* D, const float* B, int n, int res, int mode
 int fd_selftest_rowwindow(const float* coef, int n, int res, unsigned long long* out);
 
 /* Verification only: the row loop's decisions without a division.  For n
- * edge-plane triples (as above) out receives 3 row masks per triple: the rows
+ * edge-plane triples (as above) out receives 4 row masks per triple: the rows
  * decided (none where a coefficient is not finite or above 2^78: the kernel
  * takes the general form there), those of them whose mask differs from the
- * general form's on the reference's row range, and the rows where the exact
- * form, which takes the others, differs from it. */
+ * general form's on the reference's row range, the rows where the exact form,
+ * which takes the others, differs from it, and the rows with a sample that the
+ * loop's own row range leaves out. */
 int fd_selftest_rows(const float* coef, int n, int res, unsigned long long* out);
 
 const char* fd_status_string(int code);
