@@ -2229,7 +2229,7 @@ __device__ __forceinline__ void occlude_body(const FdArgs& a, const int blkIn) {
     constexpr bool SHARE_FULL = NW > 1 && !CTA;
     T* const fullSh = (T*)(lds + wpr * R * FD_ROW_STRIDE);
     // the receivers' rectangles and depths (after the full-row masks), for the
-    // cull of the few pairs that get there: five registers more per lane spill
+    // cull of the pairs: five registers more per lane spill
     float* const rectSh = (float*)(fullSh + 64);
     if (!CTA && wv == 0) {
         fullSh[lane] = (T)0;
@@ -2525,7 +2525,7 @@ __device__ __forceinline__ void occlude_body(const FdArgs& a, const int blkIn) {
         }
         rows_fast(e, valid, __float_as_int(sl.y));
     };
-    // one pair (triangle tid, this wave's receivers): sample window, cull,
+    // one pair (triangle tid, this wave's receivers): cull, sample window,
     // planes, rows
     auto step = [&](const int tid, auto axialT) {
         constexpr bool AXIAL = decltype(axialT)::value;
@@ -2533,10 +2533,12 @@ __device__ __forceinline__ void occlude_body(const FdArgs& a, const int blkIn) {
         const FdTri t = tris[tid];
         // the whole record in one round trip
         if (!COUNT) asm volatile("" ::"s"(t.v0[0]), "s"(t.bminx), "s"(t.minz), "s"(t.n[0]), "s"(t.e20[2]));
-        if (COUNT) {
-            if (full == FULL || culled(t)) return;
-            ++nPass;
-        }
+        // the cull first: where the receivers' heights spread (boxes on a ground),
+        // a third of these pairs pass the work item's bounds and no receiver's own
+        // (1.2 M triangles of tessellated boxes and ground, 1920 x 1080 receivers,
+        // tilted light, 16 x 16 samples: 8268 us after the window, 5966 before it)
+        if (full == FULL || culled(t)) return;
+        if (COUNT) ++nPass;
         // planes (Q,v0,v1), (Q,v1,v2), (Q,v2,v0) (:150-172) start from
         // a_k = v_{k+1} - Q; a_2 = v0 - Q also gives
         // dir = dot(Q - v0, n) (:130-132) = -dot(v0 - Q, n), exactly (every
@@ -2584,7 +2586,7 @@ __device__ __forceinline__ void occlude_body(const FdArgs& a, const int blkIn) {
             valid = may ? interval_bits<T>((unsigned)w, (unsigned)l0) : (T)0;
         }
         valid &= (~full) & FULL;
-        if (!COUNT && (valid == (T)0 || culled(t))) return;
+        if (!COUNT && valid == (T)0) return;
         // The reference negates t0, t1, L0_Q when dir < 0.  The sign is put
         // into L0 - Q and the light axes before the products (a sign flip
         // commutes with every rounding): A, B, C come out negated, identical
