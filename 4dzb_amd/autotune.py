@@ -40,6 +40,7 @@ SPLITS = (1, 2, 4, 8, 16)       # stretches per bin list tried against the autom
 
 WAVES8_ITEMS = 8192   # FD_WAVES8_ITEMS: frames of up to this many work items default to 8 waves
 WAVES8_ITEMS64 = 28672   # FD_WAVES8_ITEMS64: the same with light grids above 32x32
+WAVES8_ITEMS_WIDE = 45056   # FD_WAVES8_ITEMS_WIDE: above 48x48
 
 
 def work_items(w, h, bins=16):
@@ -51,7 +52,8 @@ def work_items(w, h, bins=16):
 def library_waves(res, w, h, bins=16):
     """The library's own default waves per occlusion work item of a plain w x h
     frame with a res x res light grid (fd_set_occlusion_waves 0)."""
-    return 8 if work_items(w, h, bins) <= (WAVES8_ITEMS64 if res > 32 else WAVES8_ITEMS) else 4
+    most = WAVES8_ITEMS_WIDE if res > 48 else WAVES8_ITEMS64 if res > 32 else WAVES8_ITEMS
+    return 8 if work_items(w, h, bins) <= most else 4
 
 
 def default_waves(res, w=None, h=None, bins=16):

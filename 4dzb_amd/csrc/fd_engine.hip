@@ -101,7 +101,7 @@ struct fd_ctx {
     int tileLog2 = 3;     // 8x8 receiver tiles
     int occVariant = FD_OCC_PER_SAMPLE;
     int triOrder = FD_TRI_ORDER_AUTO;
-    int occWaves = 0;     // 0: fd_default_waves of the frame's row width and work items
+    int occWaves = 0;     // 0: fd_default_waves of the frame's light grid and work items
     int listSplit = 0;    // 0: the automatic rule
     size_t maxTris = 0, maxVerts = 0;
     int W = 0, H = 0;
@@ -259,7 +259,7 @@ int frame_args(fd_ctx* c, FdArgs& a) {
     a.occVariant = c->occVariant;
     a.triOrder = c->triOrder;
     a.wavesReq = c->occWaves;
-    a.occWaves = a.wavesReq ? a.wavesReq : fd_default_waves(a.L.wpr, a.chunkSlots);
+    a.occWaves = a.wavesReq ? a.wavesReq : fd_default_waves(a.L.res, a.chunkSlots);
     apply_split(a, c->listSplit);
     return FD_OK;
 }
@@ -849,7 +849,7 @@ extern "C" int fd_batch_create(fd_ctx* c, const fd_instance* in, int n, fd_batch
         b->args[i].triOrder = q.tri_order ? q.tri_order : c->triOrder;
         const int waves = q.occ_waves ? q.occ_waves : c->occWaves;
         b->args[i].wavesReq = waves;
-        b->args[i].occWaves = waves ? waves : fd_default_waves(L.wpr, b->args[i].chunkSlots);
+        b->args[i].occWaves = waves ? waves : fd_default_waves(L.res, b->args[i].chunkSlots);
         apply_split(b->args[i], q.list_split ? q.list_split : c->listSplit);   // after occWaves
         FdArgs probe = b->args[i];
         off[i + 1] = off[i] + ((layout(probe, nullptr, false) + 255) & ~(size_t)255);

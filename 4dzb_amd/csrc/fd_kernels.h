@@ -132,16 +132,22 @@ inline int fd_split_max(long ntris, int nb) {
 // rows and full-row masks and split its triangle list.  8 for frames of up to
 // FD_WAVES8_ITEMS work items (too few to fill the GPU with 4 waves each), 4 for
 // larger frames: the fewer waves share a work item the less they walk past one
-// another.  64-bit rows leave LDS for 4 work items of 4 waves per CU at 64 x 64
-// samples, or 3 of 8, so that 4 waves also leave fewer of them in flight, and
-// what outlasts the frame, its longest lists, is walked by fewer: 4 only from
-// FD_WAVES8_ITEMS64 items on (us, 8 / 4 waves, 48 x 48 samples: 1 M triangle
-// soup 817 / 1252 at 720 x 720 receivers, 940 / 1106 at 960 x 960, 1697 / 1406
-// at 1920 x 1080; 300 k triangles of 20 spheres 2071 / 3275, 2865 / 3214 and
-// 5421 / 5236; 500 spheres of 200 k triangles 1254 / 1147 and 3933 / 3315; with
-// 64 x 64 samples at 1920 x 1080 1938 / 1784, 5790 / 6118 and 4641 / 4270).
+// another.  64-bit rows leave LDS for 5 work items of 4 waves per CU at 48 x 48
+// samples and 4 at 64 x 64, where 3 of 8 fit either way: 4 waves then also leave
+// fewer in flight, and the longest lists, which outlast the frame, to fewer:
+// 4 only from FD_WAVES8_ITEMS64 items on (us, 8 / 4 waves, 48 x 48 samples: 1 M
+// triangle soup 817 / 1252 at 720 x 720 receivers, 940 / 1106 at 960 x 960, 1697 /
+// 1406 at 1920 x 1080; 300 k triangles of 20 spheres 2071 / 3275, 2865 / 3214 and
+// 5421 / 5236; 500 spheres of 200 k triangles 1254 / 1147 and 3933 / 3315), and
+// above 48 samples a side from FD_WAVES8_ITEMS_WIDE on (64 x 64 samples, occluders
+// that the receivers lie on, at 1920 x 1080 and 2560 x 1440: 1.2 M triangles of
+// tessellated boxes 5949 / 7602 and 8299 / 8784, the same without their ground 2192
+// / 2682 and 3329 / 3335, slivers 10655 / 11562 and 17904 / 19330, terrain 3677 /
+// 3919 and 5814 / 5934; short and sparse lists go the other way: a canopy 1208 /
+// 1014 and 2050 / 1718, the evenly spread boxes 3518 / 3392 and 5827 / 5487).
 #define FD_WAVES8_ITEMS 8192
 #define FD_WAVES8_ITEMS64 28672
+#define FD_WAVES8_ITEMS_WIDE 45056
 // In a batch of more than FD_BATCH_WAVES4_ITEMS work items in all, its small
 // frames of 32-bit rows take 4 as well: the others fill the GPU beside them (us, 8
 // / 4 waves: four of 700 x 700 receivers, 32 k items, 16 x 16 samples: spheres of
@@ -152,7 +158,9 @@ inline int fd_split_max(long ntris, int nb) {
 // of 700 x 700, 24 k items, 16 x 16: soup of 1 M 1702 / 1979), and 64-bit rows lose
 // there and at 31 k items (0 to 11% with 64 x 64 samples).
 #define FD_BATCH_WAVES4_ITEMS 28672
-inline int fd_default_waves(int wpr, long items) { return items <= (wpr == 2 ? FD_WAVES8_ITEMS64 : FD_WAVES8_ITEMS) ? 8 : 4; }
+inline int fd_default_waves(int res, long items) {
+    return items <= (res > 48 ? FD_WAVES8_ITEMS_WIDE : res > 32 ? FD_WAVES8_ITEMS64 : FD_WAVES8_ITEMS) ? 8 : 4;
+}
 inline bool fd_valid_waves(int w) { return w == 2 || w == 4 || w == 8; }
 
 // LDS of an occlusion work item: the tile windows of each wave's block (64

@@ -3298,7 +3298,7 @@ hipError_t enqueue_frame(const FdArgs& a, hipStream_t st, hipEvent_t* ev) {
             if (wpr == 1) k_occlude<uint32_t, true, 1><<<chunks, 64, shm, st>>>(a);
             else k_occlude<uint64_t, true, 1><<<chunks, 64, shm, st>>>(a);
         } else {
-            const int nw = fd_valid_waves(a.occWaves) ? a.occWaves : fd_default_waves(wpr, a.chunkSlots);
+            const int nw = fd_valid_waves(a.occWaves) ? a.occWaves : fd_default_waves(a.L.res, a.chunkSlots);
             const int c = fd_occ_class(wpr, nw);
             const size_t shm = fd_occ_lds(wpr, a.L.res, nw);
             switch (c) {

@@ -320,7 +320,7 @@ long long fd_server_submit(fd_server* s, const fd_request* r) {
     fill_args(q.args, md, (const float4*)r->d_position4, (const float4*)r->d_normal4, r->width,
               r->height, L, s->cfg.eps, s->cfg.backface_cull, g, tl, r->d_shadow, r->d_masks, s->cfg.max_pairs);
     q.args.wavesReq = waves;
-    q.args.occWaves = waves ? waves : fd_default_waves(L.wpr, q.args.chunkSlots);
+    q.args.occWaves = waves ? waves : fd_default_waves(L.res, q.args.chunkSlots);
     q.args.triOrder = order;
     apply_split(q.args, split);
     FdArgs probe = q.args;

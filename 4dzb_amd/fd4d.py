@@ -351,8 +351,8 @@ class Context:
 
     def set_occlusion_waves(self, waves):
         """Waves per occlusion work item: 2, 4 or 8; 0 = the default (8 for frames
-        of up to 8192 work items, 28672 for light grids above 32x32, else 4).
-        Changes no result."""
+        of up to 8192 work items, 28672 for light grids above 32x32, 45056 above
+        48x48, else 4).  Changes no result."""
         _check(lib().fd_set_occlusion_waves(self.h, int(waves)), f"fd_set_occlusion_waves({waves})")
 
     def set_list_split(self, segs):

@@ -792,7 +792,7 @@ def main():
     ap.add_argument("--tile", type=int, default=0, help="receiver tile width (default 8)")
     ap.add_argument("--waves", type=int, default=0, choices=[0, 2, 4, 8],
                     help="waves per occlusion work item (default: 8 for frames of up to 8192 work items, 28672 above 32x32 light "
-                         "samples, else 4)")
+                         "samples, 45056 above 48x48, else 4)")
     ap.add_argument("--leg", choices=["batched", "served", "target", "app_pipeline", "shard_tile"], default=None,
                     help="run only this leg and print its JSON (for profiler runs)")
     args = ap.parse_args()

@@ -171,8 +171,8 @@ int fd_set_triangle_order(fd_ctx* ctx, int order);
  * item of the per-sample occlusion (64 receivers of one bin, whose triangle
  * list the waves split): 2, 4 or 8; 0 (the default) selects 8 for frames of
  * up to 8192 work items (about 710 x 710 receivers at 16 x 16 bins), for light
- * grids above 32 x 32 up to 28672 (about 1348 x 1348), 4 for larger ones; light
- * grids up to 32 x 32 also take 4 in a batch of more than 28672 work items in
+ * grids above 32 x 32 up to 28672 (about 1348 x 1348), above 48 x 48 up to 45056
+ * (1692 x 1692), 4 for larger ones; light grids up to 32 x 32 also take 4 in a batch of more than 28672 work items in
  * all.  Results do not depend on it.  The
  * batched form takes it per instance (fd_instance.occ_waves), the serving
  * form per class (fd_tune_entry.occ_waves). */
