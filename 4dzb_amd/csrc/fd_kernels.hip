@@ -2930,7 +2930,7 @@ __global__ __launch_bounds__(64) void k_occlude_finish(FdArgs a) { occlude_finis
 // runs one wave per work item: each receiver then meets its triangles in
 // list order with the full-row state of all earlier ones, as in the
 // reference, so its work counters do not depend on the schedule.
-// 6 waves per SIMD, 80 vector registers, of which 26 to 38 spill in the timed
+// 6 waves per SIMD, 80 vector registers, of which 28 to 33 spill in the timed
 // variants; at 8 (64) and 7 (72) more do (heightfield-1k 2944 / 2754 / 2739 us at
 // 8 / 7 / 6 waves, 1080p soup with 32 x 32 samples 2510 / 2201 / 2100 us when the
 // projected window came in), at 5 too few waves hide the record loads.
@@ -2973,9 +2973,9 @@ FD_BATCHED(kb_tri_order, FD_ORDER_THREADS, tri_order_body)
 // An instance's arguments where the scalar unit can read them again (its address
 // in scalar registers, in the constant address space), as a single frame's are in
 // its kernel arguments.  A copy of them was held in vector registers: 62 (64-bit
-// rows 68) spilled, now 26 (35), and batches of 16 frames of 256 x 256 receivers
-// and 16 x 16 samples over a soup of 300 k triangles took 2097 us, now 1942, over
-// spheres of 200 k 3360, now 3128.
+// rows 68) spilled, then 26 (35), and batches of 16 frames of 256 x 256 receivers
+// and 16 x 16 samples over a soup of 300 k triangles took 2097 us, then 1942, over
+// spheres of 200 k 3360, then 3128.
 __device__ __forceinline__ const FdArgs& inst_args(const FdArgs* inst, int i) {
 #if defined(__HIP_DEVICE_COMPILE__)
     typedef const __attribute__((address_space(4))) FdArgs* cargs_p;
