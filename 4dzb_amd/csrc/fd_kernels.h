@@ -141,7 +141,7 @@ inline int fd_split_max(long ntris, int nb) {
 // 5421 / 5236; 500 spheres of 200 k triangles 1254 / 1147 and 3933 / 3315), and
 // above 48 samples a side from FD_WAVES8_ITEMS_WIDE on (64 x 64 samples, occluders
 // that the receivers lie on, at 1920 x 1080 and 2560 x 1440: 1.2 M triangles of
-// tessellated boxes 5949 / 7602 and 8299 / 8784, the same without their ground 2192
+// tessellated boxes and ground 5949 / 7602 and 8299 / 8784, 216 k of boxes alone 2192
 // / 2682 and 3329 / 3335, slivers 10655 / 11562 and 17904 / 19330, terrain 3677 /
 // 3919 and 5814 / 5934; short and sparse lists go the other way: a canopy 1208 /
 // 1014 and 2050 / 1718, the evenly spread boxes 3518 / 3392 and 5827 / 5487).
